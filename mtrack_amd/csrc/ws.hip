@@ -3,22 +3,18 @@
 // worker_weakstrong (src/manager_weakstrong.c:7-263, src/worker_weakstrong.c:14-247).
 //
 // Each filled bunch is 2 Nslc + 1 slice centroids (tau, delta, x, x', z, z')
-// resident in HBM.  One turn is four launch groups on one stream:
+// resident in HBM.  The launches of a turn, on one stream:
 //
-//   k_ws_phase1  one block per bunch: synchrotron step of the centroids
-//                (transformSbunch_shortrange, src/rw_weakstrong.c:10-67), bunch
-//                centroid, CM history append (src/bunch.c:94-115), monitor-turn
-//                statistics (src/bunch.c:516-550); with FBII, one thread per
-//                point, the Bassetti-Erskine field of every slice on the 5 x 5
-//                absolute grid (two Faddeeva evaluations per point), then
-//                k_ws_create: the ions each bunch creates, one thread each,
-//                kicked by the bunch's later slices (fbi_weakstrong_bunch,
+//   k_ws_step    (without FBII) one block per bunch: phase 2 of the turn before
+//                and phase 1 of this one; with FBII it only ends a call;
+//   k_ws_phase1  (with FBII) blocks 0 .. G-1: the ion kicks of the turn before and
+//                phase 1; the others, one thread per point, the Bassetti-Erskine
+//                field of every slice on the 5 x 5 absolute grid (two Faddeeva
+//                evaluations per point);
+//   k_ws_create  the ions each bunch creates, one thread each, kicked by the
+//                bunch's later slices (fbi_weakstrong_bunch,
 //                src/fbi_weakstrong.c:49-298);
-//   k_ws_phase2  one block per bunch: betatron rotation of the centroids
-//                (transformSbunch_optic, :194-253) and the resistive-wall kick of
-//                every other bucket's centroid history (transformSbunch_longrange,
-//                :69-192), one lane per source bucket;
-//   train        the reference's manager relay (fbi_weakstrong_train
+//   k_ws_ions    the reference's manager relay (fbi_weakstrong_train
 //                :301-451): the accumulated ion cloud drifts to each bunch in
 //                train order, passes its slices (bilinear field interpolation,
 //                src/fbi_weakstrong.c:454-580), kicks the slice centroids with
@@ -26,14 +22,19 @@
 //                An ion's path depends only on the field tables phase 1 made
 //                and on the drift times, never on the kicks the train gives the
 //                electrons, so the whole relay is one launch with one lane per
-//                ion over every later bunch (k_ws_ions: per-slice wave sums,
-//                block partials per bunch), a per-bunch, per-quantity sum of
-//                the partials (k_ws_ksum) and the kicks (in k_ws_end);
-//                k_ws_cloud_reset + k_ws_train keep the bunch-by-bunch relay
-//                (one launch per bunch) for MBT_WS_SERIAL_TRAIN and for trains
-//                whose partials would not fit;
-//   k_ws_end     the ion-parallel train's kicks and cloud sums, and the
-//                slice-averaged vertical centroid of every bucket.
+//                ion over every later bunch (per-slice wave sums, block partials
+//                per bunch);
+//   k_ws_ksum    a per-bunch, per-quantity sum of the partials, and phase 2 of the
+//                turn in blocks beside.
+//
+// Phase 1 is the synchrotron step of the centroids (transformSbunch_shortrange,
+// src/rw_weakstrong.c:10-67), the bunch centroid, the CM history append
+// (src/bunch.c:94-115) and the monitor-turn statistics (src/bunch.c:516-550);
+// phase 2 the betatron rotation (transformSbunch_optic, :194-253) and the
+// resistive-wall kick of every other bucket's centroid history
+// (transformSbunch_longrange, :69-192).  k_ws_cloud_reset + k_ws_train keep the
+// bunch-by-bunch relay (one launch per bunch) for MBT_WS_SERIAL_TRAIN and for
+// trains whose partials would not fit.
 //
 // Everything but the ion-field sums, sin and the Faddeeva function keeps the
 // reference's operation order; constants derived with libm are computed on the
@@ -52,6 +53,7 @@
 #define WS_PTS 1250   // 50 slices x 25 grid points
 #define WS_TQ (2 * WS_S + 3 + 12) // per bunch in WSD::tot: 2 S + 3 train sums, 4 x 3 own-ion sums
 #define WS_HIST 30    // CM history depth (src/bunch.h:155)
+#define WS_RING 31    // rows of the dipole history: the depth and the row being written
 #define WS_MSG 5000   // doubles of the history message (src/manager_weakstrong.c:170-173)
 #define WS_T 256      // turns of outputs per device buffer block
 #define WS_WG 256
@@ -80,9 +82,10 @@ struct WSP {
   double eps, wrf, phai0, Urad, T0, ac;                 // synchrotron step
   double gamma1[3], alpha1[3], beta1[3];                // statistics
   double v11, v12, v21, v22, h11, h12, h21, h22;        // one-turn rotation (glibc cos/sin)
-  double rwa11[2], rwa12[2], prfrw[2], prfrw_trig[2];   // RW: [HOR, VER]
+  double rwa11[2], rwa12[2];                            // RW: [HOR, VER]
   int triggerRW;
-  double Pref0, fNp, Dub0, Lc;
+  double fNp;
+  double ntot; // macro-electrons in the slices
   double factBE, sxx, szz, deltT, aAx, aAz, aLx, aLz, den_dQ; // FBII fields
   double iaAx, iaAz;                                          // 1 / aAx, 1 / aAz
   double factF, factjp0, CdeltT;
@@ -93,9 +96,10 @@ struct WSD {
   double *sl;       // [G][6][S] xtau xeps xx xp zz zp
   const int *npop;  // [S]
   const int *nofe;  // [S*25]
-  const int *bucket, *fill; // [G], [h]
-  const double *Ibunch, *nelec, *convion; // [h] mA, [G], [G]
-  double *hist;     // [4][h][WS_HIST] x x' z z' (the manager's history)
+  const int *bucket; // [G]
+  const double *wallcur, *nelec, *convion; // [G] RW constant times bunch current, electrons, ions per macro-ion
+  double *dip;      // [2][WS_RING][G] wall dipoles of the bunches' centroids (HOR, VER), a row per turn
+  const double *wall; // [trigger][2][Nmlt + 1][h] wake per tap and distance in buckets (entry d - 1)
   double2 *Exy;     // [G][S*25] (Ex, Ey) of every grid point
   double *li;       // [5][G][S*25] local ions: Nri x x' y y'
   double *cl;       // [5][cap] ion cloud
@@ -192,20 +196,6 @@ __device__ __forceinline__ double wsum64x8(const double v[8])
   return y;
 }
 
-// bunch_strong_updateCM, src/bunch_strong.c:221-266 (sequential, one lane)
-__device__ void ws_cm(const double *u, const double *p, const int *npop, int S, double &pos, double &slope)
-{
-  double uu = 0.0, up = 0.0;
-  int n = 0;
-  for (int ic = 0; ic < S; ic++) {
-    uu += u[ic] * ((double)npop[ic]);
-    up += p[ic] * ((double)npop[ic]);
-    n += npop[ic];
-  }
-  pos = uu / ((double)n);
-  slope = up / ((double)n);
-}
-
 // get_linearly_interpolated_Efields, src/fbi_weakstrong.c:454-580, on one
 // slice's 25 field values, stored as (Ex, Ey) pairs so that one 16-byte LDS
 // read fetches both fields of a grid point.  The grid quotients multiply by the
@@ -239,87 +229,237 @@ __device__ __forceinline__ void ws_interp(const double2 *t, double aAx, double a
   Ex = x5 + sz * (x6 - x5);
 }
 
-// ------------------------------------------------------------------- phase 1
+// ------------------------------------------------------------- the electron side
 
-// Per bunch (blocks 0 .. G-1): the synchrotron step of every slice, the
-// centroids it reports, the manager's history and the monitor statistics.
-// With FBII every thread of the grid (G S 25 / WS_WG blocks, at least G) also
-// evaluates the Bassetti-Erskine field at one absolute grid point of one slice
-// of one bunch; the field needs the slices' transverse positions only, which
-// the synchrotron step leaves alone.
-__global__ __launch_bounds__(WS_WG) void k_ws_phase1(WSP P, WSD D, long long rev, int slot, int monitor)
+// The electron side of a turn for one bunch per block, on the bunch's slices
+// staged in LDS.  Three parts, any of which a launch may ask for:
+//   kicks of the ion train of the turn before (the sums of k_ws_ksum);
+//   phase 2 of turn rev2: the betatron rotation, the resistive-wall kick of every
+//     bunch's centroid history and the slice-averaged vertical centroid of the
+//     bunch's bucket (writeoutVCMmotionsPM2, src/fbi_weakstrong.c:688-737; the
+//     train's kicks, on the slopes, leave it alone);
+//   phase 1 of turn rev1: the synchrotron step of every slice, the centroids the
+//     bunch reports, the dipole history and the monitor statistics.
+// Phase 1 of a turn needs nothing but the bunch's own slices after phase 2 of the
+// turn before, so without FBII a turn is one launch (phase 2 of the turn before,
+// then phase 1) and one more ends the call.  The resistive wall reads only
+// dipoles of earlier launches: the history is a ring of WS_RING rows, and the row
+// phase 1 writes is older than any the same launch reads.
+// Bound: latency (sums of 41 slices and of up to h kicks kept in the
+// reference's order, one lane each).  416 bunches, 10 wall turns, per turn: 107 us
+// as three launches (one lane for all of a bunch's sums; a test of the filling, a
+// square root and two divisions per tap) -> 12.5 us as one.
+struct WSStep {
+  int kick;            // slot of the turn whose ion sums to apply, -1: none
+  long long rev2;      // phase 2 of this turn, -1: none
+  int slot2;
+  long long rev1;      // phase 1 of this turn, -1: none
+  int slot1, monitor;
+};
+
+#ifndef WS_STEP_WG
+#define WS_STEP_WG 512
+#endif
+
+// Row of turn rev - age in the dipole history ring.
+__device__ __forceinline__ int ws_row(long long rev, int age)
 {
-  const int tid = threadIdx.x, S = P.S;
-  if (blockIdx.x < P.G) {
-    const int b = blockIdx.x;
-    const int kb = D.bucket[b];
-    double *xtau = D.sl + (size_t)b * 6 * S, *xeps = xtau + S, *xx = xeps + S, *xp = xx + S, *zz = xp + S,
-           *zp = zz + S;
-    for (int ic = tid; ic < S; ic += WS_WG) {
+  const int r = (int)((rev - age) % WS_RING);
+  return r < 0 ? r + WS_RING : r;
+}
+
+// The resistive-wall kick bunch b (bucket kb) gets from bunch s, plane pl: the
+// taps j = 0 .. Nmlt of the source's dipole history over the tabulated wake
+// (transformSbunch_longrange, src/rw_weakstrong.c:69-192).  The worker's copy of
+// the history holds zeros where jb + j h falls outside the 5000-double message.
+__device__ __forceinline__ double ws_wall_kick(const WSP &P, const WSD &D, int kb, int s, int pl, long long rev)
+{
+  if (rev < P.Nmlt) return 0.0;
+  const int jb = D.bucket[s], h = P.h;
+  const double cur = D.wallcur[s];
+  // distance in buckets, h for the bunch's own (a full turn)
+  const int d = jb > kb ? jb - kb : h + jb - kb;
+  const int trig = P.triggerRW && rev < 50 ? 1 : 0;
+  const double *W = D.wall + (size_t)(trig * 2 + pl) * (P.Nmlt + 1) * h + d - 1;
+  const double *dip = D.dip + (size_t)pl * WS_RING * P.G + s;
+  const int a0 = jb > kb ? 0 : 1;
+  // oldest age the history and the message hold
+  const int amax = min(P.NmultiT - 1, (WS_MSG - 1 - jb) / h);
+  int row = ws_row(rev, a0);
+  double Dup = 0.0;
+  const int nj = min(P.Nmlt + 1, amax - a0 + 1);
+#pragma unroll 8
+  for (int j = 0; j < nj; j++) {
+    Dup = Dup + dip[row * P.G] * W[j * h];
+    row = row == 0 ? WS_RING - 1 : row - 1;
+  }
+  return cur * Dup;
+}
+
+// a + k[0] + k[1] + ... + k[n - 1] in that order, k in LDS, 16-byte aligned and
+// zero from n to the next multiple of 16.  The chain of additions is the
+// reference's; the reads of a group of eight are under way while the group before
+// is added (read one by one, the 416 kicks of a full ring took 5 us more).
+__device__ __forceinline__ double ws_add_in_order(double a, const double *k, int n)
+{
+  const double2 *q = (const double2 *)k;
+  double2 u[4], v[4];
+#pragma unroll
+  for (int i = 0; i < 4; i++) u[i] = q[i];
+  for (int s = 0; s < n; s += 16, q += 8) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = q[4 + i];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      a += u[i].x;
+      a += u[i].y;
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) u[i] = q[8 + i]; // past the end at the last group: unused
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      a += v[i].x;
+      a += v[i].y;
+    }
+  }
+  return a;
+}
+
+// LDS of ws_electrons, in doubles: the six slice arrays, populations and six rows
+// of products, each row and the two rows of kicks padded for ws_add_in_order.
+#define WS_PAD16(n) (((n) + 15) / 16 * 16)
+__host__ __device__ __forceinline__ int ws_electrons_lds(int S, int G)
+{
+  return 13 * WS_PAD16(S) + 2 * WS_PAD16(G) + 8;
+}
+
+// One block's bunch b; sm: ws_electrons_lds(S, G) doubles, 16-byte aligned.
+__device__ void ws_electrons(const WSP &P, const WSD &D, int b, const WSStep &T, double *sm)
+{
+  const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wv = tid >> 6, S = P.S, G = P.G;
+  const int kb = D.bucket[b];
+  const int SP = WS_PAD16(S), GP = WS_PAD16(G);
+  double *xtau = sm, *xeps = xtau + SP, *xx = xeps + SP, *xp = xx + SP, *zz = xp + SP, *zp = zz + SP;
+  double *np = zp + SP, *wt = np + SP, *dup = wt + 6 * SP;
+  __shared__ double cms[6];
+  double *sl = D.sl + (size_t)b * 6 * S;
+  for (int i = tid; i < 6 * SP; i += nt) {
+    const int c = i / SP, ic = i - c * SP;
+    sm[i] = ic < S ? sl[c * S + ic] : 0.0;
+  }
+  for (int i = tid; i < SP; i += nt) np[i] = i < S ? (double)D.npop[i] : 0.0;
+  const bool p2 = T.rev2 >= 0, p1 = T.rev1 >= 0, wall = p2 && P.rw;
+  if (wall)
+    for (int e = tid; e < 2 * GP; e += nt) {
+      const int pl = e >= GP, s = e - pl * GP;
+      dup[e] = s < G && (pl ? P.track_v : P.track_h) ? ws_wall_kick(P, D, kb, s, pl, T.rev2) : 0.0;
+    }
+  __syncthreads();
+  if (T.kick >= 0) {
+    const int NQ = 2 * S + 3;
+    const double *tot = D.tot + (size_t)b * WS_TQ;
+    if (b > 0) {
+      const double nel = D.nelec[b];
+      for (int c = tid; c < S; c += nt) {
+        const double dQ = nel * D.npop[c] * K_E;
+        const double fjp = dQ > 0.0 ? P.factjp0 / dQ : 0.0;
+        const double sx = fjp * tot[2 * c], sy = fjp * tot[2 * c + 1];
+        xp[c] = xp[c] + P.CdeltT * sx;
+        zp[c] = zp[c] + P.CdeltT * sy;
+      }
+    }
+    if (tid >= 64 && tid < 67) {
+      const int m = tid - 64;
+      double v = b > 0 ? tot[2 * S + m] : 0.0;
+      for (int w = 0; w < WS_WG / 64; w++) v += tot[NQ + 3 * w + m];
+      D.ion[((size_t)T.kick * G + b) * 3 + m] = v;
+    }
+    __syncthreads();
+  }
+  if (p2) {
+    // wave 0 the horizontal plane, wave 1 the vertical one, a lane per slice
+    if (wv < 2 && lane < S) {
+      double *u = wv ? zz : xx, *q = wv ? zp : xp;
+      const double m11 = wv ? P.v11 : P.h11, m12 = wv ? P.v12 : P.h12, m21 = wv ? P.v21 : P.h21,
+                   m22 = wv ? P.v22 : P.h22;
+      const double un = m11 * u[lane] + m12 * q[lane];
+      double a = m21 * u[lane] + m22 * q[lane];
+      if (wall && (wv ? P.track_v : P.track_h)) a = ws_add_in_order(a, dup + wv * GP, G); // in bucket order
+      u[lane] = un;
+      q[lane] = a;
+    }
+    __syncthreads();
+    if (tid == 128) D.zcm[(size_t)T.slot2 * P.h + kb] = ws_add_in_order(0.0, zz, S) / ((double)S);
+  }
+  if (p1) {
+    for (int ic = tid; ic < S; ic += nt) {
       const double e0 = xeps[ic];
       const double gain = P.eps * sin(P.wrf * xtau[ic] + P.phai0);
       xeps[ic] = e0 + gain - P.Urad;
       xtau[ic] = xtau[ic] - e0 * P.T0 * P.ac;
     }
     __syncthreads();
-    if (tid == 0) {
-      double pos[3], slope[3];
-      ws_cm(xtau, xeps, D.npop, S, pos[0], slope[0]);
-      ws_cm(xx, xp, D.npop, S, pos[1], slope[1]);
-      ws_cm(zz, zp, D.npop, S, pos[2], slope[2]);
-      double *o = D.cm + ((size_t)slot * P.G + b) * 4;
-      o[0] = pos[1];
-      o[1] = slope[1];
-      o[2] = pos[2];
-      o[3] = slope[2];
-      // the manager's history of this bucket: shift by one, newest at 0
-      const double nw[4] = {pos[1], slope[1], pos[2], slope[2]};
-      for (int a = 0; a < 4; a++) {
-        double *hrow = D.hist + ((size_t)a * P.h + kb) * WS_HIST;
-        for (int i = 0; i < P.NmultiT; i++) {
-          const int j = P.NmultiT - i - 2;
-          if (j >= 0) hrow[j + 1] = hrow[j];
-          else hrow[0] = nw[a];
-        }
+    // bunch_strong_updateCM (src/bunch_strong.c:221-266), one lane per coordinate
+    for (int i = tid; i < 6 * SP; i += nt) wt[i] = sm[i] * np[i % SP];
+    __syncthreads();
+    if (tid < 6) cms[tid] = ws_add_in_order(0.0, wt + tid * SP, S) / P.ntot;
+    __syncthreads();
+    if (tid < 4) D.cm[((size_t)T.slot1 * G + b) * 4 + tid] = cms[2 + tid];
+    if (P.rw && tid < 2)
+      D.dip[((size_t)tid * WS_RING + ws_row(T.rev1, 0)) * G + b] =
+          P.fNp * (P.rwa11[tid] * cms[2 + 2 * tid] + P.rwa12[tid] * cms[3 + 2 * tid]);
+    if (T.monitor && tid < 18) {
+      // quantity k (position, its rms, slope, its rms, ampinv, its centroid's) of plane pl
+      const int k = tid / 3, pl = tid % 3;
+      const double *u = sm + 2 * pl * SP, *p = u + SP, avr = cms[2 * pl], avs = cms[2 * pl + 1];
+      double v = 0.0;
+      if (k == 1 || k == 3) {
+        const double *w = k == 1 ? u : p, av = k == 1 ? avr : avs;
+        for (int ic = 0; ic < S; ic++) v += (w[ic] - av) * (w[ic] - av) * np[ic];
+        v = sqrt(v / P.ntot);
+      } else if (k == 4) {
+        for (int ic = 0; ic < S; ic++)
+          v += np[ic] * (P.gamma1[pl] * (u[ic] * u[ic]) + 2.0 * P.alpha1[pl] * u[ic] * p[ic] +
+                         P.beta1[pl] * (p[ic] * p[ic]));
+        v = v / P.ntot;
+      } else if (k == 5) {
+        v = P.gamma1[pl] * (avr * avr) + 2.0 * P.alpha1[pl] * avr * avs + P.beta1[pl] * (avs * avs);
+      } else {
+        v = k == 0 ? avr : avs;
       }
-      if (monitor) {
-        double *m = D.mon + ((size_t)slot * P.G + b) * 18;
-        const double *U[3] = {xtau, xx, zz}, *Q[3] = {xeps, xp, zp};
-        for (int pl = 0; pl < 3; pl++) {
-          for (int k = 0; k < 6; k++) m[3 * k + pl] = 0.0;
-          if (!P.track[pl]) continue;
-          const double *u = U[pl], *p = Q[pl];
-          double avr, avs;
-          ws_cm(u, p, D.npop, S, avr, avs);
-          double sq = 0.0, sqs = 0.0, amp = 0.0;
-          int w1 = 0, w2 = 0, n = 0;
-          for (int ic = 0; ic < S; ic++) {
-            sq += (u[ic] - avr) * (u[ic] - avr) * D.npop[ic];
-            w1 += D.npop[ic];
-          }
-          for (int ic = 0; ic < S; ic++) {
-            sqs += (p[ic] - avs) * (p[ic] - avs) * D.npop[ic];
-            w2 += D.npop[ic];
-          }
-          for (int ic = 0; ic < S; ic++) {
-            amp += D.npop[ic] * (P.gamma1[pl] * (u[ic] * u[ic]) + 2.0 * P.alpha1[pl] * u[ic] * p[ic] +
-                                 P.beta1[pl] * (p[ic] * p[ic]));
-            n += D.npop[ic];
-          }
-          m[pl] = avr;
-          m[3 + pl] = sqrt(sq / ((double)w1));
-          m[6 + pl] = avs;
-          m[9 + pl] = sqrt(sqs / ((double)w2));
-          m[12 + pl] = amp / ((double)n);
-          m[15 + pl] = P.gamma1[pl] * (avr * avr) + 2.0 * P.alpha1[pl] * avr * avs + P.beta1[pl] * (avs * avs);
-        }
-      }
+      D.mon[((size_t)T.slot1 * G + b) * 18 + 3 * k + pl] = P.track[pl] ? v : 0.0;
     }
   }
-  if (!P.fbii) return;
-  // ---- Bassetti-Erskine field of one slice at one absolute grid point
+  // back to memory: tau and delta move in phase 1 only, the positions in phase 2
+  // only (other blocks of a launch without it read them)
+  __syncthreads();
+  for (int i = tid; i < 6 * S; i += nt) {
+    const int c = i / S;
+    if (c < 2 ? p1 : (c == 2 || c == 4 ? p2 : p2 || T.kick >= 0)) sl[i] = sm[c * SP + i - c * S];
+  }
+}
+
+// Blocks 0 .. G-1: the electron side of a bunch each.
+__global__ __launch_bounds__(WS_STEP_WG) void k_ws_step(WSP P, WSD D, WSStep T)
+{
+  extern __shared__ double sm[];
+  ws_electrons(P, D, blockIdx.x, T, sm);
+}
+
+// With FBII, phase 1: blocks 0 .. G-1 the electron side (the train's kicks of the
+// turn before and phase 1), the others the Bassetti-Erskine field at one absolute
+// grid point of one slice of one bunch per thread; the field needs the slices'
+// transverse positions only, which kicks and phase 1 leave alone.
+__global__ __launch_bounds__(WS_WG) void k_ws_phase1(WSP P, WSD D, WSStep T)
+{
+  extern __shared__ double sm[];
+  const int tid = threadIdx.x, S = P.S;
+  if ((int)blockIdx.x < P.G) {
+    ws_electrons(P, D, blockIdx.x, T, sm);
+    return;
+  }
   const int npts = S * 25;
-  const long long gq = (long long)blockIdx.x * WS_WG + tid;
+  const long long gq = (long long)(blockIdx.x - P.G) * WS_WG + tid;
   if (gq >= (long long)P.G * npts) return;
   const int b = (int)(gq / npts), q = (int)(gq - (long long)b * npts);
   const double *xx = D.sl + (size_t)b * 6 * S + 2 * S, *zz = xx + 2 * S;
@@ -378,69 +518,6 @@ __global__ __launch_bounds__(WS_WG) void k_ws_create(WSP P, WSD D)
   D.li[2 * GP + gq] = xd;
   D.li[3 * GP + gq] = y;
   D.li[4 * GP + gq] = yd;
-}
-
-// ------------------------------------------------------------------- phase 2
-
-__global__ __launch_bounds__(WS_WG) void k_ws_phase2(WSP P, WSD D, long long rev)
-{
-  extern __shared__ double dup[]; // [2][h]
-  const int b = blockIdx.x, tid = threadIdx.x, S = P.S, h = P.h;
-  const int kb = D.bucket[b];
-  double *xx = D.sl + (size_t)b * 6 * S + 2 * S, *xp = xx + S, *zz = xp + S, *zp = zz + S;
-  for (int ic = tid; ic < S; ic += WS_WG) {
-    const double y = P.v11 * zz[ic] + P.v12 * zp[ic];
-    const double yp = P.v21 * zz[ic] + P.v22 * zp[ic];
-    zz[ic] = y;
-    zp[ic] = yp;
-    const double x = P.h11 * xx[ic] + P.h12 * xp[ic];
-    const double xq = P.h21 * xx[ic] + P.h22 * xp[ic];
-    xx[ic] = x;
-    xp[ic] = xq;
-  }
-  if (!P.rw) return;
-  // the kick of every filled source bucket jb, one lane each; the worker's copy
-  // of the history holds zeros where jb + j h falls outside the 5000-double message
-  for (int pl = 0; pl < 2; pl++) {
-    if (!(pl == 0 ? P.track_h : P.track_v)) continue;
-    const double *uh = D.hist + (size_t)(pl == 0 ? 0 : 2) * h * WS_HIST;
-    const double *ph = uh + (size_t)h * WS_HIST;
-    const double prf = (P.triggerRW && rev < 50) ? P.prfrw_trig[pl] : P.prfrw[pl];
-    for (int jb = tid; jb < h; jb += WS_WG) {
-      double Dup = 0.0;
-      if (D.fill[jb]) {
-        double D0;
-        if (jb == kb) D0 = P.Lc;
-        else if (jb > kb) D0 = ((double)(jb - kb)) * P.Dub0;
-        else D0 = ((double)(h + jb - kb)) * P.Dub0;
-        for (int j = 0; j < P.Nmlt + 1; j++) {
-          const double Du = D0 + ((double)j) * P.Lc;
-          const double Dt = Du / K_C;
-          const double W = prf / sqrt(Dt);
-          const int jm = jb > kb ? j : j + 1;
-          const bool in = jb + jm * h < WS_MSG;
-          const double u = in ? uh[(size_t)jb * WS_HIST + jm] : 0.0, p = in ? ph[(size_t)jb * WS_HIST + jm] : 0.0;
-          const double ujb = P.rwa11[pl] * u + P.rwa12[pl] * p;
-          const double dip = P.fNp * ujb;
-          Dup = Dup + dip * W;
-        }
-        Dup = P.Pref0 * D.Ibunch[jb] * Dup;
-        if (rev < P.Nmlt) Dup = 0.0;
-      }
-      dup[pl * h + jb] = Dup;
-    }
-  }
-  __syncthreads();
-  for (int pl = 0; pl < 2; pl++) {
-    if (!(pl == 0 ? P.track_h : P.track_v)) continue;
-    double *up = pl == 0 ? xp : zp;
-    for (int ic = tid; ic < S; ic += WS_WG) {
-      double a = up[ic];
-      for (int jb = 0; jb < h; jb++)
-        if (D.fill[jb]) a += dup[pl * h + jb];
-      up[ic] = a;
-    }
-  }
 }
 
 // ------------------------------------------------------------------ the train
@@ -829,16 +906,23 @@ __global__ __launch_bounds__(WS_WG) void k_ws_ions(WSP P, WSD D)
 // Per bunch ib (blockIdx.x) and group of KSUM_Q quantities (blockIdx.y): the
 // blocks' partials summed in a fixed order, one quantity per wave (lane l adds
 // blocks l, l + 64, ... in turn, then the wave sum), into D.tot[ib][i].  The
-// last group of each bunch sums instead the bunch's own ions (Nri x, Nri y,
-// Nri over its S * 25 ions, four waves' sums in order) into D.tot[ib][NQ + 3 w
-// + m], which k_ws_end adds to the cloud sums after the bunch.
+// last group but one of each bunch sums instead the bunch's own ions (Nri x, Nri
+// y, Nri over its S * 25 ions, four waves' sums in order) into D.tot[ib][NQ + 3 w
+// + m], which the kicks add to the cloud sums after the bunch.  The last group is
+// phase 2 of the turn (nothing of the train reads the slices once the ions are
+// made), a launch fewer per turn.
 #define KSUM_Q 8
-__global__ __launch_bounds__(64 * KSUM_Q) void k_ws_ksum(WSP P, WSD D)
+__global__ __launch_bounds__(64 * KSUM_Q) void k_ws_ksum(WSP P, WSD D, WSStep T)
 {
+  extern __shared__ double sm[];
+  if (blockIdx.y == gridDim.y - 1) {
+    ws_electrons(P, D, blockIdx.x, T, sm);
+    return;
+  }
   const int ib = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, S = P.S, npts = S * 25;
   const int NQ = 2 * S + 3;
   double *tot = D.tot + (size_t)ib * WS_TQ;
-  if (blockIdx.y == gridDim.y - 1) {
+  if (blockIdx.y == gridDim.y - 2) {
     if (tid >= WS_WG) return;
     const size_t GP = (size_t)P.G * npts;
     double t0 = 0.0, t1 = 0.0, t2 = 0.0;
@@ -870,47 +954,6 @@ __global__ __launch_bounds__(64 * KSUM_Q) void k_ws_ksum(WSP P, WSD D)
   if (lane == 0) tot[i] = v;
 }
 
-// Blocks 0 .. nkick-1 (the ion-parallel train, nkick = G): bunch b's slice
-// kicks from the ion field sums and the cloud sums after it with its own ions
-// appended (the sums of k_ws_ksum).  The blocks after them: the slice-averaged
-// vertical centroid of every bucket (writeoutVCMmotionsPM2,
-// src/fbi_weakstrong.c:688-737), which the kicks (on the slopes) leave alone.
-__global__ void k_ws_end(WSP P, WSD D, const int *bunch_of_bucket, int slot, int nkick)
-{
-  const int tid = threadIdx.x, S = P.S;
-  if ((int)blockIdx.x < nkick) {
-    const int ib = blockIdx.x, NQ = 2 * S + 3;
-    const double *tot = D.tot + (size_t)ib * WS_TQ;
-    if (ib > 0) {
-      const double nel = D.nelec[ib];
-      double *xp = D.sl + (size_t)ib * 6 * S + 3 * S, *zp = xp + 2 * S;
-      for (int c = tid; c < S; c += blockDim.x) {
-        const double dQ = nel * D.npop[c] * K_E;
-        const double fjp = dQ > 0.0 ? P.factjp0 / dQ : 0.0;
-        const double sx = fjp * tot[2 * c], sy = fjp * tot[2 * c + 1];
-        xp[c] = xp[c] + P.CdeltT * sx;
-        zp[c] = zp[c] + P.CdeltT * sy;
-      }
-    }
-    if (tid < 3) {
-      double v = ib > 0 ? tot[2 * S + tid] : 0.0;
-      for (int w = 0; w < WS_WG / 64; w++) v += tot[NQ + 3 * w + tid];
-      D.ion[((size_t)slot * P.G + ib) * 3 + tid] = v;
-    }
-    return;
-  }
-  const int kb = (blockIdx.x - nkick) * blockDim.x + tid;
-  if (kb >= P.h) return;
-  double z = 0.0;
-  const int b = bunch_of_bucket[kb];
-  if (b >= 0) {
-    const double *zz = D.sl + (size_t)b * 6 * P.S + 4 * P.S;
-    for (int ic = 0; ic < P.S; ic++) z = z + zz[ic];
-    z = z / ((double)P.S);
-  }
-  D.zcm[(size_t)slot * P.h + kb] = z;
-}
-
 // ================================================================ host side
 
 struct mbt_ws {
@@ -919,16 +962,16 @@ struct mbt_ws {
   hipStream_t stream;
   WSP P;
   WSD D;
-  int *d_bucket, *d_fill, *d_npop, *d_nofe, *d_bob;
-  double *d_Ibunch, *d_nelec, *d_convion;
-  int *bucket_h, *fill_h;
+  int *d_bucket, *d_npop, *d_nofe;
+  double *d_wallcur, *d_nelec, *d_convion;
+  int *bucket_h;
   int npop_h[WS_S];
   double *dist; // generated macro-electrons [6][Np]
   double *nelec_h;
   long long rev;
   int maxblk;
   int serial;          // bunch-by-bunch relay instead of the ion-parallel train
-  double *d_dtime;
+  double *d_dtime, *d_wall;
   long long *d_toff;
   int timing;         // HIP events around the ion train of every turn
   hipEvent_t *ev;     // [2 WS_T] train start / end per turn of a block
@@ -954,9 +997,9 @@ extern "C" void mbt_ws_destroy(mbt_ws *w)
   if (!w) return;
   (void)hipSetDevice(w->device);
   if (w->stream) (void)hipStreamSynchronize(w->stream); // turns of mbt_ws_track_async may still run
-  void *p[] = {w->D.sl,  w->D.hist, w->D.Exy, w->D.li,     w->D.cl,     w->D.part,    w->D.psum,
-               w->D.done, w->D.cm,  w->D.mon,  w->D.ion, w->D.zcm,    w->d_bucket, w->d_fill,    w->d_npop,
-               w->d_nofe, w->d_bob, w->d_Ibunch, w->d_nelec, w->d_convion, w->D.tpart, w->d_dtime, w->d_toff,
+  void *p[] = {w->D.sl,  w->D.dip, w->d_wall, w->D.Exy, w->D.li,     w->D.cl,     w->D.part,    w->D.psum,
+               w->D.done, w->D.cm,  w->D.mon,  w->D.ion, w->D.zcm,    w->d_bucket, w->d_npop,
+               w->d_nofe, w->d_wallcur, w->d_nelec, w->d_convion, w->D.tpart, w->d_dtime, w->d_toff,
                w->D.tot};
   for (size_t i = 0; i < sizeof p / sizeof p[0]; i++)
     if (p[i]) (void)hipFree(p[i]);
@@ -965,7 +1008,6 @@ extern "C" void mbt_ws_destroy(mbt_ws *w)
   free(w->ev);
   if (w->stream) (void)hipStreamDestroy(w->stream);
   free(w->bucket_h);
-  free(w->fill_h);
   free(w->dist);
   free(w->nelec_h);
   free(w);
@@ -1031,9 +1073,7 @@ extern "C" int mbt_ws_create(const mbt_config *c, int device, int flags, mbt_ws 
     return rc;
   }
   w->bucket_h = (int *)malloc(sizeof(int) * G);
-  w->fill_h = (int *)malloc(sizeof(int) * H);
   memcpy(w->bucket_h, c->bucket, sizeof(int) * G);
-  memcpy(w->fill_h, c->nfFill, sizeof(int) * H);
   double *Ib = (double *)calloc(H, sizeof(double));
   if (flags & MBT_WS_BUNCH_CURRENTS) memcpy(Ib, c->Ibunch, sizeof(double) * H);
   // ---- constants (glibc on the host, the reference's expressions)
@@ -1056,6 +1096,7 @@ extern "C" int mbt_ws_create(const mbt_config *c, int device, int flags, mbt_ws 
   P.Urad = c->Urad;
   P.T0 = c->T0;
   P.ac = c->ac;
+  double prfrw[2], prfrw_trig[2]; // wake strengths of the resistive wall, the second with the trigger
   for (int p = 0; p < 3; p++) {
     P.gamma1[p] = c->gamma1[p];
     P.alpha1[p] = c->alpha1[p];
@@ -1081,16 +1122,14 @@ extern "C" int mbt_ws_create(const mbt_config *c, int device, int flags, mbt_ws 
       P.rwa12[pl] = +c->beta1[plane] * sp;
       const double kappa = 1.0 / 2.8e-08;
       double beff3 = pow(plane == 1 ? c->beffH[0] : c->beffV[0], 3);
-      P.prfrw[pl] = 2.0 * c->R / (beff3) / sqrt(M_PI * kappa * K_EPS0) / 1.0;
+      prfrw[pl] = 2.0 * c->R / (beff3) / sqrt(M_PI * kappa * K_EPS0) / 1.0;
       beff3 = pow(2.0e-3, 3);
-      P.prfrw_trig[pl] = 2.0 * c->R / (beff3) / sqrt(M_PI * kappa * K_EPS0) / 1.0;
+      prfrw_trig[pl] = 2.0 * c->R / (beff3) / sqrt(M_PI * kappa * K_EPS0) / 1.0;
     }
   }
   P.triggerRW = c->triggerRW;
-  P.Pref0 = c->T0 / c->E0 / c->fNp / MBT_FTERA;
   P.fNp = c->fNp;
-  P.Dub0 = c->Lc / ((double)c->Nharm);
-  P.Lc = c->Lc;
+  for (int i = 0; i < S; i++) P.ntot += w->npop_h[i];
   P.factBE = sqrt(2 * (c->sgm_xx * c->sgm_xx - c->sgm_zz * c->sgm_zz)) / MBT_FKILO;
   P.sxx = c->sgm_xx;
   P.szz = c->sgm_zz;
@@ -1109,10 +1148,12 @@ extern "C" int mbt_ws_create(const mbt_config *c, int device, int flags, mbt_ws 
     P.CdeltT = K_C * P.deltT;
     P.dtF = P.deltT * P.factF;
     w->nelec_h = (double *)malloc(sizeof(double) * G);
-    double *conv = (double *)malloc(sizeof(double) * G);
+    const double Pref0 = c->T0 / c->E0 / c->fNp / MBT_FTERA;
+    double *conv = (double *)malloc(sizeof(double) * G), *wcur = (double *)malloc(sizeof(double) * G);
     for (int b = 0; b < G; b++) {
       w->nelec_h[b] = (Ib[c->bucket[b]] * c->T0 / (c->Np * K_E * MBT_FKILO));
       conv[b] = w->nelec_h[b] * Ldmsgm;
+      wcur[b] = c->nfFill[c->bucket[b]] ? Pref0 * Ib[c->bucket[b]] : 0.0; // only filled buckets act
     }
     // ---- device memory
     const size_t npts = (size_t)S * 25;
@@ -1120,12 +1161,32 @@ extern "C" int mbt_ws_create(const mbt_config *c, int device, int flags, mbt_ws 
     WA(w->d_npop, S);
     WA(w->d_nofe, npts);
     WA(w->d_bucket, G);
-    WA(w->d_fill, H);
-    WA(w->d_bob, H);
-    WA(w->d_Ibunch, H);
+    WA(w->d_wallcur, G);
     WA(w->d_nelec, G);
     WA(w->d_convion, G);
-    WA(w->D.hist, (size_t)4 * H * WS_HIST);
+    if (P.rw) {
+      // the wake W = prf / sqrt(D / c) of every distance a dipole can act over, D =
+      // d buckets (d = h: the bunch's own, one turn) and j turns
+      const size_t nw = (size_t)4 * (c->Nmlt + 1) * H;
+      double *wl = (double *)malloc(sizeof(double) * nw);
+      const double Dub0 = c->Lc / ((double)c->Nharm);
+      for (int t = 0, i = 0; t < 2; t++)
+        for (int pl = 0; pl < 2; pl++)
+          for (int j = 0; j <= c->Nmlt; j++)
+            for (int d = 1; d <= H; d++, i++) {
+              const double D0 = d == H ? c->Lc : ((double)d) * Dub0, Du = D0 + ((double)j) * c->Lc;
+              const double Dt = Du / K_C;
+              wl[i] = (t ? prfrw_trig[pl] : prfrw[pl]) / sqrt(Dt);
+            }
+      const int rca = walloc(&w->d_wall, nw);
+      if (!rca && hipMemcpy(w->d_wall, wl, sizeof(double) * nw, hipMemcpyHostToDevice) != hipSuccess) rc = MBT_EDEVICE;
+      free(wl);
+      if (rca || rc) {
+        mbt_ws_destroy(w);
+        return rca ? rca : rc;
+      }
+      WA(w->D.dip, (size_t)2 * WS_RING * G);
+    }
     WA(w->D.Exy, (size_t)G * npts);
     WA(w->D.li, (size_t)5 * G * npts);
     // train: drift times, then the ion-parallel form's partials (one block
@@ -1168,37 +1229,31 @@ extern "C" int mbt_ws_create(const mbt_config *c, int device, int flags, mbt_ws 
     WA(w->D.ion, (size_t)WS_T * G * 3);
     WA(w->D.zcm, (size_t)WS_T * H);
     double *sl = (double *)malloc(sizeof(double) * 6 * (size_t)S * G);
-    int *bob = (int *)malloc(sizeof(int) * H);
-    for (int kb = 0; kb < H; kb++) bob[kb] = -1;
-    for (int b = 0; b < G; b++) {
+    for (int b = 0; b < G; b++)
       memcpy(sl + (size_t)b * 6 * S, slices + (size_t)c->bucket[b] * 6 * S, sizeof(double) * 6 * S);
-      bob[c->bucket[b]] = b;
-    }
     WUP(w->D.sl, sl, (size_t)G * 6 * S);
     WUP(w->d_npop, w->npop_h, S);
     WUP(w->d_nofe, nofe, npts);
     WUP(w->d_bucket, w->bucket_h, G);
-    WUP(w->d_fill, w->fill_h, H);
-    WUP(w->d_bob, bob, H);
-    WUP(w->d_Ibunch, Ib, H);
+    WUP(w->d_wallcur, wcur, G);
     WUP(w->d_nelec, w->nelec_h, G);
     WUP(w->d_convion, conv, G);
     CK(hipStreamSynchronize(w->stream));
     free(sl);
-    free(bob);
     free(conv);
+    free(wcur);
   }
   free(slices);
   free(Ib);
   w->D.npop = w->d_npop;
   w->D.nofe = w->d_nofe;
   w->D.bucket = w->d_bucket;
-  w->D.fill = w->d_fill;
-  w->D.Ibunch = w->d_Ibunch;
+  w->D.wallcur = w->d_wallcur;
   w->D.nelec = w->d_nelec;
   w->D.convion = w->d_convion;
   w->D.dtime = w->d_dtime;
   w->D.toff = w->d_toff;
+  w->D.wall = w->d_wall;
   *out = w;
   return MBT_OK;
 }
@@ -1219,37 +1274,50 @@ static int ws_download(mbt_ws *w, long n, double *cm, double *mon, double *ion, 
 // when timing is on).
 static int ws_enqueue(mbt_ws *w, long n)
 {
-  const int G = w->P.G, H = w->P.h;
-  const size_t lds2 = sizeof(double) * 2 * H;
-  // phase 1: a block per bunch, and with FBII one thread per grid point of
-  // every slice of every bunch (for the fields, then the ions)
-  const long long np = (long long)G * w->P.S * 25;
-  const int nbp = (int)((np + WS_WG - 1) / WS_WG), nb1 = w->P.fbii && nbp > G ? nbp : G;
-  const int nkick = w->P.fbii && !w->serial ? G : 0;
+  const int G = w->P.G, S = w->P.S;
+  const size_t lds = sizeof(double) * ws_electrons_lds(S, G);
+  const bool fbii = w->P.fbii != 0, relay = fbii && w->serial;
+  // phase 1 with FBII: a block per bunch, then one thread per grid point of every
+  // slice of every bunch (for the fields, then the ions)
+  const long long np = (long long)G * S * 25;
+  const int nbp = (int)((np + WS_WG - 1) / WS_WG);
   CK(hipMemsetAsync(w->D.mon, 0, sizeof(double) * 18 * G * n, w->stream));
   CK(hipMemsetAsync(w->D.ion, 0, sizeof(double) * 3 * G * n, w->stream));
+  int kick = -1; // slot of the turn whose ion kicks are still to apply
   for (long t = 0; t < n; t++) {
     const long long rev = w->rev;
-    const int monitor = rev % w->cfg.NrevMon == 0;
-    hipLaunchKernelGGL(k_ws_phase1, dim3(nb1), dim3(WS_WG), 0, w->stream, w->P, w->D, rev, (int)t, monitor);
-    CK(hipGetLastError());
-    if (w->P.fbii) {
-      // the ions start from the slices' positions before the betatron rotation
-      hipLaunchKernelGGL(k_ws_create, dim3(nbp), dim3(WS_WG), 0, w->stream, w->P, w->D);
+    WSStep T = {kick, -1, 0, rev, (int)t, rev % w->cfg.NrevMon == 0};
+    kick = -1;
+    if (!fbii) {
+      if (t > 0) {
+        T.rev2 = rev - 1;
+        T.slot2 = (int)t - 1;
+      }
+      hipLaunchKernelGGL(k_ws_step, dim3(G), dim3(WS_STEP_WG), lds, w->stream, w->P, w->D, T);
       CK(hipGetLastError());
+      w->rev++;
+      continue;
     }
-    hipLaunchKernelGGL(k_ws_phase2, dim3(G), dim3(WS_WG), lds2, w->stream, w->P, w->D, rev);
+    hipLaunchKernelGGL(k_ws_phase1, dim3(G + nbp), dim3(WS_WG), lds, w->stream, w->P, w->D, T);
     CK(hipGetLastError());
-    if (w->timing && w->P.fbii) CK(hipEventRecord(w->ev[2 * t], w->stream));
-    if (w->P.fbii && !w->serial) {
+    // the ions start from the slices' positions before the betatron rotation
+    hipLaunchKernelGGL(k_ws_create, dim3(nbp), dim3(WS_WG), 0, w->stream, w->P, w->D);
+    CK(hipGetLastError());
+    const WSStep T2 = {-1, rev, (int)t, -1, 0, 0};
+    if (!relay) {
+      if (w->timing) CK(hipEventRecord(w->ev[2 * t], w->stream));
       hipLaunchKernelGGL(k_ws_ions, dim3(w->D.nblk_ions), dim3(WS_WG), sizeof(double2) * 2 * WS_QT * min(w->P.S, WS_CH),
                          w->stream, w->P, w->D);
       CK(hipGetLastError());
       if (w->timing) CK(hipEventRecord(w->ev[2 * t + 1], w->stream));
-      hipLaunchKernelGGL(k_ws_ksum, dim3(G, (2 * w->P.S + 3 + KSUM_Q - 1) / KSUM_Q + 1), dim3(64 * KSUM_Q), 0,
-                         w->stream, w->P, w->D);
+      hipLaunchKernelGGL(k_ws_ksum, dim3(G, (2 * S + 3 + KSUM_Q - 1) / KSUM_Q + 2), dim3(64 * KSUM_Q), lds, w->stream,
+                         w->P, w->D, T2);
       CK(hipGetLastError());
-    } else if (w->P.fbii) {
+      kick = (int)t;
+    } else {
+      hipLaunchKernelGGL(k_ws_step, dim3(G), dim3(WS_STEP_WG), lds, w->stream, w->P, w->D, T2);
+      CK(hipGetLastError());
+      if (w->timing) CK(hipEventRecord(w->ev[2 * t], w->stream));
       hipLaunchKernelGGL(k_ws_cloud_reset, dim3(1), dim3(WS_WG), 0, w->stream, w->P, w->D, (int)t);
       CK(hipGetLastError());
       for (int ib = 1; ib < G; ib++) {
@@ -1262,10 +1330,13 @@ static int ws_enqueue(mbt_ws *w, long n)
       }
       if (w->timing) CK(hipEventRecord(w->ev[2 * t + 1], w->stream));
     }
-    hipLaunchKernelGGL(k_ws_end, dim3(nkick + (H + 255) / 256), dim3(256), 0, w->stream, w->P, w->D, w->d_bob, (int)t,
-                       nkick);
-    CK(hipGetLastError());
     w->rev++;
+  }
+  // what the last turn leaves: its phase 2 (without FBII) or its train's kicks
+  const WSStep T = {kick, fbii ? -1 : w->rev - 1, (int)n - 1, -1, 0, 0};
+  if (n > 0 && (!fbii || kick >= 0)) {
+    hipLaunchKernelGGL(k_ws_step, dim3(G), dim3(WS_STEP_WG), lds, w->stream, w->P, w->D, T);
+    CK(hipGetLastError());
   }
   return MBT_OK;
 }
