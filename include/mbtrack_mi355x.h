@@ -270,7 +270,8 @@ int mbt_ring_rf_state(const mbt_ring *r, int ring, double *out);
  * (src/worker_weakweak.c:203-219). */
 int mbt_ring_rw_history(const mbt_ring *r, double *out);
 /* Kernel timing of the last mbt_ring_track call, milliseconds per kernel class:
- * [0] turn map pass, [1] per-bunch reduction, [2] LR recurrence, [3] RW sum. */
+ * [0] turn map pass, [1] per-bunch reduction, [2] turn end with the LR
+ * recurrence and RF feedback, [3] RW sum (for small rings with the turn end). */
 int mbt_ring_kernel_times(const mbt_ring *r, double *ms, long *launches);
 /* Bytes of HBM the turn map pass must move per turn (algorithmic). */
 double mbt_ring_bytes_per_turn(const mbt_ring *r);

@@ -15,22 +15,21 @@
 //   k_reduce  per bunch: statistics (src/statistics.c:91-195), RW dipole history,
 //             LR histograms (src/transform_weak.c:839-865) and the selffield
 //             convolutions for the next turn (src/transform_weak.c:633-731);
-//   k_rw_fresh, k_end (large rings) or k_rw (small rings)
+//   k_rw_fresh (large rings) or k_rw (small rings)
 //             per bunch: resistive-wall long-range sum over (Nmlt+1) h past
 //             buckets (src/transform_weak.c:780-833), applied as a pending kick
 //             at the start of the next pass; for large rings the taps of earlier
 //             turns' rows are summed by k_turn's leading blocks during the map
-//             and k_rw_fresh adds this turn's row after k_reduce; then the turn
-//             end.  For ensembles of rings sharing one tap table the sum is one
-//             MFMA GEMM instead (k_rwg_tile, k_rwg_sum, then k_end);
-//   k_lr_par  with long-range resonators: the phasor recurrence over all buckets
-//             and the RF-feedback samples (construct_wake_phasor
-//             src/transform_weak.c:961-1048), linear, so one block per resonator
-//             with the buckets in parallel and one short chain over bucket start
-//             phasors (also for the replayed turns of wake_phasor_init); k_lr
-//             keeps the one-lane recurrence (the reference's arithmetic) for
-//             h > 1365; then k_lr_sum and k_fb_solve, the RF-feedback solve
-//             (src/worker_weakweak.c:268-278).
+//             and k_rw_fresh adds this turn's row after k_reduce.  For ensembles
+//             of rings sharing one tap table the sum is one MFMA GEMM instead
+//             (k_rwg_tile, k_rwg_sum);
+//   k_ring_end one block per ring: the turn end and, with long-range resonators,
+//             the phasor recurrence over all buckets (construct_wake_phasor
+//             src/transform_weak.c:961-1048) as a scan of affine maps, the
+//             RF-feedback samples and the RF-feedback solve
+//             (src/worker_weakweak.c:268-278); what it needs of each bunch's
+//             histogram, and the bunch's own wake, k_reduce makes, and the next
+//             k_turn adds the incoming phasor's wake to its kick tables.
 //
 // Determinism: histogram dipole sums are accumulated as exact 128-bit fixed-point
 // integers (LDS then global integer atomics), moment sums by fixed-order
@@ -79,10 +78,8 @@
 #define AUTOTUNE_ROUNDS 3
 #define AUTOTUNE_REPS 2
 #define MAX_CHUNK_ITEMS 64
-#define LR_PREFETCH 16
-// dynamic LDS of the bucket-parallel LR recurrence (6 doubles per bucket): up
-// to h = 1365; larger rings use the one-lane recurrence
-#define LR_PAR_LDS_MAX (64 * 1024)
+// buckets per lane and pass of the phasor scan
+#define LR_SEG 8
 // Coordinates in tiles of TILE slots: tile t holds coordinate k (tau, delta,
 // x, x', z, z') of slots t TILE .. t TILE + TILE - 1 at (6 t + k) TILE, so a
 // work-group's chunk reads and writes six 32 KB runs of one 192 KB region.
@@ -120,6 +117,8 @@
 // reference's formulas so that every constant equals the reference's.
 struct DevParams {
   int ring, Nb, h, Nc, Nmlt;
+  int lrp[4];       // first long-range resonator of the planes LON, HOR, VER and the end
+  long long lr_off; // of the ring's [h + 1][resonators] entries in LRDev::L and V
   // bound on |x| and |z| of a particle whose dipole enters the exact fixed-point
   // slice sums: min(2^20, 2^27 / Np), so that the sum of a whole bunch stays
   // inside the 128-bit range (|sum| < 2^27 at the quantum 2^-100); a particle
@@ -175,12 +174,29 @@ struct LRConst {
   int ring, plane, l, fb;
   int h, bucket_off;
   int init_turns; // wake_phasor_init replay length Nbumax / h
-  long long lrc_off;
   double pr0, pr1;   // one bin
   double ge, gc, gs; // bucket gap
   double ee, ec, es; // empty bucket
   double pb0, pb1, pa0, pa1;
   double fac;
+};
+
+// Long-range resonators.  Buckets are visited from the last to the first, so the
+// per-bucket arrays run over m = h - 1 - bucket.  A filled bucket that finds the
+// phasor V leaves G (p^Nc V - I fac L) behind, L = sum_j f_j p^(Nc-1-j) over its
+// slices (one bin turns the phasor by p, the gap after the slices by G), and its
+// slice j feels
+//   Re(p^(j+1) V) - I fac (f_j / 2 + sum_(k<j) f_k Re p^(j-k)):
+// the incoming phasor's wake and a convolution of the bunch's own histogram.
+struct LRDev {
+  const LRConst *lc;
+  const double2 *pw; // [resonator][Nc + 1] p^k
+  double2 *L;        // per ring [m][resonator] slice sums of the last turn's histograms
+  double2 *V;        // per ring [m][resonator] phasor each bucket finds; row h: after the turn
+  const double *G;   // [ring][3][Nc] own wake of a plane's resonators per unit of current
+  double *self;      // [3][bunches][Nc] its convolution with the histogram, per unit of current
+  double *fb_hist;
+  int Gtot;
 };
 
 // ---------------------------------------------------------------- device math
@@ -492,6 +508,22 @@ __device__ void rw_old_tile(const DevParams *__restrict__ Pr, const RwOld &RO, i
   }
 }
 
+// Wake of the ring's long-range resonators of plane pl at slice i of bunch b
+// (bucket kb, current I [mA]): resonators in order, then the bunch's own part.
+__device__ __forceinline__ double lr_wake_at(const DevParams &P, const LRDev &R, int b, int kb, int pl, int i, double I)
+{
+  const int r0 = P.lrp[pl], r1 = P.lrp[pl + 1];
+  if (r0 == r1) return 0.0;
+  const int Nc = P.Nc, nr = P.lrp[3] - P.lrp[0];
+  const double2 *V = R.V + P.lr_off + (long long)(P.h - 1 - kb) * nr - P.lrp[0];
+  double w = 0.0;
+  for (int r = r0; r < r1; r++) {
+    const double2 v = V[r], p = R.pw[(size_t)r * (Nc + 1) + i + 1];
+    w += v.x * p.x - v.y * p.y;
+  }
+  return w + I * R.self[((size_t)pl * R.Gtot + b) * Nc + i];
+}
+
 template <int MODE, bool QE, bool DIP, bool GEN, bool MON>
 __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams *__restrict__ Pr, Coords C,
                                                                 const long long *wg_first, const long long *wg_end,
@@ -499,7 +531,7 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
                                                                 const int *bucket, const long long *bunch_first,
                                                                 const double *shift, const double *sfL,
                                                                 const double *sfV, const double *sfH,
-                                                                const double *lr_wake, long long lr_plane_stride,
+                                                                LRDev LR, const double *Ibunch,
                                                                 const double *pending, double *partial, HistPtr H,
                                                                 const TurnState *__restrict__ tsr, RwOld RO)
 {
@@ -533,9 +565,8 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
   const int tid = threadIdx.x;
   const long long rev = ts->rev;
   const bool do_hist = Nc > 0 && MODE != MODE_FINAL;
-  const double *lrL = lr_wake + (size_t)(P.bucket_off + kb) * Nc;
-  const double *lrH = lrL + lr_plane_stride;
-  const double *lrV = lrH + lr_plane_stride;
+  const bool lr = P.lrp[3] > P.lrp[0];
+  const double Ikb = lr ? Ibunch[P.bucket_off + kb] : 0.0;
 
   if (DIP)
     for (int i = tid; i < 2 * Nc; i += WG) {
@@ -545,9 +576,16 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
   for (int i = tid; i < Nc; i += WG) {
     lcnt[i] = 0;
     if (MODE == MODE_TURN || MODE == MODE_TUNE) {
-      if (P.kickL) kL[i] = sfL[(size_t)b * Nc + i] + lrL[i];
-      if (P.kickV) kV[i] = sfV[(size_t)b * Nc + i] + lrV[i];
-      if (P.kickH) kH[i] = sfH[(size_t)b * Nc + i] + lrH[i];
+      double l = P.kickL ? sfL[(size_t)b * Nc + i] : 0.0, v = P.kickV ? sfV[(size_t)b * Nc + i] : 0.0,
+             h = P.kickH ? sfH[(size_t)b * Nc + i] : 0.0;
+      if (lr) {
+        l += lr_wake_at(P, LR, b, kb, 0, i, Ikb);
+        if (P.kickV) v += lr_wake_at(P, LR, b, kb, 2, i, Ikb);
+        if (P.kickH) h += lr_wake_at(P, LR, b, kb, 1, i, Ikb);
+      }
+      if (P.kickL) kL[i] = l;
+      if (P.kickV) kV[i] = v;
+      if (P.kickH) kH[i] = h;
     }
   }
   if (tid < 8) ltr[tid] = 0;
@@ -792,8 +830,6 @@ struct RedOut {
   double *amp;       // [STATS_TURNS][G][6]
   double *shift;     // [G][6]
   double *rwhist;    // per ring [(Nmlt+2)h][2] at rw_off
-  double *fnp_ring;  // [3][H*Nc]
-  long long plane_stride; // H*Nc
   double *sfL, *sfV, *sfH;
   double *fnp_out, *dipV_out, *dipH_out; // last clamped histograms [G*Nc]
   int *trash_tot;    // [G*2] cumulative (consumed)
@@ -806,12 +842,37 @@ struct RedOut {
   int R;
 };
 
+// sum over k = 0 .. i of src[k] g[i - k] by the Q lanes of a group (q: the lane's
+// place): terms i - q, i - q - Q, ... per lane, then a fixed tree; every lane of
+// the group returns the sum.  MIXED: the terms in compensated FP32.
+__device__ __forceinline__ double conv_at(const double *src, const double *g, int i, int q, int Q, int mixed)
+{
+  double a = 0.0;
+  if (mixed) {
+    F2 s = {0.0f, 0.0f};
+    for (int k = i - q; k >= 0; k -= Q) f2_add_prod(s, src[k], g[i - k]);
+    a = (double)s.hi + (double)s.lo;
+  } else {
+#pragma unroll 4
+    for (int k = i - q; k >= 0; k -= Q) a += src[k] * g[i - k];
+  }
+  for (int o = Q >> 1; o >= 1; o >>= 1) a += __shfl_xor(a, o, Q);
+  return a;
+}
+
 // phase: 0 = means only (shift <- mean), 1 = initial statistics + RW history
-// fill, 2 = turn, 3 = final statistics
-__global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr, const double *partial,
-                                               const int *bunch_wg0, const int *bunch_ring, const int *bucket,
-                                               HistPtr H, RedOut R, const TurnState *__restrict__ tsr, int phase,
-                                               const int *lr_planes, int dip)
+// fill, 2 = turn, 3 = final statistics.
+// Bound: latency (one block per bunch, a chain of loads, sums and convolutions).
+// The convolutions take two slices i and Nc - 1 - i per group of Q lanes, so that
+// every lane has the same (Nc + 1) / Q terms and only the planes that have a wake
+// are visited: 333 bunches x 50 slices with the sums and own wakes of three
+// resonators 26.7 -> 14.7 us (one lane per slice and plane before), 416 x 100
+// without resonators 18.6 -> 17.
+__global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr, const double *__restrict__ partial,
+                                               const int *__restrict__ bunch_wg0, const int *__restrict__ bunch_ring,
+                                               const int *__restrict__ bucket, HistPtr H, RedOut R,
+                                               const TurnState *__restrict__ tsr, int phase, int dip, LRDev LR,
+                                               int lr_lds)
 {
   extern __shared__ double sm[];
   const int b = blockIdx.x, tid = threadIdx.x;
@@ -824,10 +885,16 @@ __global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr,
   double *dV = fnp + Nc;
   double *dH = dV + Nc;
   double *Gs = dH + Nc;  // the ring's three Green's functions, [plane][Nc]
+  // with LR resonators: their own wakes, [plane][Nc], in LDS where it holds them,
+  // and the edge slices' sums without the particles beyond them
+  const double *Gl = lr_lds ? Gs + 3 * Nc : LR.G + (size_t)ring * 3 * Nc;
+  __shared__ double edge[3][2];
   __shared__ double mom[NMOM];
   __shared__ int icmin_s, icmax_s;
   const long long rev = ts->rev;
   const int w0 = bunch_wg0[b], w1 = bunch_wg0[b + 1];
+  // the final statistics leave the wakes of the next turn alone
+  const bool lrp = (phase == 1 || phase == 2) && P.lrp[3] > P.lrp[0];
   const double Np = (double)R.np[b];
   {
     // moment sums over the bunch's workgroups: 16 lanes per moment, each summing
@@ -835,6 +902,7 @@ __global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr,
     const int q = tid >> 4, j = tid & 15;
     double s = 0.0;
     if (q < NMOM)
+#pragma unroll 4
       for (int w = w0 + j; w < w1; w += 16) s += partial[(size_t)w * NMOM + q];
     for (int o = 8; o >= 1; o >>= 1) s += __shfl_xor(s, o, 16);
     if (q < NMOM && j == 0) mom[q] = s;
@@ -842,6 +910,10 @@ __global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr,
   if (phase != 0 && Nc > 0) {
     const double *Gr = R.G + (size_t)ring * 3 * Nc;
     for (int i = tid; i < 3 * Nc; i += WG) Gs[i] = Gr[i];
+    if (lrp && lr_lds) {
+      const double *Lr = LR.G + (size_t)ring * 3 * Nc;
+      for (int i = tid; i < 3 * Nc; i += WG) Gs[3 * Nc + i] = Lr[i];
+    }
   }
   if (tid == 0) {
     icmin_s = Nc - 1;
@@ -849,60 +921,39 @@ __global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr,
   }
   __syncthreads();
   const int slot = (int)(((rev % STATS_TURNS) + STATS_TURNS) % STATS_TURNS);
-  if (tid == 0) {
-    double st[12];
-    const int track[3] = {1, P.track_h, P.track_v};
-    for (int pl = 0; pl < 3; pl++) {
-      int cp = 2 * pl, cs = 2 * pl + 1;
-      double mp = mom[cp] / Np, ms = mom[cs] / Np;
-      double pos = R.shift[b * 6 + cp] + mp, slope = R.shift[b * 6 + cs] + ms;
-      double vp = mom[6 + cp] / Np - mp * mp, vs = mom[6 + cs] / Np - ms * ms;
-      st[pl] = track[pl] ? pos : 0.0;
-      st[3 + pl] = track[pl] ? sqrt(vp > 0.0 ? vp : 0.0) : 0.0;
-      st[6 + pl] = track[pl] ? slope : 0.0;
-      st[9 + pl] = track[pl] ? sqrt(vs > 0.0 ? vs : 0.0) : 0.0;
-    }
-    if (phase == 0) {
-      for (int pl = 0; pl < 3; pl++) {
-        R.shift[b * 6 + 2 * pl] = st[pl];
-        R.shift[b * 6 + 2 * pl + 1] = st[6 + pl];
-      }
-    } else {
-      double *o = R.stats + ((size_t)slot * R.Gtot + b) * 12;
-      for (int i = 0; i < 12; i++) o[i] = st[i];
-      for (int pl = 0; pl < 3; pl++) {
-        R.shift[b * 6 + 2 * pl] = st[pl];
-        R.shift[b * 6 + 2 * pl + 1] = st[6 + pl];
-      }
-      if (phase == 2 && b == P.bunch_off) {
-        // nothing changes phai0 / Vrf0 between the map and this point of the turn
-        R.rfbuf[((size_t)slot * R.R + ring) * 2] = ts->phai0;
-        R.rfbuf[((size_t)slot * R.R + ring) * 2 + 1] = ts->Vrf0;
-      }
+  if (tid < 6) {
+    // one lane per coordinate (tau, delta, x, x', z, z')
+    const int pl = tid >> 1, c = tid & 1;
+    const bool track = pl == 0 || (pl == 1 ? P.track_h : P.track_v);
+    const double mp = mom[tid] / Np, v = mom[6 + tid] / Np - mp * mp;
+    const double mean = track ? R.shift[b * 6 + tid] + mp : 0.0;
+    R.shift[b * 6 + tid] = mean;
+    if (phase != 0) {
+      double *o = R.stats + ((size_t)slot * R.Gtot + b) * 12 + 6 * c + pl;
+      o[0] = mean;
+      o[3] = track ? sqrt(v > 0.0 ? v : 0.0) : 0.0;
       if (phase == 2 && (rev + 1) % P.monitor_every == 0) {
-        double *a = R.amp + ((size_t)slot * R.Gtot + b) * 6;
-        for (int pl = 0; pl < 3; pl++) {
-          a[pl] = track[pl] ? mom[12 + pl] / Np : 0.0;
-          a[3 + pl] = track[pl] ? P.gamma1[pl] * (st[pl] * st[pl]) + 2.0 * P.alpha1[pl] * st[pl] * st[6 + pl] +
-                                      P.beta1[pl] * (st[6 + pl] * st[6 + pl])
-                                : 0.0;
-        }
+        const double other = __shfl_xor(mean, 1, 2), pos = c ? other : mean, slope = c ? mean : other;
+        double *a = R.amp + ((size_t)slot * R.Gtot + b) * 6 + 3 * c + pl;
+        *a = !track ? 0.0
+                    : (c == 0 ? mom[12 + pl] / Np
+                              : P.gamma1[pl] * (pos * pos) + 2.0 * P.alpha1[pl] * pos * slope +
+                                    P.beta1[pl] * (slope * slope));
       }
-      if (P.rw && phase != 3) {
-        double *hist = R.rwhist + P.rw_off;
-        long long n = (long long)(P.Nmlt + 2) * P.h;
-        long long k = (phase == 1 ? 0 : -rev * P.h) + kb;
-        long long idx = ((k % n) + n) % n;
-        hist[2 * idx] = st[1];
-        hist[2 * idx + 1] = st[2];
+      if (P.rw && phase != 3 && c == 0 && pl > 0) {
+        double *hist = R.rwhist + P.rw_off + pl - 1;
+        const long long n = (long long)(P.Nmlt + 2) * P.h;
+        const long long k = (phase == 1 ? 0 : -rev * P.h) + kb;
+        hist[2 * (((k % n) + n) % n)] = mean;
         if (phase == 1)
-          for (int jj = 1; jj < P.Nmlt; jj++) {
-            long long i2 = ((long long)jj * P.h + kb) % n;
-            hist[2 * i2] = st[1];
-            hist[2 * i2 + 1] = st[2];
-          }
+          for (int jj = 1; jj < P.Nmlt; jj++) hist[2 * (((long long)jj * P.h + kb) % n)] = mean;
       }
     }
+  }
+  if (phase == 2 && b == P.bunch_off && tid == 64) {
+    // nothing changes phai0 / Vrf0 between the map and this point of the turn
+    R.rfbuf[((size_t)slot * R.R + ring) * 2] = ts->phai0;
+    R.rfbuf[((size_t)slot * R.R + ring) * 2 + 1] = ts->Vrf0;
   }
   if (phase == 0 || Nc <= 0) {
     // consume (and clear) the histogram only on the stats passes
@@ -927,10 +978,9 @@ __global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr,
   // dipole sums at the zeros the last clear wrote, so they are neither read
   // nor cleared here (the outputs get the same zeros)
   const bool bad = H.bad[b] != 0;
-  const size_t lrrow = (size_t)(P.bucket_off + kb) * Nc;
   for (int i = tid; i < Nc; i += WG) {
     size_t g = (size_t)b * Nc + i;
-    double cnt = (double)H.cnt[g];
+    unsigned int c = H.cnt[g];
     unsigned long long xl = 0, xh = 0, zl = 0, zh = 0;
     if (dip) {
       xl = H.sx[2 * g];
@@ -938,39 +988,33 @@ __global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr,
       zl = H.sz[2 * g];
       zh = H.sz[2 * g + 1];
     }
-    double sx = bad ? NAN : fx_to_double(xl, xh);
-    double sz = bad ? NAN : fx_to_double(zl, zh);
-    if (lr_planes[0]) R.fnp_ring[lrrow + i] = cnt;
-    if (lr_planes[1]) R.fnp_ring[R.plane_stride + lrrow + i] = sx;
-    if (lr_planes[2]) R.fnp_ring[2 * R.plane_stride + lrrow + i] = sz;
-    // clamped: out-of-range particles join the edge bins
-    unsigned int c = H.cnt[g];
-    for (int tt = 0; tt < 2; tt++) {
-      if (!((tt == 0 && i == 0) || (tt == 1 && i == Nc - 1))) continue;
-      c += H.tcnt[2 * b + tt];
-      if (!dip) continue;
-      unsigned long long al = H.tsx[4 * b + 2 * tt], ah = H.tsx[4 * b + 2 * tt + 1];
-      unsigned long long nl = xl + al;
-      xh = xh + ah + (nl < xl ? 1ULL : 0ULL);
-      xl = nl;
-      al = H.tsz[4 * b + 2 * tt];
-      ah = H.tsz[4 * b + 2 * tt + 1];
-      nl = zl + al;
-      zh = zh + ah + (nl < zl ? 1ULL : 0ULL);
-      zl = nl;
+    if (i == 0 || i == Nc - 1) {
+      // dropped: the sums of the edge slices alone; clamped: out-of-range
+      // particles join them (one slice takes both edges)
+      for (int e = 0; e < 2; e++) {
+        if (i != (e ? Nc - 1 : 0)) continue;
+        edge[0][e] = (double)H.cnt[g];
+        edge[1][e] = bad ? NAN : fx_to_double(dip ? H.sx[2 * g] : 0, dip ? H.sx[2 * g + 1] : 0);
+        edge[2][e] = bad ? NAN : fx_to_double(dip ? H.sz[2 * g] : 0, dip ? H.sz[2 * g + 1] : 0);
+        c += H.tcnt[2 * b + e];
+        if (!dip) continue;
+        fx_add(xl, xh, H.tsx[4 * b + 2 * e], H.tsx[4 * b + 2 * e + 1]);
+        fx_add(zl, zh, H.tsz[4 * b + 2 * e], H.tsz[4 * b + 2 * e + 1]);
+      }
     }
-    fnp[i] = (double)c;
     // icellmin / icellmax of src/transform_weak.c:633-651: the first and last
     // occupied slice (Nc - 1 and 0 when there is none)
     if (c > 0) {
       atomicMin(&icmin_s, i);
       atomicMax(&icmax_s, i);
     }
-    dV[i] = bad ? NAN : fx_to_double(zl, zh);
-    dH[i] = bad ? NAN : fx_to_double(xl, xh);
-    R.fnp_out[g] = fnp[i];
-    R.dipV_out[g] = dV[i];
-    R.dipH_out[g] = dH[i];
+    const double n = (double)c, sz = bad ? NAN : fx_to_double(zl, zh), sx = bad ? NAN : fx_to_double(xl, xh);
+    fnp[i] = n;
+    dV[i] = sz;
+    dH[i] = sx;
+    R.fnp_out[g] = n;
+    R.dipV_out[g] = sz;
+    R.dipH_out[g] = sx;
   }
   if (tid == 0) {
     // trash counters: the previous pending binning is consumed by this turn's kick
@@ -1005,59 +1049,86 @@ __global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr,
   if (phase == 2 && P.scan == 1 && (rev + 1) % P.NrevScan == 0) Ib += P.scan_step / (((double)P.Nb) * 1.0e3);
   const double factG = -P.T0 * Ib / (R.np[b] * P.E0 * 1.0e9);
   const double sgm = P.sigma_tau, sgm2 = sgm * sgm, dT2 = P.dT * P.dT;
-  // one (plane, slice) convolution per task; tasks run from the last slice down
-  // so that the second sweep of the block gets the short ones
-  for (int t = tid; t < 3 * Nc; t += WG) {
-    const int pl = t % 3, i = Nc - 1 - t / 3;
-    const double *Gp = Gs + pl * Nc;
-    const double *src = pl == 0 ? fnp : (pl == 1 ? dV : dH);
-    double val = 0.0;
-    if (pl == 0) {
-      if (P.convL && i >= icmin) {
-        double Gn = 0.0;
-        if (P.mixed) {
-          F2 g = {0.0f, 0.0f};
-          for (int k = i; k >= icmin; k--) f2_add_prod(g, src[k], Gp[i - k]);
-          Gn = (double)g.hi + (double)g.lo;
-        } else {
-#pragma unroll 4
-          for (int k = i; k >= icmin; k--) Gn += src[k] * Gp[i - k];
-        }
-        double GL1 = 1 * Gn;
-        // resistive and inductive smoothing, src/transform_weak.c:670-683; reads
-        // outside [0, Ncell) count as zero
-#define F(q) (((q) >= 0 && (q) < Nc) ? fnp[q] : 0.0)
-        if (P.RsisL > 0 && i >= icmin + 1 && i <= icmax) {
-          double nt = (0.5 * F(i - 1) + F(i) + 0.5 * F(i + 1)) / 2.0;
-          GL1 += P.RsisL * nt / (sgm * P.dT);
-        }
-        if (P.aindL > 0 && i >= icmin + 1 && i <= icmax) {
-          double n0 = (0.25 * F(i - 3) + 0.5 * F(i - 2) + F(i - 1) + 0.5 * F(i) + 0.25 * F(i + 1)) / 2.5;
-          double n1 = (0.25 * F(i - 1) + 0.5 * F(i) + F(i + 1) + 0.5 * F(i + 2) + 0.25 * F(i + 3)) / 2.5;
-          GL1 += (n1 - n0) / (2.0 * sgm2 * dT2) * P.aindL;
-        }
+  const int np2 = (Nc + 1) >> 1; // pairs of slices (i, Nc - 1 - i)
+  int Q = 16;
+  while (Q > 1 && Q * np2 > WG) Q >>= 1;
+  const int q = tid & (Q - 1);
+  if (P.convL || P.kickV || P.kickH || P.sf_active)
+    for (int t = tid / Q; t < np2; t += WG / Q)
+      for (int half = 0; half < 2; half++) {
+        const int i = half ? t : Nc - 1 - t;
+        if (half && i == Nc - 1 - t) break; // the middle slice of an odd count
+        const size_t g = (size_t)b * Nc + i;
+        {
+          double val = 0.0;
+          if (P.convL && i >= icmin) {
+            // slices below icmin are empty: nothing to add from them
+            double GL1 = conv_at(fnp, Gs, i, q, Q, P.mixed);
+            // resistive and inductive smoothing, src/transform_weak.c:670-683; reads
+            // outside [0, Ncell) count as zero
+#define F(k) (((k) >= 0 && (k) < Nc) ? fnp[k] : 0.0)
+            if (P.RsisL > 0 && i >= icmin + 1 && i <= icmax) {
+              double nt = (0.5 * F(i - 1) + F(i) + 0.5 * F(i + 1)) / 2.0;
+              GL1 += P.RsisL * nt / (sgm * P.dT);
+            }
+            if (P.aindL > 0 && i >= icmin + 1 && i <= icmax) {
+              double n0 = (0.25 * F(i - 3) + 0.5 * F(i - 2) + F(i - 1) + 0.5 * F(i) + 0.25 * F(i + 1)) / 2.5;
+              double n1 = (0.25 * F(i - 1) + 0.5 * F(i) + F(i + 1) + 0.5 * F(i + 2) + 0.25 * F(i + 3)) / 2.5;
+              GL1 += (n1 - n0) / (2.0 * sgm2 * dT2) * P.aindL;
+            }
 #undef F
-        val = GL1;
-      }
-      R.sfL[(size_t)b * Nc + i] = factG * val;
-    } else {
-      if (pl == 1 ? P.kickV : (P.kickH && i >= 1)) {
-        double Gn = 0.0;
-        if (P.mixed) {
-          F2 g = {0.0f, 0.0f};
-          for (int k = i; k >= 0; k--) f2_add_prod(g, src[k], Gp[i - k]);
-          Gn = (double)g.hi + (double)g.lo;
-        } else {
-#pragma unroll 4
-          for (int k = i; k >= 0; k--) Gn += src[k] * Gp[i - k];
+            val = GL1;
+          }
+          if (q == 0) R.sfL[g] = factG * val;
         }
-        val = 1 * Gn;
+        // a plane without a kick keeps the +0.0 of its allocation (its value
+        // here, -factG * 0 with factG <= 0), so its table is not rewritten
+        if (P.kickV) {
+          const double val = conv_at(dV, Gs + Nc, i, q, Q, P.mixed);
+          if (q == 0) R.sfV[g] = -factG * val;
+        }
+        if (P.kickH) {
+          const double val = i >= 1 ? conv_at(dH, Gs + 2 * Nc, i, q, Q, P.mixed) : 0.0;
+          if (q == 0) R.sfH[g] = -factG * val;
+        }
       }
-      // a plane without a kick keeps the +0.0 of its allocation (its value
-      // here, -factG * 0 with factG <= 0), so its table is not rewritten
-      if (pl == 1 ? P.kickV : P.kickH) (pl == 1 ? R.sfV : R.sfH)[(size_t)b * Nc + i] = -factG * val;
-    }
+  else
+    for (int i = tid; i < Nc; i += WG) R.sfL[(size_t)b * Nc + i] = factG * 0.0;
+  if (!lrp) return;
+  // ---- LR resonators: the histograms without the particles beyond the edges
+  __syncthreads();
+  if (tid < 6) {
+    const int pl = tid >> 1, e = tid & 1;
+    (pl == 0 ? fnp : (pl == 1 ? dH : dV))[e ? Nc - 1 : 0] = edge[pl][e];
   }
+  __syncthreads();
+  // slice sums the phasor recurrence needs, one wave per resonator
+  const int nr = P.lrp[3] - P.lrp[0];
+  for (int r = P.lrp[0] + (tid >> 6); r < P.lrp[3]; r += WG / 64) {
+    const double *f = r < P.lrp[1] ? fnp : (r < P.lrp[2] ? dH : dV);
+    const double2 *p = LR.pw + (size_t)r * (Nc + 1);
+    double sr = 0.0, si = 0.0;
+    for (int j = tid & 63; j < Nc; j += 64) {
+      const double2 w = p[Nc - 1 - j];
+      sr += f[j] * w.x;
+      si += f[j] * w.y;
+    }
+    sr = wave_sum(sr);
+    si = wave_sum(si);
+    if ((tid & 63) == 0)
+      LR.L[P.lr_off + (long long)(P.h - 1 - kb) * nr + r - P.lrp[0]] = make_double2(sr, si);
+  }
+  // the bunch's own long-range wake
+  for (int t = tid / Q; t < np2; t += WG / Q)
+    for (int half = 0; half < 2; half++) {
+      const int i = half ? t : Nc - 1 - t;
+      if (half && i == Nc - 1 - t) break;
+      for (int pl = 0; pl < 3; pl++) {
+        if (P.lrp[pl] == P.lrp[pl + 1]) continue;
+        const double a = conv_at(pl == 0 ? fnp : (pl == 1 ? dH : dV), Gl + pl * Nc, i, q, Q, 0);
+        if (q == 0) LR.self[((size_t)pl * LR.Gtot + b) * Nc + i] = a;
+      }
+    }
 }
 
 // ------------------------------------------------------------- k_rw_fresh, k_rw
@@ -1458,299 +1529,178 @@ __global__ __launch_bounds__(256) void k_rwg_sum(RWGemm Gm, const DevParams *__r
   pending[2 * g + pl] = on ? (P.fNp * sum) * P.rwconst[pl][trig] : 0.0;
 }
 
-// Turn end, one block per ring, for turns without a resistive-wall pass;
-// with fb_here also the RF-feedback step (no long-range resonators anywhere).
-__global__ void k_end(const DevParams *__restrict__ Pr, TurnState *tsr, double *bunch_Ib, double *Ibunch,
-                      const int *nfFill, int fb_here)
-{
-  if (threadIdx.x != 0) return;
-  const int ring = blockIdx.x;
-  TurnState *ts = tsr + ring;
-  end_turn(Pr[ring], ts, bunch_Ib, Ibunch, nfFill);
-  if (fb_here) fb_solve(Pr[ring], ts, nullptr, 0);
-}
+// ------------------------------------------------------------ turn end, LR
 
-// ------------------------------------------------------------------- k_lr
-
-// One lane per long-range resonator (of any ring): the recurrence of
-// construct_wake_phasor (src/transform_weak.c:961-1048) or, with init set,
-// wake_phasor_init (:869-952).  Constants come from the host (glibc exp/cos/sin),
-// the update order is the reference's, so the phasors are bit-identical.
-__global__ void k_lr(int nres, const LRConst *lc, const DevParams *__restrict__ Pr, const double *fnp_ring,
-                     long long plane_stride, const double *Ibunch, const int *nfFill, int Nc, double *phasor_end,
-                     double *lrc, double *fb_hist, TurnState *tsr, int init)
+__device__ __forceinline__ void fb_sample(double *fbh, int fb_len, long long c, double2 V, double p0, double p1)
 {
-  int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= nres) return;
-  const LRConst L = lc[r];
-  const DevParams &P = Pr[L.ring];
-  TurnState *ts = tsr + L.ring;
-  const int h = L.h;
-  const double *fnp = fnp_ring + (size_t)L.plane * plane_stride + (size_t)L.bucket_off * Nc;
-  const double *Ib = Ibunch + L.bucket_off;
-  const int *fill = nfFill + L.bucket_off;
-  double *__restrict__ out = lrc + L.lrc_off;
-  double *__restrict__ fbh = fb_hist + P.fbh_off;
-  const int fb_len = P.fb_len;
-  const int nturn = init ? L.init_turns : 1;
-  if (nturn <= 0) return;
-  double Vo0, Vo1, Vn0, Vn1;
-  if (init) {
-    Vo0 = 0.0;
-    Vo1 = 0.0;
-  } else {
-    Vo0 = phasor_end[2 * r];
-    Vo1 = phasor_end[2 * r + 1];
-  }
-  Vn0 = phasor_end[2 * r];
-  Vn1 = phasor_end[2 * r + 1];
-  const bool fb = L.fb && ts->has_fb;
-  long long cnt = ts->fb_count;
-  for (int k = 0; k < nturn; k++)
-    for (int m = 0; m < h; m++) {
-      int i = h - m - 1;
-      if (fb) {
-        double vr = Vn0 * L.pb0 - Vn1 * L.pb1, vi = Vn0 * L.pb1 + Vn1 * L.pb0;
-        unsigned key = ((unsigned)cnt % (unsigned)fb_len) * 2;
-        fbh[key] = sqrt(vr * vr + vi * vi);
-        fbh[key + 1] = atan2(vr, vi);
-        cnt++;
-      }
-      if (fill[i] == 1) {
-        double Ii = Ib[i];
-        const double *__restrict__ f = fnp + (size_t)i * Nc;
-        double *__restrict__ o = out + (size_t)i * Nc;
-        // the recurrence is latency-bound: fetch the bucket's slice values a
-        // block ahead of the dependent chain
-        for (int j0 = 0; j0 < Nc; j0 += LR_PREFETCH) {
-          double fv[LR_PREFETCH];
-#pragma unroll
-          for (int k2 = 0; k2 < LR_PREFETCH; k2++) fv[k2] = j0 + k2 < Nc ? f[j0 + k2] : 0.0;
-#pragma unroll
-          for (int k2 = 0; k2 < LR_PREFETCH; k2++) {
-            if (j0 + k2 >= Nc) break;
-            Vn0 = (Vo0 * L.pr0 - Vo1 * L.pr1) - Ii * fv[k2] * L.fac;
-            Vn1 = (Vo0 * L.pr1 + Vo1 * L.pr0);
-            if (!init) o[j0 + k2] = Vn0 + 0.5 * Ii * fv[k2] * L.fac;
-            Vo0 = Vn0;
-            Vo1 = Vn1;
-          }
-        }
-        Vn0 = (Vo0 * L.ge * L.gc - Vo1 * L.ge * L.gs);
-        Vn1 = (Vo0 * L.ge * L.gs + Vo1 * L.ge * L.gc);
-        Vo0 = Vn0;
-        Vo1 = Vn1;
-      } else {
-        Vn0 = (Vo0 * L.ee * L.ec - Vo1 * L.ee * L.es);
-        Vn1 = (Vo0 * L.ee * L.es + Vo1 * L.ee * L.ec);
-        Vo0 = Vn0;
-        Vo1 = Vn1;
-      }
-      if (fb) {
-        double vr = Vn0 * L.pa0 - Vn1 * L.pa1, vi = Vn0 * L.pa1 + Vn1 * L.pa0;
-        unsigned key = ((unsigned)cnt % (unsigned)fb_len) * 2;
-        fbh[key] = sqrt(vr * vr + vi * vi);
-        fbh[key + 1] = atan2(vr, vi);
-        cnt++;
-      }
-    }
-  phasor_end[2 * r] = Vn0;
-  phasor_end[2 * r + 1] = Vn1;
-  if (fb) ts->fb_count = cnt;
-}
-
-// The per-turn recurrence of one resonator with its buckets in parallel (one
-// block per resonator).  The recurrence is linear: a filled bucket maps its
-// start phasor V to G (p^Nc V + L), with L the bucket's own sum started from
-// zero, an empty one to E V.  Phase A: every bucket's L (one lane per bucket,
-// the recurrence's own operations); phase B: one lane chains the h start
-// phasors; phase C: every bucket replays its slices from its start phasor
-// (again the recurrence's own operations) and writes the slice terms and the
-// RF-feedback samples.  Only the start phasors are rounded differently from
-// the sequential loop (by the closed form of phase B).  Dynamic LDS: 6 h doubles.
-__device__ __forceinline__ void fb_sample(double *fbh, int fb_len, long long c, double v0, double v1, double p0,
-                                          double p1)
-{
-  const double vr = v0 * p0 - v1 * p1, vi = v0 * p1 + v1 * p0;
+  const double vr = V.x * p0 - V.y * p1, vi = V.x * p1 + V.y * p0;
   const unsigned key = ((unsigned)c % (unsigned)fb_len) * 2;
   fbh[key] = sqrt(vr * vr + vi * vi);
   fbh[key + 1] = atan2(vr, vi);
 }
 
-__global__ __launch_bounds__(256) void k_lr_par(const LRConst *lc, const DevParams *__restrict__ Pr,
-                                                const double *fnp_ring, long long plane_stride, const double *Ibunch,
-                                                const int *nfFill, int Nc, double *phasor_end, double *lrc,
-                                                double *fb_hist, TurnState *tsr, int init)
+__device__ __forceinline__ double2 cmul(double2 a, double2 b)
 {
-  extern __shared__ double lsm[];
-  __shared__ double Pn[2];
-  const int r = blockIdx.x, tid = threadIdx.x, nth = blockDim.x;
-  const LRConst L = lc[r];
-  const DevParams &P = Pr[L.ring];
-  TurnState *ts = tsr + L.ring;
-  const int h = L.h;
-  const double *fnp = fnp_ring + (size_t)L.plane * plane_stride + (size_t)L.bucket_off * Nc;
-  const double *Ib = Ibunch + L.bucket_off;
-  const int *fill = nfFill + L.bucket_off;
-  double *__restrict__ out = lrc + L.lrc_off;
-  double *__restrict__ fbh = fb_hist + P.fbh_off;
-  const int fb_len = P.fb_len;
-  const bool fb = L.fb && ts->has_fb;
-  const long long cnt0 = ts->fb_count;
-  // wake_phasor_init (init): the same turn replayed init_turns times from a
-  // zero phasor without slice terms (src/transform_weak.c:869-952)
-  const int nturn = init ? L.init_turns : 1;
-  if (nturn <= 0) return;
-  double *Lr = lsm, *Li = Lr + h, *Sr = Li + h, *Si = Sr + h, *Ar = Si + h, *Ai = Ar + h;
-  // ---- phase A
-  for (int i = tid; i < h; i += nth) {
-    double V0 = 0.0, V1 = 0.0;
-    if (fill[i] == 1) {
-      const double Ii = Ib[i];
-      const double *f = fnp + (size_t)i * Nc;
-      for (int j = 0; j < Nc; j++) {
-        const double n0 = (V0 * L.pr0 - V1 * L.pr1) - Ii * f[j] * L.fac;
-        const double n1 = (V0 * L.pr1 + V1 * L.pr0);
-        V0 = n0;
-        V1 = n1;
-      }
-    }
-    Lr[i] = V0;
-    Li[i] = V1;
-  }
-  if (tid == 0) {
-    double a = 1.0, b = 0.0;
-    for (int j = 0; j < Nc; j++) {
-      const double na = a * L.pr0 - b * L.pr1, nb = a * L.pr1 + b * L.pr0;
-      a = na;
-      b = nb;
-    }
-    Pn[0] = a;
-    Pn[1] = b;
-  }
-  __syncthreads();
-  // ---- phase B, in the recurrence's bucket order (last bucket first); when
-  // replaying (init) it also takes the feedback samples that survive in the
-  // sample ring, one lane in order
-  if (tid == 0) {
-    double V0 = init ? 0.0 : phasor_end[2 * r], V1 = init ? 0.0 : phasor_end[2 * r + 1];
-    double W0 = phasor_end[2 * r], W1 = phasor_end[2 * r + 1]; // what the first sample reads
-    const double g0 = L.ge * L.gc, g1 = L.ge * L.gs, e0 = L.ee * L.ec, e1 = L.ee * L.es;
-    const long long keep_init = cnt0 + 2LL * h * nturn - fb_len;
-    long long c = cnt0;
-    for (int k = 0; k < nturn; k++)
-      for (int m = 0; m < h; m++) {
-        const int i = h - m - 1;
-        if (init && fb) {
-          if (c >= keep_init) fb_sample(fbh, fb_len, c, W0, W1, L.pb0, L.pb1);
-          c++;
-        }
-        Sr[i] = V0;
-        Si[i] = V1;
-        if (fill[i] == 1) {
-          const double w0 = (V0 * Pn[0] - V1 * Pn[1]) + Lr[i], w1 = (V0 * Pn[1] + V1 * Pn[0]) + Li[i];
-          V0 = w0 * g0 - w1 * g1;
-          V1 = w0 * g1 + w1 * g0;
-        } else {
-          const double n0 = V0 * e0 - V1 * e1, n1 = V0 * e1 + V1 * e0;
-          V0 = n0;
-          V1 = n1;
-        }
-        Ar[i] = V0;
-        Ai[i] = V1;
-        W0 = V0;
-        W1 = V1;
-        if (init && fb) {
-          if (c >= keep_init) fb_sample(fbh, fb_len, c, W0, W1, L.pa0, L.pa1);
-          c++;
-        }
-      }
-    phasor_end[2 * r] = V0;
-    phasor_end[2 * r + 1] = V1;
-  }
-  __syncthreads();
-  if (init) {
-    if (tid == 0 && fb) ts->fb_count = cnt0 + 2LL * h * nturn;
-    return;
-  }
-  // ---- phase C; of the 2 h feedback samples only the last fb_len survive in
-  // the sample ring, so only those are written (no two lanes share a slot)
-  const long long keep_from = cnt0 + 2LL * h - fb_len;
-  for (int i = tid; i < h; i += nth) {
-    if (fill[i] == 1) {
-      double V0 = Sr[i], V1 = Si[i];
-      const double Ii = Ib[i];
-      const double *f = fnp + (size_t)i * Nc;
-      double *o = out + (size_t)i * Nc;
-      for (int j = 0; j < Nc; j++) {
-        const double fj = f[j];
-        const double n0 = (V0 * L.pr0 - V1 * L.pr1) - Ii * fj * L.fac;
-        const double n1 = (V0 * L.pr1 + V1 * L.pr0);
-        o[j] = n0 + 0.5 * Ii * fj * L.fac;
-        V0 = n0;
-        V1 = n1;
-      }
-    }
-    if (fb) {
-      const long long c = cnt0 + 2LL * (h - i - 1);
-      if (c >= keep_from) fb_sample(fbh, fb_len, c, Sr[i], Si[i], L.pb0, L.pb1);
-      if (c + 1 >= keep_from) fb_sample(fbh, fb_len, c + 1, Ar[i], Ai[i], L.pa0, L.pa1);
-    }
-  }
-  __syncthreads(); // every lane has read the sample counter
-  if (tid == 0 && fb) ts->fb_count = cnt0 + 2LL * h;
+  return make_double2(a.x * b.x - a.y * b.y, a.x * b.y + a.y * b.x);
 }
 
-// lr_wake[plane][global bucket][j] = sum over the ring's resonators of that
-// plane, in order, of their terms
-__global__ void k_lr_sum(const int *lr_first, const LRConst *lc, const double *lrc, const DevParams *__restrict__ Pr,
-                         const int *bunch_ring, const int *bucket, int G, int Nc, int4 planes,
-                         long long plane_stride, double *lr_wake)
+__device__ __forceinline__ double2 cadd(double2 a, double2 b) { return make_double2(a.x + b.x, a.y + b.y); }
+
+__device__ __forceinline__ double2 shfl_up2(double2 v, int d)
 {
-  // (plane among the planes.x active ones, bunch, slice): only the buckets of
-  // bunches are read by the kick; the rows of empty buckets and of planes
-  // without resonators stay zero from the allocation
-  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  const long long per = (long long)G * Nc;
-  if (e >= planes.x * per) return;
-  const int pi = (int)(e / per);
-  const int plane = pi == 0 ? planes.y : (pi == 1 ? planes.z : planes.w);
-  const long long bj = e % per;
-  const int b = (int)(bj / Nc), j = (int)(bj % Nc);
-  const int ring = bunch_ring[b];
-  const int q = Pr[ring].bucket_off + bucket[b];
-  double s = 0.0;
-  // the ring's resonators are contiguous in lc (ring-major, then plane, then index)
-  for (int r = lr_first[ring]; r < lr_first[ring + 1]; r++)
-    if (lc[r].plane == plane) s += lrc[lc[r].lrc_off + (size_t)(q - lc[r].bucket_off) * Nc + j];
-  lr_wake[plane * plane_stride + (long long)q * Nc + j] = s;
+  return make_double2(__shfl_up(v.x, d, 64), __shfl_up(v.y, d, 64));
 }
 
-// RF feedback, one lane per ring: rffb_calc_mean_voltage_phase
-// (src/feedback_rf.c:21-34) and the solve of src/worker_weakweak.c:268-278.
-// One wave per ring: the samples summed by 64 lanes (fixed order), then the solve.
-__global__ __launch_bounds__(64) void k_fb_solve(int nrings, const DevParams *__restrict__ Pr, TurnState *tsr,
-                                                 const double *fb_hist, int init)
+// One turn of resonator r by one wave: from the phasor V0 before the first bucket
+// (the last one of the ring) the phasor every bucket finds, stored; returns the
+// phasor after the turn (in every lane).  Each bucket is an affine map of the
+// phasor, so LR_SEG of them per lane are composed, the compositions scanned over
+// the wave, and every lane walks its own buckets from the phasor that reaches
+// them: about 30 dependent complex products a pass of 512 buckets instead of one
+// chain over them (which took 150 us a turn with its slices, 333 bunches in
+// 416 buckets x 50 slices, 3 resonators; the whole kernel now takes 12).
+// fbh: also take the feedback samples from number keep on (the first one is c0;
+// W: what the first reads).
+__device__ double2 lr_turn(const LRConst &L, const LRDev &R, const DevParams &P, int r, const double *Ib, const int *fill,
+                           double2 V0, double2 W, double *fbh, int fb_len, long long c0, long long keep)
 {
-  const int ring = blockIdx.x, lane = threadIdx.x;
-  if (ring >= nrings) return;
+  const int lane = threadIdx.x & 63, h = P.h, Nc = P.Nc, nr = P.lrp[3] - P.lrp[0];
+  const double2 g = make_double2(L.ge * L.gc, L.ge * L.gs), e = make_double2(L.ee * L.ec, L.ee * L.es);
+  const double2 mf = cmul(R.pw[(size_t)r * (Nc + 1) + Nc], g);
+  const double2 *Ls = R.L + P.lr_off + r - P.lrp[0];
+  double2 *Vs = R.V + P.lr_off + r - P.lrp[0];
+  for (int base = 0; base < h; base += 64 * LR_SEG) {
+    const int m0 = base + lane * LR_SEG;
+    double2 c[LR_SEG];
+    unsigned filled = 0;
+#pragma unroll
+    for (int k = 0; k < LR_SEG; k++) {
+      const int m = min(m0 + k, h - 1), bk = h - 1 - m;
+      const double2 l = Ls[m * nr];
+      const double a = -Ib[bk] * L.fac;
+      const bool f = fill[bk] == 1;
+      if (f) filled |= 1u << k;
+      c[k] = f ? cmul(make_double2(a * l.x, a * l.y), g) : make_double2(0.0, 0.0);
+    }
+    double2 A = make_double2(1.0, 0.0), B = make_double2(0.0, 0.0);
+#pragma unroll
+    for (int k = 0; k < LR_SEG; k++)
+      if (m0 + k < h) {
+        const double2 M = filled >> k & 1 ? mf : e;
+        A = cmul(M, A);
+        B = cadd(cmul(M, B), c[k]);
+      }
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const double2 Ap = shfl_up2(A, d), Bp = shfl_up2(B, d);
+      if (lane >= d) {
+        B = cadd(cmul(A, Bp), B);
+        A = cmul(A, Ap);
+      }
+    }
+    const double2 E = cadd(cmul(A, V0), B); // after the lane's buckets
+    double2 V = shfl_up2(E, 1);
+    if (lane == 0) V = V0;
+#pragma unroll
+    for (int k = 0; k < LR_SEG; k++)
+      if (m0 + k < h) {
+        Vs[(m0 + k) * nr] = V;
+        const double2 before = V, M = filled >> k & 1 ? mf : e;
+        V = cadd(cmul(M, V), c[k]);
+        if (fbh) {
+          const long long q = c0 + 2LL * (m0 + k);
+          if (q >= keep) fb_sample(fbh, fb_len, q, m0 + k == 0 ? W : before, L.pb0, L.pb1);
+          if (q + 1 >= keep) fb_sample(fbh, fb_len, q + 1, V, L.pa0, L.pa1);
+        }
+      }
+    V0 = make_double2(__shfl(E.x, 63, 64), __shfl(E.y, 63, 64));
+  }
+  if (lane == 0) Vs[h * nr] = V0;
+  return V0;
+}
+
+// One block per ring: the turn end (end), the phasors of its resonators (a wave
+// each), the RF-feedback samples and the RF-feedback solve.  init:
+// wake_phasor_init (src/transform_weak.c:869-952), the same turn replayed
+// init_turns times from a zero phasor, one wave in order taking the samples.
+__global__ __launch_bounds__(256) void k_ring_end(const DevParams *__restrict__ Pr, TurnState *tsr, double *bunch_Ib,
+                                                  double *Ibunch, const int *nfFill, LRDev R, int end, int init)
+{
+  const int ring = blockIdx.x, tid = threadIdx.x, lane = tid & 63, nw = blockDim.x >> 6;
   const DevParams &P = Pr[ring];
   TurnState *ts = tsr + ring;
-  const int has = ts->has_fb;
+  if (end && tid == 0) end_turn(P, ts, bunch_Ib, Ibunch, nfFill);
+  const int lr0 = P.lrp[0], nr = P.lrp[3] - lr0;
+  if (nr == 0) {
+    if (tid == 0) fb_solve(P, ts, R.fb_hist, init);
+    return;
+  }
+  __syncthreads();
+  const int h = P.h, fb_len = P.fb_len;
+  const double *Ib = Ibunch + P.bucket_off;
+  const int *fill = nfFill + P.bucket_off;
+  double *fbh = R.fb_hist + P.fbh_off;
+  const bool has = ts->has_fb;
+  const long long cnt0 = ts->fb_count;
+  long long cnt1 = cnt0;
+  for (int r = lr0 + (tid >> 6); r < lr0 + nr; r += nw) {
+    const LRConst &L = R.lc[r];
+    const double2 last = R.V[P.lr_off + (long long)h * nr + r - lr0];
+    if (!init) {
+      lr_turn(L, R, P, r, Ib, fill, last, last, nullptr, fb_len, 0, 0);
+      continue;
+    }
+    double2 V = make_double2(0.0, 0.0);
+    const long long all = 2LL * h * L.init_turns, keep = cnt0 + all - fb_len;
+    for (int k = 0; k < L.init_turns; k++) {
+      const long long c0 = cnt0 + 2LL * h * k;
+      V = lr_turn(L, R, P, r, Ib, fill, V, k == 0 ? last : V, L.fb && has && c0 + 2LL * h > keep ? fbh : nullptr,
+                  fb_len, c0, keep);
+    }
+  }
+  __syncthreads();
+  if (has)
+    for (int r = lr0; r < lr0 + nr; r++) {
+      const LRConst &L = R.lc[r];
+      if (!L.fb) continue;
+      cnt1 += 2LL * h * (init ? L.init_turns : 1);
+      if (init) continue;
+      // of the 2 h samples only the last fb_len survive in the sample ring, so only
+      // those are written (no two lanes share a slot)
+      const double2 *V = R.V + P.lr_off + r - lr0;
+      for (long long q = max(0LL, 2LL * h - fb_len) + tid; q < 2LL * h; q += blockDim.x) {
+        const int m = (int)(q >> 1);
+        if (q & 1) fb_sample(fbh, fb_len, cnt0 + q, V[(m + 1) * nr], L.pa0, L.pa1);
+        else fb_sample(fbh, fb_len, cnt0 + q, V[m * nr], L.pb0, L.pb1);
+      }
+    }
+  __syncthreads(); // the samples are written, every lane has read the sample counter
+  if (tid >= 64) return;
   if (lane == 0) {
     ts->phai0_prev = ts->phai0;
     ts->Vrf0_prev = ts->Vrf0;
+    ts->fb_count = cnt1;
   }
   if (!has) return;
-  const double *fbh = fb_hist + P.fbh_off;
+  // rffb_calc_mean_voltage_phase (src/feedback_rf.c:21-34): the samples summed by
+  // 64 lanes in a fixed order, then the solve
   double vs = 0.0, ps = 0.0;
-  for (int m = lane; m < P.fb_len; m += 64) {
+  for (int m = lane; m < fb_len; m += 64) {
     vs += fbh[2 * m];
     ps += fbh[2 * m + 1];
   }
   vs = wave_sum(vs);
   ps = wave_sum(ps);
   if (lane == 0) fb_apply(P, ts, vs, ps, init);
+}
+
+// The long-range wake of one bunch's slices (longitudinal), as the next turn adds it.
+__global__ void k_lr_row(const DevParams *__restrict__ Pr, LRDev R, const double *Ibunch, int ring, int b, int kb,
+                         double *out)
+{
+  const DevParams &P = Pr[ring];
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < P.Nc) out[i] = lr_wake_at(P, R, b, kb, 0, i, Ibunch[P.bucket_off + kb]);
 }
 
 // =============================================================== host side
@@ -1789,15 +1739,14 @@ struct mbt_ring {
   int chunk_items;   // macroparticles per lane of one work-group's chunk
   int min_items;     // smallest chunk the buffers allow (1 for small rings, else 4)
   int any_qe, any_dip, any_gen, nrev_mon;
-  int sf_any;
   Coords C;
   long long *wg_first, *wg_end, *bunch_first;
-  int *wg_bunch, *bunch_wg0, *bucket, *bunch_ring, *bucket_ring, *np, *nfFill, *lr_planes;
+  int *wg_bunch, *bunch_wg0, *bucket, *bunch_ring, *bucket_ring, *np, *nfFill;
   DevParams *P;
   double *partial, *shift;
   HistPtr Hs;
   RedOut Ro;
-  double *sfL, *sfV, *sfH, *lr_wake, *fnp_ring, *lrc;
+  double *sfL, *sfV, *sfH;
   double *Gf;
   double *pending, *rwhist, *sqrt_tt, *rsqrt_tt, *Ibunch, *bunch_Ib;
   double *peek; // one bunch's six coordinates in SoA order, for mbt_ensemble_get_bunch
@@ -1816,14 +1765,15 @@ struct mbt_ring {
   long graph_builds; // turn graphs captured and instantiated so far
   int place_candidates; // coordinate allocations tried at set-up
   double place_gbps;    // k_stream rate of the chosen one (0 when not searched)
+  LRDev LR;
   LRConst *lc;
-  int *lr_first; // [R+1] first resonator of each ring in lc
+  double2 *lr_pw, *lr_L, *lr_V;
+  double *lr_G, *lr_self, *lr_row; // lr_row: one bunch's long-range wake for mbt_ring_potentials
   int nres;
-  int lr_hmax; // largest h among the resonators' rings
-  int4 lr_planes_active; // x: planes with a resonator in some ring, y..w: those planes
-  double *phasor_end, *fb_hist;
+  double *fb_hist;
   long long rw_total, st_total, fbh_total;
   size_t lds_turn, lds_red;
+  int lr_lds; // k_reduce keeps the LR resonators' own wakes in LDS
   long long rev_host;
   double *pot_host;    // pinned staging of mbt_ring_potentials: 7 Nc doubles, then a TurnState
   long async_n;        // turns enqueued by mbt_ring_track_async, not yet collected (0: none)
@@ -1994,10 +1944,11 @@ extern "C" void mbt_ring_destroy(mbt_ring *r)
   if (r->pot_host) (void)hipHostFree(r->pot_host);
   void *ptrs[] = {r->C.s, r->wg_first, r->wg_end, r->bunch_first,
                   r->wg_bunch, r->bunch_wg0, r->bucket, r->bunch_ring, r->bucket_ring, r->np, r->nfFill,
-                  r->lr_planes, r->P, r->partial, r->shift, r->Hs.cnt, r->Hs.sx, r->Hs.sz, r->Hs.tcnt, r->Hs.tsx,
-                  r->Hs.tsz, r->Hs.bad, r->sfL, r->sfV, r->sfH, r->lr_wake, r->fnp_ring, r->lrc, r->Gf, r->pending, r->peek,
+                  r->P, r->partial, r->shift, r->Hs.cnt, r->Hs.sx, r->Hs.sz, r->Hs.tcnt, r->Hs.tsx,
+                  r->Hs.tsz, r->Hs.bad, r->sfL, r->sfV, r->sfH, r->Gf, r->pending, r->peek,
                   r->rwhist, r->sqrt_tt, r->rsqrt_tt, r->Ibunch, r->bunch_Ib, r->stats, r->amp, r->rfbuf, r->fnp_out,
-                  r->dipV_out, r->dipH_out, r->trash_tot, r->trash_pend, r->ts, r->rw_tiles, r->rw_part, r->ring_done, r->lc, r->lr_first, r->phasor_end, r->fb_hist,
+                  r->dipV_out, r->dipH_out, r->trash_tot, r->trash_pend, r->ts, r->rw_tiles, r->rw_part, r->ring_done, r->lc, r->lr_pw, r->lr_L,
+                  r->lr_V, r->lr_G, r->lr_self, r->lr_row, r->fb_hist,
                   r->rwg_col_ring, r->rwg_bucket_bunch, r->rwg_c, r->rwg_part};
   for (size_t i = 0; i < sizeof ptrs / sizeof ptrs[0]; i++)
     if (ptrs[i]) (void)hipFree(ptrs[i]);
@@ -2528,7 +2479,6 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
     r->any_qe |= P.qe;
     r->any_dip |= P.kickV || P.kickH || hh->lr_plane[1] || hh->lr_plane[2];
     r->any_gen |= P.ideal_hc || P.n_ahc > 0 || P.amp_dq;
-    r->sf_any |= P.sf_active;
   }
   r->G = G;
   r->H = H;
@@ -2584,7 +2534,6 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
   DA(r->bucket_ring, H);
   DA(r->np, G);
   DA(r->nfFill, H);
-  DA(r->lr_planes, 3);
   DA(r->P, R);
   DA(r->partial, (size_t)nwg * NMOM);
   DA(r->shift, (size_t)G * 6);
@@ -2598,8 +2547,6 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
   DA(r->sfL, (size_t)G * NcA);
   DA(r->sfV, (size_t)G * NcA);
   DA(r->sfH, (size_t)G * NcA);
-  DA(r->lr_wake, (size_t)3 * H * NcA);
-  DA(r->fnp_ring, (size_t)3 * H * NcA);
   DA(r->Gf, (size_t)R * 3 * NcA);
   DA(r->pending, (size_t)G * 2);
   {
@@ -2636,23 +2583,16 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
     for (int p = 0; p < 3; p++)
       if (r->rh[k].lr_plane[p]) nres += r->rh[k].cfg.n_lr[p];
   LRConst *lc = (LRConst *)calloc(nres > 0 ? nres : 1, sizeof(LRConst));
-  {
-    int act[3] = {0, 0, 0}, na = 0, pl[3] = {0, 0, 0};
-    for (int k = 0; k < R; k++)
-      for (int p = 0; p < 3; p++)
-        if (r->rh[k].lr_plane[p] && r->rh[k].cfg.n_lr[p] > 0) act[p] = 1;
-    for (int p = 0; p < 3; p++)
-      if (act[p]) pl[na++] = p;
-    r->lr_planes_active = make_int4(na, pl[0], pl[1], pl[2]);
-  }
-  int *lrf = (int *)calloc(R + 1, sizeof(int));
-  long long lrc_total = 0;
+  double2 *pwh = (double2 *)calloc((size_t)(nres > 0 ? nres : 1) * (NcA + 1), sizeof(double2));
+  double *lgh = (double *)calloc((size_t)R * 3 * NcA, sizeof(double));
+  long long lr_total = 0;
   {
     int ir = 0;
     for (int k = 0; k < R; k++) {
-      lrf[k] = ir;
+      r->Ph[k].lr_off = lr_total;
       const mbt_config *cf = &r->rh[k].cfg;
       for (int p = 0; p < 3; p++) {
+        r->Ph[k].lrp[p] = ir;
         if (!r->rh[k].lr_plane[p]) continue;
         for (int l = 0; l < cf->n_lr[p]; l++) {
           const mbt_lr_resonator *res = &cf->lr[p][l];
@@ -2661,11 +2601,8 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
           L.plane = p;
           L.l = l;
           L.h = (int)cf->Nharm;
-          if (L.h > r->lr_hmax) r->lr_hmax = L.h;
           L.bucket_off = r->Ph[k].bucket_off;
-          L.lrc_off = lrc_total;
           L.init_turns = (int)(cf->Nbumax / cf->h);
-          lrc_total += (long long)cf->Nharm * NcA;
           double alpha = res->wr * 0.5 / res->Qfactor;
           double Amp = 2 * alpha * res->Rs * cf->T0 / cf->E0 / MBT_FGIGA;
           double dTau = cf->dT * cf->sigma_tau;
@@ -2691,17 +2628,32 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
           L.pb1 = exp(C0 * taubeam) * sin(C1 * taubeam);
           L.pa0 = exp(C0 * taub2beam) * cos(C1 * taub2beam);
           L.pa1 = exp(C0 * taub2beam) * sin(C1 * taub2beam);
+          // powers of the one-bin rotation, and the wake of the bunch's own slices
+          double2 *pw = pwh + (size_t)(ir - 1) * (NcA + 1);
+          double *lg = lgh + ((size_t)k * 3 + p) * NcA;
+          long double a = 1.0L, b = 0.0L;
+          for (int j = 0; j <= NcA; j++) {
+            pw[j] = make_double2((double)a, (double)b);
+            if (j < NcA) lg[j] -= L.fac * (j ? (double)a : 0.5);
+            const long double na = a * L.pr0 - b * L.pr1, nb = a * L.pr1 + b * L.pr0;
+            a = na;
+            b = nb;
+          }
         }
       }
+      r->Ph[k].lrp[3] = ir;
+      lr_total += (long long)(ir - r->Ph[k].lrp[0]) * ((int)cf->Nharm + 1);
     }
   }
-  lrf[R] = nres;
   r->nres = nres;
   DA(r->lc, nres > 0 ? nres : 1);
-  DA(r->lr_first, R + 1);
-  UP(r->lr_first, lrf, R + 1);
-  DA(r->lrc, lrc_total > 0 ? lrc_total : 1);
-  DA(r->phasor_end, (size_t)2 * (nres > 0 ? nres : 1));
+  DA(r->lr_pw, (size_t)(nres > 0 ? nres : 1) * (NcA + 1));
+  DA(r->lr_L, lr_total > 0 ? lr_total : 1);
+  DA(r->lr_V, lr_total > 0 ? lr_total : 1);
+  DA(r->lr_G, (size_t)R * 3 * NcA);
+  DA(r->lr_self, nres > 0 ? (size_t)3 * G * NcA : 1);
+  DA(r->lr_row, NcA);
+  r->LR = {r->lc, r->lr_pw, r->lr_L, r->lr_V, r->lr_G, r->lr_self, r->fb_hist, G};
   // ---- uploads
   UP(r->bunch_first, bfirst, G);
   UP(r->np, nph, G);
@@ -2714,11 +2666,9 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
   UP(r->Gf, Gf, (size_t)R * 3 * NcA);
   UP(r->P, r->Ph, R);
   if (nres > 0) UP(r->lc, lc, nres);
-  {
-    int lp[3] = {0, 0, 0};
-    for (int k = 0; k < R; k++)
-      for (int p = 0; p < 3; p++) lp[p] |= r->rh[k].lr_plane[p];
-    UP(r->lr_planes, lp, 3);
+  if (nres > 0) {
+    UP(r->lr_pw, pwh, (size_t)nres * (NcA + 1));
+    UP(r->lr_G, lgh, (size_t)R * 3 * NcA);
   }
   if (st_total > 0) {
     double *st = (double *)malloc(st_total * sizeof(double));
@@ -2763,14 +2713,13 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
   free(bIb);
   free(Gf);
   free(lc);
-  free(lrf);
+  free(pwh);
+  free(lgh);
   RedOut &Ro = r->Ro;
   Ro.stats = r->stats;
   Ro.amp = r->amp;
   Ro.shift = r->shift;
   Ro.rwhist = r->rwhist;
-  Ro.fnp_ring = r->fnp_ring;
-  Ro.plane_stride = (long long)H * NcA;
   Ro.sfL = r->sfL;
   Ro.sfV = r->sfV;
   Ro.sfH = r->sfH;
@@ -2787,7 +2736,8 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
   Ro.R = R;
   r->use_graphs = !(flags & MBT_RING_NO_GRAPHS);
   r->lds_turn = turn_lds(Nc);
-  r->lds_red = (size_t)6 * NcA * 8 + 64;
+  r->lr_lds = nres > 0 && (size_t)9 * NcA * 8 + 64 <= 64 * 1024;
+  r->lds_red = (size_t)(r->lr_lds ? 9 : 6) * NcA * 8 + 64;
   if (r->lds_turn > 64 * 1024 || r->lds_red > 64 * 1024) {
     mbt_set_error("Ncell %d too large for the LDS histogram", Nc);
     mbt_ring_destroy(r);
@@ -2964,7 +2914,7 @@ extern "C" int mbt_ring_get_bunch(const mbt_ring *r, int ib, double *s) { return
 
 typedef void (*turn_kernel_t)(const DevParams *, Coords, const long long *, const long long *, const int *,
                               const int *, const int *, const long long *, const double *, const double *,
-                              const double *, const double *, const double *, long long, const double *, double *,
+                              const double *, const double *, LRDev, const double *, const double *, double *,
                               HistPtr, const TurnState *, RwOld);
 
 #define TK(Q, D, G, M) k_turn<MODE_TURN, Q, D, G, M>
@@ -2991,7 +2941,6 @@ static int launch_turn_pass(mbt_ring *r, int mode)
     const bool mon = ((r->rev_host + 1) % r->nrev_mon) == 0;
     k = g_turn_kernels[(r->any_qe ? 8 : 0) + (r->any_dip ? 4 : 0) + (r->any_gen ? 2 : 0) + (mon ? 1 : 0)];
   }
-  const long long stride = (long long)r->H * (r->Nc > 0 ? r->Nc : 1);
   // the turn pass also carries the resistive-wall tiles of earlier turns' rows
   RwOld ro = {};
   size_t lds = r->lds_turn;
@@ -3002,7 +2951,7 @@ static int launch_turn_pass(mbt_ring *r, int mode)
   }
   hipLaunchKernelGGL(k, dim3(r->nwg + ro.nlead), dim3(WG), lds, r->stream, r->P, r->C, r->wg_first, r->wg_end,
                      r->wg_bunch, r->bunch_ring, r->bucket, r->bunch_first, r->shift, r->sfL, r->sfV, r->sfH,
-                     r->lr_wake, stride, r->pending, r->partial, r->Hs, r->ts, ro);
+                     r->LR, r->Ibunch, r->pending, r->partial, r->Hs, r->ts, ro);
   CK(hipGetLastError());
   return MBT_OK;
 }
@@ -3013,46 +2962,18 @@ static int launch_reduce(mbt_ring *r, int phase)
   // pass only when a ring's kicks or LR resonators need them
   const int dip = phase != 2 || r->any_dip;
   hipLaunchKernelGGL(k_reduce, dim3(r->G), dim3(WG), r->lds_red, r->stream, r->P, r->partial, r->bunch_wg0,
-                     r->bunch_ring, r->bucket, r->Hs, r->Ro, r->ts, phase, r->lr_planes, dip);
+                     r->bunch_ring, r->bucket, r->Hs, r->Ro, r->ts, phase, dip, r->LR, r->lr_lds);
   CK(hipGetLastError());
   return MBT_OK;
 }
 
-static int launch_lr(mbt_ring *r, int init)
+// Turn end (end), long-range recurrence and RF-feedback solve of every ring.
+static int launch_ring_end(mbt_ring *r, int end, int init)
 {
-  if (r->nres == 0) return MBT_OK;
-  const long long stride = (long long)r->H * (r->Nc > 0 ? r->Nc : 1);
-  const size_t lds = sizeof(double) * 6 * (size_t)r->lr_hmax;
-  if (lds <= LR_PAR_LDS_MAX)
-    hipLaunchKernelGGL(k_lr_par, dim3(r->nres), dim3(256), lds, r->stream, r->lc, r->P, r->fnp_ring, stride,
-                       r->Ibunch, r->nfFill, r->Nc, r->phasor_end, r->lrc, r->fb_hist, r->ts, init);
-  else
-    hipLaunchKernelGGL(k_lr, dim3((r->nres + 63) / 64), dim3(64), 0, r->stream, r->nres, r->lc, r->P, r->fnp_ring,
-                       stride, r->Ibunch, r->nfFill, r->Nc, r->phasor_end, r->lrc, r->fb_hist, r->ts, init);
-  CK(hipGetLastError());
-  if (!init && r->lr_planes_active.x > 0) {
-    const long long tot = (long long)r->lr_planes_active.x * r->G * r->Nc;
-    hipLaunchKernelGGL(k_lr_sum, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, r->stream, r->lr_first, r->lc,
-                       r->lrc, r->P, r->bunch_ring, r->bucket, r->G, r->Nc, r->lr_planes_active,
-                       (long long)r->H * r->Nc, r->lr_wake);
-    CK(hipGetLastError());
-  }
-  return MBT_OK;
-}
-
-static int launch_fb_solve(mbt_ring *r, int init)
-{
-  hipLaunchKernelGGL(k_fb_solve, dim3(r->R), dim3(64), 0, r->stream, r->R, r->P, r->ts, r->fb_hist, init);
+  hipLaunchKernelGGL(k_ring_end, dim3(r->R), dim3(r->nres > 0 ? 256 : 64), 0, r->stream, r->P, r->ts, r->bunch_Ib,
+                     r->Ibunch, r->nfFill, r->LR, end, init);
   CK(hipGetLastError());
   return MBT_OK;
-}
-
-// Long-range recurrence and RF-feedback solve that precede a turn.
-static int pre_turn(mbt_ring *r)
-{
-  int rc;
-  if (r->sf_any && (rc = launch_lr(r, 0))) return rc;
-  return launch_fb_solve(r, 0);
 }
 
 static int download_slots(mbt_ring *r, long long rev0, long n, double *stats, double *ampinv, double *rf)
@@ -3116,10 +3037,10 @@ extern "C" int mbt_ring_prepare(mbt_ring *r, double *init_stats)
     CK(hipStreamSynchronize(r->stream));
     free(ts);
     // each resonator replays its ring's Nbumax / h turns (none when that is 0)
-    if ((rc = launch_lr(r, 1))) return rc;
-    if ((rc = launch_fb_solve(r, 1))) return rc;
+    if ((rc = launch_ring_end(r, 0, 1))) return rc;
   }
-  if ((rc = pre_turn(r))) return rc;
+  // the recurrence and the RF-feedback solve that precede the first turn
+  if ((rc = launch_ring_end(r, 0, 0))) return rc;
   CK(hipStreamSynchronize(r->stream));
   r->rev_host = 0;
   return MBT_OK;
@@ -3132,7 +3053,6 @@ extern "C" int mbt_ring_prepare(mbt_ring *r, double *init_stats)
 static int enqueue_turn(mbt_ring *r, hipEvent_t *E)
 {
   int rc;
-  const int lr_launch = r->sf_any && r->nres > 0;
   const int rw_split = r->rw_split;
   if (E) CK(hipEventRecord(E[0], r->stream));
   if ((rc = launch_turn_pass(r, MODE_TURN))) return rc;
@@ -3151,27 +3071,17 @@ static int enqueue_turn(mbt_ring *r, hipEvent_t *E)
     const long long tot = (long long)r->rwg.h * r->rwg.N;
     hipLaunchKernelGGL(k_rwg_sum, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, r->stream, r->rwg, r->P, r->ts,
                        r->pending);
-    CK(hipGetLastError());
-    hipLaunchKernelGGL(k_end, dim3(r->R), dim3(64), 0, r->stream, r->P, r->ts, r->bunch_Ib, r->Ibunch, r->nfFill,
-                       !lr_launch);
   } else if (rw_split) {
     hipLaunchKernelGGL(k_rw_fresh, dim3(r->G), dim3(WG), 0, r->stream, r->P, r->bunch_ring, r->rwhist, r->sqrt_tt,
                        r->Ibunch, r->nfFill, r->bucket, r->ts, r->rw_part, r->G, r->pending);
-    CK(hipGetLastError());
-    hipLaunchKernelGGL(k_end, dim3(r->R), dim3(64), 0, r->stream, r->P, r->ts, r->bunch_Ib, r->Ibunch, r->nfFill,
-                       !lr_launch);
   } else if (r->rw_total > 0)
     hipLaunchKernelGGL(k_rw, dim3(r->G), dim3(RW_WG), 0, r->stream, r->P, r->bunch_ring, r->rwhist, r->sqrt_tt,
-                       r->Ibunch, r->nfFill, r->bucket, r->pending, r->ts, r->ring_done, r->bunch_Ib, !lr_launch);
-  else
-    hipLaunchKernelGGL(k_end, dim3(r->R), dim3(64), 0, r->stream, r->P, r->ts, r->bunch_Ib, r->Ibunch, r->nfFill,
-                       !lr_launch);
+                       r->Ibunch, r->nfFill, r->bucket, r->pending, r->ts, r->ring_done, r->bunch_Ib, r->nres == 0);
   CK(hipGetLastError());
   if (E) CK(hipEventRecord(E[3], r->stream));
-  if (lr_launch) {
-    if ((rc = launch_lr(r, 0))) return rc;
-    if ((rc = launch_fb_solve(r, 0))) return rc;
-  }
+  // k_rw's last block ends the turn itself
+  const int end = r->rwg_on || rw_split || r->rw_total == 0;
+  if ((end || r->nres > 0) && (rc = launch_ring_end(r, end, 0))) return rc;
   if (E) CK(hipEventRecord(E[4], r->stream));
   r->rev_host++;
   return MBT_OK;
@@ -3401,8 +3311,11 @@ extern "C" int mbt_ring_potentials(const mbt_ring *r, int ib, double *out, doubl
   int ring = 0, local = ib;
   while (local >= r->rh[ring].cfg.Nbunch) local -= r->rh[ring++].cfg.Nbunch;
   const size_t Nc = r->Nc, off = (size_t)ib * Nc;
-  const size_t loff = (size_t)(r->Ph[ring].bucket_off + r->rh[ring].cfg.bucket[local]) * Nc;
-  const double *src[7] = {r->sfL + off, r->lr_wake + loff, r->fnp_out + off, r->sfV + off, r->dipV_out + off,
+  (void)hipGetLastError();
+  hipLaunchKernelGGL(k_lr_row, dim3((unsigned)((Nc + 255) / 256)), dim3(256), 0, r->stream, r->P, r->LR,
+                     (const double *)r->Ibunch, ring, ib, r->rh[ring].cfg.bucket[local], r->lr_row);
+  CK(hipGetLastError());
+  const double *src[7] = {r->sfL + off, r->lr_row, r->fnp_out + off, r->sfV + off, r->dipV_out + off,
                           r->sfH + off, r->dipH_out + off};
   // eight small copies into pinned memory, one wait
   double *stage = r->pot_host;
@@ -3540,7 +3453,6 @@ extern "C" int mbt_ring_autotune(mbt_ring *r, int *best_items, double *ms)
   CK(hipEventCreate(&e1));
   // the turn's own variant, run as a timing pass (coordinates unchanged)
   const turn_kernel_t k = g_tune_kernels[(r->any_qe ? 4 : 0) + (r->any_dip ? 2 : 0) + (r->any_gen ? 1 : 0)];
-  const long long stride = (long long)r->H * (r->Nc > 0 ? r->Nc : 1);
   // candidates interleaved over AUTOTUNE_ROUNDS rounds, each timed over
   // AUTOTUNE_REPS passes after one untimed pass; a candidate's time is its best
   // round (the least disturbed by clocks and other work)
@@ -3556,7 +3468,7 @@ extern "C" int mbt_ring_autotune(mbt_ring *r, int *best_items, double *ms)
         if (rep == 1) CK(hipEventRecord(e0, r->stream));
         hipLaunchKernelGGL(k, dim3(r->nwg), dim3(WG), r->lds_turn, r->stream, r->P, r->C, r->wg_first, r->wg_end,
                            r->wg_bunch, r->bunch_ring, r->bucket, r->bunch_first, r->shift, r->sfL, r->sfV, r->sfH,
-                           r->lr_wake, stride, r->pending, r->partial, r->Hs, r->ts, RwOld{});
+                           r->LR, r->Ibunch, r->pending, r->partial, r->Hs, r->ts, RwOld{});
         CK(hipGetLastError());
       }
       CK(hipEventRecord(e1, r->stream));
