@@ -102,6 +102,8 @@
 #define STC(v, p) (*(p) = (v))
 #endif
 #define MAXLR (3 * MBT_MAX_LR)
+// slices a work-group's LDS histograms take (81 KB with dipoles at the most)
+#define NCELL_MAX 1090
 
 #define CK(x)                                                                                    \
   do {                                                                                           \
@@ -129,6 +131,7 @@ struct DevParams {
   int bunch_off;  // first global bunch of the ring
   int bucket_off; // first global bucket of the ring
   long long rw_off, st_off; // offsets into the RW history and sqrt table
+  int flags; // the TF_ switches of the turn's map, one load per work-group
   int track_h, track_v;
   int qe, ideal_hc, amp_dq;
   int kickL, kickV, kickH; // selffield kick of the plane is applied
@@ -158,6 +161,10 @@ struct DevParams {
   int fb_len, fb_switch_off;
   long long fbh_off;
   double vrf_design, phi0_design;
+};
+
+enum {
+  TF_SF = 1, TF_KICK_L = 2, TF_KICK_V = 4, TF_KICK_H = 8, TF_TRACK_V = 16, TF_TRACK_H = 32, TF_IDEAL = 64, TF_AMP = 128
 };
 
 struct TurnState {
@@ -201,76 +208,92 @@ struct LRDev {
 
 // ---------------------------------------------------------------- device math
 
-// Philox4x32-10 and the QE normals: identical algorithm to the oracle's
-// orc_qe_normals (float Box-Muller from explicit-FMA polynomials), so the
-// normals are bit-identical on CPU and GPU.
+// Philox4x32-10 and the QE normals: the oracle's orc_qe_normals (float Box-Muller
+// from explicit-FMA polynomials) bit for bit.  With quantum excitation the turn
+// is VALU-bound, so each step is the fewest instructions that give the same
+// bits (checked over all 2^24 inputs of both Box-Muller functions): the product
+// of a Philox round as one v_mad_u64_u32, its three-way xor as one v_bitop3_b32,
+// no scaling of operands that cannot leave the normal range, no branches.  The
+// loop of k_turn with excitation went from 730 vector instructions a
+// macroparticle to 600 (with dipole histograms too from 790 to 615; see the note
+// at its loops for the time).
+__device__ __forceinline__ uint32_t xor3(uint32_t a, uint32_t b, uint32_t c)
+{
+  return __builtin_amdgcn_bitop3_b32(a, b, c, 0x96);
+}
+
 __device__ __forceinline__ void philox(uint32_t c[4], uint32_t k0, uint32_t k1)
 {
 #pragma unroll
   for (int r = 0; r < 10; r++) {
-    uint32_t lo0 = 0xD2511F53u * c[0], hi0 = __umulhi(0xD2511F53u, c[0]);
-    uint32_t lo1 = 0xCD9E8D57u * c[2], hi1 = __umulhi(0xCD9E8D57u, c[2]);
-    uint32_t n0 = hi1 ^ c[1] ^ k0, n2 = hi0 ^ c[3] ^ k1;
+    const uint64_t p0 = (uint64_t)0xD2511F53u * c[0], p1 = (uint64_t)0xCD9E8D57u * c[2];
+    const uint32_t n0 = xor3((uint32_t)(p1 >> 32), c[1], k0), n2 = xor3((uint32_t)(p0 >> 32), c[3], k1);
     c[0] = n0;
-    c[1] = lo1;
+    c[1] = (uint32_t)p1;
     c[2] = n2;
-    c[3] = lo0;
+    c[3] = (uint32_t)p0;
     k0 += 0x9E3779B9u;
     k1 += 0xBB67AE85u;
   }
 }
 
-__device__ __forceinline__ float qe_logf(float u)
+// sqrt(-2 ln u), u = ((x >> 8) + 1) / 2^24 in (0, 1].  ln u from u = 2^e m, m in
+// [0.70710677, 1.4142135], as 2 atanh(s), s = (m - 1) / (m + 1).
+__device__ __forceinline__ float qe_radius(uint32_t x)
 {
-  uint32_t i = __float_as_uint(u);
-  int e = (int)((i >> 23) & 0xff) - 127;
-  float m = __uint_as_float((i & 0x007fffffu) | 0x3f800000u);
-  if (m > 1.41421356f) {
-    m = m * 0.5f;
-    e += 1;
-  }
-  float s = (m - 1.0f) / (m + 1.0f);
-  float s2 = s * s;
+  // subtracting the bits of 2^24 0.70710677 leaves e in the exponent field
+  const uint32_t ix = __float_as_uint((float)((x >> 8) + 1u)) - (0x3f3504f4u + (24u << 23));
+  const float e = (float)((int)ix >> 23), m = __uint_as_float((ix & 0x007fffffu) + 0x3f3504f4u);
+  // the quotient rounded to nearest: a reciprocal improved by one Newton step, the
+  // quotient by its exact remainder (Markstein, IBM J. Res. Dev. 34 (1990) 111)
+  const float n = m - 1.0f, d = m + 1.0f;
+  float y = __builtin_amdgcn_rcpf(d);
+  y = fmaf(fmaf(-d, y, 1.0f), y, y);
+  float s = n * y;
+  s = fmaf(fmaf(-d, s, n), y, s);
+  const float s2 = s * s;
   float p = fmaf(s2, 0.11111111f, 0.14285715f);
   p = fmaf(s2, p, 0.2f);
   p = fmaf(s2, p, 0.33333334f);
   p = fmaf(s2, p, 1.0f);
-  float lm = 2.0f * s * p;
-  return fmaf((float)e, 0.69314718f, lm);
+  const float v = -2.0f * fmaf(e, 0.69314718f, 2.0f * s * p);
+  // the square root rounded to nearest: the hardware's, within one unit in the
+  // last place, or its neighbour, by the sign of the exact residuals
+  const float g = __builtin_amdgcn_sqrtf(v);
+  const float lo = __uint_as_float(__float_as_uint(g) - 1u), hi = __uint_as_float(__float_as_uint(g) + 1u);
+  float r = fmaf(-lo, g, v) <= 0.0f ? lo : g;
+  r = fmaf(-hi, g, v) > 0.0f ? hi : r;
+  return r;
 }
 
-__device__ __forceinline__ void qe_sincos2pi(float t, float *s, float *c)
+// sin and cos of 2 pi u, u as above: u = q / 4 + r exactly, |r| <= 1 / 8
+__device__ __forceinline__ void qe_sincos(uint32_t b, float *s, float *c)
 {
-  if (t > 0.5f) t = t - 1.0f;
-  float q = rintf(4.0f * t);
-  float r = fmaf(q, -0.25f, t);
-  float x = r * 6.2831855f;
-  float x2 = x * x;
+  const float k = (float)((b >> 8) + 1u);
+  const float q = rintf(k * 2.3841858e-7f); // k / 2^22
+  const float x = fmaf(q, -4194304.0f, k) * (6.2831855f * 5.9604645e-8f);
+  const float x2 = x * x;
   float sp = fmaf(x2, 2.7557319e-6f, -1.9841270e-4f);
   sp = fmaf(x2, sp, 8.3333333e-3f);
   sp = fmaf(x2, sp, -0.16666667f);
-  float sn = fmaf(x * x2, sp, x);
+  const float sn = fmaf(x * x2, sp, x);
   float cp = fmaf(x2, 2.4801587e-5f, -1.3888889e-3f);
   cp = fmaf(x2, cp, 4.1666667e-2f);
   cp = fmaf(x2, cp, -0.5f);
-  float cs = fmaf(x2, cp, 1.0f);
-  int iq = ((int)q) & 3;
-  float so, co;
-  if (iq == 0) { so = sn; co = cs; }
-  else if (iq == 1) { so = cs; co = -sn; }
-  else if (iq == 2) { so = -sn; co = -cs; }
-  else { so = -cs; co = sn; }
-  *s = so;
-  *c = co;
+  const float cs = fmaf(x2, cp, 1.0f);
+  // quadrant q mod 4: swap on odd, sin negative for 2 and 3, cos for 1 and 2
+  const uint32_t iq = (uint32_t)(int)q;
+  const bool odd = iq & 1u;
+  const uint32_t sb = __float_as_uint(odd ? cs : sn), cb = __float_as_uint(odd ? sn : cs);
+  *s = __uint_as_float(__builtin_amdgcn_bitop3_b32(sb, iq << 30, 0x80000000u, 0x78));        // sb ^ (bit 1 of q)
+  *c = __uint_as_float(__builtin_amdgcn_bitop3_b32(cb, (iq + 1u) << 30, 0x80000000u, 0x78));
 }
-
-__device__ __forceinline__ float u01(uint32_t x) { return ((float)((x >> 8) + 1u)) * 5.9604645e-8f; }
 
 __device__ __forceinline__ void bm_pair(uint32_t a, uint32_t b, double &n0, double &n1)
 {
-  float r = sqrtf(-2.0f * qe_logf(u01(a)));
+  const float r = qe_radius(a);
   float s, c;
-  qe_sincos2pi(u01(b), &s, &c);
+  qe_sincos(b, &s, &c);
   n0 = (double)(r * c);
   n1 = (double)(r * s);
 }
@@ -305,6 +328,44 @@ __device__ __forceinline__ void fx_atomic_add(unsigned long long *plo, unsigned 
   unsigned long long old = atomicAdd(plo, lo);
   unsigned long long carry = (old + lo) < old ? 1ULL : 0ULL;
   atomicAdd(phi, hi + carry);
+}
+
+// The block's dipole sums in LDS: x = A 2^-20 + B 2^-60 + C 2^-100 with A, B, C
+// rounded integers below 2^41 (|x| < 2^20), each added to a 64-bit accumulator of
+// its slice -- the same integer round(x 2^100) as fx_split's, cut differently, so
+// sums are as exact.  A limb is rounded by adding 1.5 2^52, whose bits then hold
+// the integer in their low half; the bits are added as they are and FX_MAGIC times
+// the particle count taken off when the block's sums are folded.  The 128-bit form
+// needed the old value of every addition for the carry, and shifts by the
+// exponent's range with a branch each: 143 instructions a macroparticle and two
+// waits for LDS, now 24 and none.
+#define FX_LIMBS 3
+#define FX_MAGIC_D 6755399441055744.0 // 1.5 2^52
+#define FX_MAGIC 0x4338000000000000ULL
+
+__device__ __forceinline__ void fx_limbs(double x, unsigned long long l[FX_LIMBS])
+{
+  const double u = 1048576.0, w = 1099511627776.0; // 2^20, 2^40
+  const double a = fma(x, u, FX_MAGIC_D);
+  double r = fma(x, u, FX_MAGIC_D - a);
+  const double b = fma(r, w, FX_MAGIC_D);
+  r = fma(r, w, FX_MAGIC_D - b);
+  const double c = fma(r, w, FX_MAGIC_D);
+  l[0] = (unsigned long long)__double_as_longlong(a);
+  l[1] = (unsigned long long)__double_as_longlong(b);
+  l[2] = (unsigned long long)__double_as_longlong(c);
+}
+
+// n particles' accumulated limbs (stride apart) as the 128-bit sum (lo, hi)
+__device__ __forceinline__ void fx_fold(const unsigned long long *l, int stride, unsigned n, unsigned long long &lo,
+                                        unsigned long long &hi)
+{
+  const long long a = (long long)(l[0] - n * FX_MAGIC), b = (long long)(l[stride] - n * FX_MAGIC),
+                  c = (long long)(l[2 * stride] - n * FX_MAGIC);
+  lo = (unsigned long long)c;
+  hi = (unsigned long long)(c >> 63);
+  fx_add(lo, hi, (unsigned long long)b << 40, (unsigned long long)(b >> 24));
+  hi += (unsigned long long)a << 16;
 }
 
 // ------------------------------------------------------------------ k_turn
@@ -346,7 +407,7 @@ __device__ __forceinline__ double wave_sum(double v)
 // parts (fdlibm's pio2_1, pio2_2, pio2_2t; the first two carry 33 bits, so k*part
 // is exact for |k| < 2^20), then Taylor polynomials to degree 17/18 on
 // [-pi/4, pi/4] (truncation < 1e-19), cos with the 1 - z/2 correction.  Larger
-// arguments fall back to the library sincos.
+// arguments (and NaN) are the library's.
 __device__ __noinline__ double2 sincos_lib(double x)
 {
   double2 r;
@@ -360,41 +421,50 @@ __device__ __noinline__ double2 sincos_lib(double x)
 // coefficient into a fresh register before every step (v_mov_b64 + v_fmac_f64,
 // measured in the gfx950 assembly of k_turn); the same IEEE fused multiply-add
 // in one instruction.  Register operands only, no memory access.
-__device__ __forceinline__ double fma3(double a, double b, double c)
+// SC: the addend in scalar registers (one scalar pair per instruction).
+template <bool SC> __device__ __forceinline__ double fma3(double a, double b, double c)
 {
   double r;
-  asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+  if (SC) asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "s"(c));
+  else asm("v_fma_f64 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
 
-__device__ __forceinline__ void sincos_cw(double x, double *s, double *c)
+// How a step whose fast form has a range treats what lies outside it: FAST clears
+// ok and goes on, EXACT has the exact form only, BOTH falls back to it at once.
+enum { FAST = 0, EXACT = 1, BOTH = 2 };
+
+template <int HOW> __device__ __forceinline__ void sincos_cw(double x, double *s, double *c, bool &ok)
 {
-  if (!(fabs(x) < 823549.6)) {
+  const bool in = fabs(x) < 823549.6;
+  if (HOW != FAST && !in) {
     const double2 r = sincos_lib(x);
     *s = r.x;
     *c = r.y;
     return;
   }
+  if (HOW == FAST) ok = ok && in;
   const double k = rint(x * 6.36619772367581382433e-01);
   double r = fma(-k, 1.57079632673412561417e+00, x);
   r = fma(-k, 6.07710050630396597660e-11, r);
   r = fma(-k, 2.02226624879595063154e-21, r);
   const double z = r * r;
-  double ps = fma3(z, 2.8114572543455206e-15, -7.647163731819816e-13);
-  ps = fma3(z, ps, 1.6059043836821613e-10);
-  ps = fma3(z, ps, -2.505210838544172e-08);
-  ps = fma3(z, ps, 2.7557319223985893e-06);
-  ps = fma3(z, ps, -0.0001984126984126984);
-  ps = fma3(z, ps, 0.008333333333333333);
-  ps = fma3(z, ps, -0.16666666666666666);
+  constexpr bool SC = HOW == FAST;
+  double ps = fma3<SC>(z, 2.8114572543455206e-15, -7.647163731819816e-13);
+  ps = fma3<SC>(z, ps, 1.6059043836821613e-10);
+  ps = fma3<SC>(z, ps, -2.505210838544172e-08);
+  ps = fma3<SC>(z, ps, 2.7557319223985893e-06);
+  ps = fma3<SC>(z, ps, -0.0001984126984126984);
+  ps = fma3<SC>(z, ps, 0.008333333333333333);
+  ps = fma3<SC>(z, ps, -0.16666666666666666);
   const double sn = fma(r * z, ps, r);
-  double pc = fma3(z, -1.5619206968586225e-16, 4.779477332387385e-14);
-  pc = fma3(z, pc, -1.1470745597729725e-11);
-  pc = fma3(z, pc, 2.08767569878681e-09);
-  pc = fma3(z, pc, -2.755731922398589e-07);
-  pc = fma3(z, pc, 2.48015873015873e-05);
-  pc = fma3(z, pc, -0.001388888888888889);
-  pc = fma3(z, pc, 0.041666666666666664);
+  double pc = fma3<SC>(z, -1.5619206968586225e-16, 4.779477332387385e-14);
+  pc = fma3<SC>(z, pc, -1.1470745597729725e-11);
+  pc = fma3<SC>(z, pc, 2.08767569878681e-09);
+  pc = fma3<SC>(z, pc, -2.755731922398589e-07);
+  pc = fma3<SC>(z, pc, 2.48015873015873e-05);
+  pc = fma3<SC>(z, pc, -0.001388888888888889);
+  pc = fma3<SC>(z, pc, 0.041666666666666664);
   const double hz = 0.5 * z;
   const double w = 1.0 - hz;
   const double cs = w + (((1.0 - w) - hz) + (z * z) * pc);
@@ -406,28 +476,29 @@ __device__ __forceinline__ void sincos_cw(double x, double *s, double *c)
   *c = ((q + 1) & 2) ? -bq : bq;
 }
 
-__device__ __forceinline__ double sin_cw(double x)
+template <int HOW> __device__ __forceinline__ double sin_cw(double x, bool &ok)
 {
   double s, c;
-  sincos_cw(x, &s, &c);
+  sincos_cw<HOW>(x, &s, &c, ok);
   return s;
 }
 
-// Slice index with reciprocal multiplies, falling back to the exact reference
-// expression (two correctly rounded divides) whenever the truncation could
-// depend on the last bits: the approximate value is within 1e-12 of the exact
-// one for |v| < 1e6.
+// Slice index with reciprocal multiplies; where the truncation could depend on
+// the last bits (the approximate value is within 1e-12 of the exact one for
+// |v| < 1e6) the exact reference expression (two correctly rounded divides) takes
+// over.
 struct BinK {
   double sgm, inv_sgm, Nsigma, dT, inv_dT;
 };
-__device__ __forceinline__ int bin_fast(double tau, const BinK &k)
+template <int HOW> __device__ __forceinline__ int bin_fast(double tau, const BinK &k, bool &ok)
 {
+  if (HOW == EXACT) return bin_of(tau, k.sgm, k.Nsigma, k.dT);
   const double vf = fma(fma(-tau, k.inv_sgm, k.Nsigma), k.inv_dT, 1.0);
-  if (fabs(vf) < 1.0e6) {
-    const double lo = trunc(vf - 1.0e-9), hi = trunc(vf + 1.0e-9);
-    if (lo == hi) return (int)lo;
-  }
-  return bin_of(tau, k.sgm, k.Nsigma, k.dT);
+  const double lo = trunc(vf - 1.0e-9), hi = trunc(vf + 1.0e-9);
+  const bool in = fabs(vf) < 1.0e6 && lo == hi;
+  if (HOW == FAST) ok = ok && in;
+  else if (!in) return bin_of(tau, k.sgm, k.Nsigma, k.dT);
+  return (int)lo;
 }
 
 // Block index -> work item, so that consecutive work items (the chunks of one
@@ -524,6 +595,120 @@ __device__ __forceinline__ double lr_wake_at(const DevParams &P, const LRDev &R,
   return w + I * R.self[((size_t)pl * R.Gtot + b) * Nc + i];
 }
 
+// What one macroparticle's turn needs beside its ring's constants.
+struct MapArgs {
+  BinK bk;
+  const double *kL, *kV, *kH; // LDS kick tables
+  double eps_const, phai0, rwx, rwz;
+  int flags, Nc, kb;
+  bool rw_h, rw_v, qe, do_hist;
+  long long rev;
+};
+
+// One macroparticle's turn: q = (tau, delta, x, x', z, z') in place, sl its slice
+// for the next turn's histogram (Nc below, Nc + 1 above the range).  ok is cleared
+// where a fast form does not cover the particle.
+template <int HOW, bool MAP, bool QE, bool GEN>
+__device__ __forceinline__ void turn_particle(const DevParams &P, const MapArgs &A, unsigned j, double q[6], int &sl,
+                                              bool &ok)
+{
+  double tau = q[0], del = q[1], x = q[2], xp = q[3], z = q[4], zp = q[5];
+  const int Nc = A.Nc, fl = A.flags;
+  if (A.rw_h) xp += A.rwx;
+  if (A.rw_v) zp += A.rwz;
+  if (MAP) {
+    if (fl & TF_SF) {
+      int bn = bin_fast<HOW>(tau, A.bk, ok);
+      bn = bn < 0 ? 0 : (bn >= Nc ? Nc - 1 : bn);
+      if (fl & TF_KICK_L) del += A.kL[bn];
+      if (fl & TF_KICK_V) zp += A.kV[bn];
+      if (fl & TF_KICK_H) xp += A.kH[bn];
+    }
+    // ---- one-turn map, src/transform_weak.c:21-192 (operation order kept)
+    const double tau0 = tau, del0 = del, x0 = x, xp0 = xp, z0 = z, zp0 = zp;
+    double g;
+    if (!GEN) {
+      g = A.eps_const * sin_cw<HOW>(P.wrf * tau0 + A.phai0, ok);
+    } else if (!(fl & TF_IDEAL)) {
+      g = A.eps_const * sin_cw<HOW>(P.wrf * tau0 + A.phai0, ok);
+      for (int a = 0; a < P.n_ahc; a++)
+        g += P.ahc_amp[a] * sin_cw<HOW>(P.ahc_wn[a] * tau0 + P.ahc_phi[a] + P.ahc_nHC[a] * A.kb * 2 * M_PI, ok);
+    } else {
+      g = A.eps_const *
+          (sin_cw<HOW>(P.wrf * tau0 + A.phai0, ok) + P.HC_k * sin_cw<HOW>(P.m_wrf * tau0 + P.m_phi, ok));
+    }
+    del = del0 + g - P.Urad;
+    double nq[5] = {0, 0, 0, 0, 0}, rff = 0.0;
+    const bool qe = QE && A.qe;
+    if (qe) {
+      qe_normals(P.seed, (uint32_t)A.kb, (unsigned long long)A.rev, j, nq);
+      del = del * P.damp + P.excite * nq[0];
+      rff = (1.0 + del0) / (1.0 + del0 + g);
+    }
+    tau = tau0 - del * P.T0 * P.ac;
+    if (fl & TF_TRACK_V) {
+      double dQ = 0.0;
+      if (GEN && (fl & TF_AMP)) {
+        double EV = P.gV * z0 * z0 + 2 * P.aV * z0 * zp0 + P.bV * zp0 * zp0;
+        double EH = P.gV * x0 * x0 + 2 * P.aV * x0 * xp0 + P.bV * xp0 * xp0;
+        dQ = P.CVH * EH + P.CVV * EV;
+      }
+      double sn, cs;
+      sincos_cw<HOW>(P.PsiV0 * (1.0 + P.Gziz * del0 + dQ), &sn, &cs, ok);
+      double a11 = cs + P.aV * sn, a12 = P.bV * sn, a21 = -P.gV * sn, a22 = cs - P.aV * sn;
+      z = a11 * z0 + a12 * zp0;
+      zp = a21 * z0 + a22 * zp0;
+      if (qe) {
+        z = z + P.qVp * nq[1];
+        zp = rff * zp + P.qVs * nq[2];
+      }
+    }
+    if (fl & TF_TRACK_H) {
+      double dQ = 0.0;
+      if (GEN && (fl & TF_AMP)) {
+        double EV = P.gV * z0 * z0 + 2 * P.aV * z0 * zp0 + P.bV * zp0 * zp0;
+        double EH = P.gV * x0 * x0 + 2 * P.aV * x0 * xp0 + P.bV * xp0 * xp0;
+        dQ = P.CHH * EH + P.CHV * EV;
+      }
+      double sn, cs;
+      sincos_cw<HOW>(P.PsiH0 * (1.0 + P.Gzix * del0 + dQ), &sn, &cs, ok);
+      double a11 = cs + P.aH * sn;
+      double a12 = P.bH * sn;
+      double a13 = (1.0 - a11) * P.dispH - a12 * P.disppH;
+      double a21 = -P.gH * sn;
+      double a22 = cs - P.aH * sn;
+      double a23 = -a21 * P.dispH + (1.0 - a22) * P.disppH;
+      x = a11 * x0 + a12 * xp0 + a13 * del;
+      xp = a21 * x0 + a22 * xp0 + a23 * del;
+      if (qe) {
+        x = x + P.qHp * nq[3];
+        xp = rff * xp + P.qHs * nq[4];
+      }
+    }
+  }
+  q[0] = tau;
+  q[1] = del;
+  q[2] = x;
+  q[3] = xp;
+  q[4] = z;
+  q[5] = zp;
+  sl = 0;
+  if (A.do_hist) {
+    const int bn = bin_fast<HOW>(tau, A.bk, ok);
+    sl = bn < 0 ? Nc : (bn < Nc ? bn : Nc + 1);
+  }
+}
+
+// The exact forms, out of line (see k_turn's loops); the slice in the return value.
+template <bool MAP, bool QE, bool GEN>
+__device__ __noinline__ int turn_particle_exact(const DevParams *P, const MapArgs *A, unsigned j, double *q)
+{
+  int sl;
+  bool ok = true;
+  turn_particle<EXACT, MAP, QE, GEN>(*P, *A, j, q, sl, ok);
+  return sl;
+}
+
 template <int MODE, bool QE, bool DIP, bool GEN, bool MON>
 __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams *__restrict__ Pr, Coords C,
                                                                 const long long *wg_first, const long long *wg_end,
@@ -548,15 +733,15 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
   const DevParams &P = Pr[ring];
   const TurnState *ts = tsr + ring;
   const int Nc = P.Nc;
-  // LDS: sx lo/hi [2Nc], sz lo/hi [2Nc], trash sums [8], kick tables [3Nc], counts [Nc] + trash [2]
+  // LDS: dipole limbs sx, sz [3][Nc + 2] (the last two: below and above the range),
+  // kick tables [3Nc], counts [Nc + 2]
+  const int Nt = Nc + 2;
   unsigned long long *lsx = smem;
-  unsigned long long *lsz = lsx + 2 * Nc;
-  unsigned long long *ltr = lsz + 2 * Nc;
-  double *kL = (double *)(ltr + 8);
+  unsigned long long *lsz = lsx + (DIP ? FX_LIMBS * Nt : 0);
+  double *kL = (double *)(lsz + (DIP ? FX_LIMBS * Nt : 0));
   double *kV = kL + Nc;
   double *kH = kV + Nc;
   unsigned int *lcnt = (unsigned int *)(kH + Nc);
-  unsigned int *ltc = lcnt + Nc;
   __shared__ double red[WG / 64][NMOM];
   __shared__ int lbad;
 
@@ -569,12 +754,9 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
   const double Ikb = lr ? Ibunch[P.bucket_off + kb] : 0.0;
 
   if (DIP)
-    for (int i = tid; i < 2 * Nc; i += WG) {
-      lsx[i] = 0;
-      lsz[i] = 0;
-    }
+    for (int i = tid; i < 2 * FX_LIMBS * Nt; i += WG) lsx[i] = 0;
+  for (int i = tid; i < Nt; i += WG) lcnt[i] = 0;
   for (int i = tid; i < Nc; i += WG) {
-    lcnt[i] = 0;
     if (MODE == MODE_TURN || MODE == MODE_TUNE) {
       double l = P.kickL ? sfL[(size_t)b * Nc + i] : 0.0, v = P.kickV ? sfV[(size_t)b * Nc + i] : 0.0,
              h = P.kickH ? sfH[(size_t)b * Nc + i] : 0.0;
@@ -588,8 +770,6 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
       if (P.kickH) kH[i] = h;
     }
   }
-  if (tid < 8) ltr[tid] = 0;
-  if (tid < 2) ltc[tid] = 0;
   if (tid == 0) lbad = 0;
   __syncthreads();
 
@@ -618,140 +798,113 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
   const unsigned cnt = (unsigned)(j1 - j0), o0 = (unsigned)(j0 & (TILE - 1));
   const unsigned jloc0 = (unsigned)(j0 - bunch_first[b]);
 
-  for (unsigned ii = tid; ii < cnt; ii += WG) {
-    // offset of the slot in the tiles from the chunk's first (chunks longer
-    // than a tile cross into the next ones)
-    const unsigned u = o0 + ii, i = ((u >> TILE_SHIFT) * 6u << TILE_SHIFT) + (u & (TILE - 1));
-    // coordinates stream through once per turn: nontemporal loads and stores
-    double tau = LDC(pt + i), del = LDC(pd + i), x = LDC(px + i), xp = LDC(pxp + i), z = LDC(pz + i),
-           zp = LDC(pzp + i);
-    const double in[6] = {tau, del, x, xp, z, zp}; // kept only by the timing pass
-    if (rw_h) xp += rwx;
-    if (rw_v) zp += rwz;
-    if (MODE == MODE_TURN || MODE == MODE_TUNE) {
-      if (P.sf_active) {
-        int bn = bin_fast(tau, bk);
-        bn = bn < 0 ? 0 : (bn >= Nc ? Nc - 1 : bn);
-        if (P.kickL) del += kL[bn];
-        if (P.kickV) zp += kV[bn];
-        if (P.kickH) xp += kH[bn];
-      }
-      // ---- one-turn map, src/transform_weak.c:21-192 (operation order kept)
-      const double tau0 = tau, del0 = del, x0 = x, xp0 = xp, z0 = z, zp0 = zp;
-      double g;
-      if (!GEN) {
-        g = eps_const * sin_cw(P.wrf * tau0 + phai0);
-      } else if (!P.ideal_hc) {
-        g = eps_const * sin_cw(P.wrf * tau0 + phai0);
-        for (int a = 0; a < P.n_ahc; a++)
-          g += P.ahc_amp[a] * sin_cw(P.ahc_wn[a] * tau0 + P.ahc_phi[a] + P.ahc_nHC[a] * kb * 2 * M_PI);
-      } else {
-        g = eps_const * (sin_cw(P.wrf * tau0 + phai0) + P.HC_k * sin_cw(P.m_wrf * tau0 + P.m_phi));
-      }
-      del = del0 + g - P.Urad;
-      double nq[5] = {0, 0, 0, 0, 0}, rff = 0.0;
-      if (qe) {
-        qe_normals(P.seed, (uint32_t)kb, (unsigned long long)rev, jloc0 + ii, nq);
-        del = del * P.damp + P.excite * nq[0];
-        rff = (1.0 + del0) / (1.0 + del0 + g);
-      }
-      tau = tau0 - del * P.T0 * P.ac;
-      if (P.track_v) {
-        double dQ = 0.0;
-        if (GEN && P.amp_dq) {
-          double EV = P.gV * z0 * z0 + 2 * P.aV * z0 * zp0 + P.bV * zp0 * zp0;
-          double EH = P.gV * x0 * x0 + 2 * P.aV * x0 * xp0 + P.bV * xp0 * xp0;
-          dQ = P.CVH * EH + P.CVV * EV;
-        }
-        double sn, cs;
-        sincos_cw(P.PsiV0 * (1.0 + P.Gziz * del0 + dQ), &sn, &cs);
-        double a11 = cs + P.aV * sn, a12 = P.bV * sn, a21 = -P.gV * sn, a22 = cs - P.aV * sn;
-        z = a11 * z0 + a12 * zp0;
-        zp = a21 * z0 + a22 * zp0;
-        if (qe) {
-          z = z + P.qVp * nq[1];
-          zp = rff * zp + P.qVs * nq[2];
-        }
-      }
-      if (P.track_h) {
-        double dQ = 0.0;
-        if (GEN && P.amp_dq) {
-          double EV = P.gV * z0 * z0 + 2 * P.aV * z0 * zp0 + P.bV * zp0 * zp0;
-          double EH = P.gV * x0 * x0 + 2 * P.aV * x0 * xp0 + P.bV * xp0 * xp0;
-          dQ = P.CHH * EH + P.CHV * EV;
-        }
-        double sn, cs;
-        sincos_cw(P.PsiH0 * (1.0 + P.Gzix * del0 + dQ), &sn, &cs);
-        double a11 = cs + P.aH * sn;
-        double a12 = P.bH * sn;
-        double a13 = (1.0 - a11) * P.dispH - a12 * P.disppH;
-        double a21 = -P.gH * sn;
-        double a22 = cs - P.aH * sn;
-        double a23 = -a21 * P.dispH + (1.0 - a22) * P.disppH;
-        x = a11 * x0 + a12 * xp0 + a13 * del;
-        xp = a21 * x0 + a22 * xp0 + a23 * del;
-        if (qe) {
-          x = x + P.qHp * nq[3];
-          xp = rff * xp + P.qHs * nq[4];
-        }
-      }
-    }
-    if (MODE == MODE_TUNE) {
-      // a value the compiler cannot prove equal to the loaded one, so the
-      // stores (and their traffic) stay; the bits written are the bits read
-      const unsigned long long zb = P.zero_bits;
-      STC(__longlong_as_double(__double_as_longlong(in[0]) ^ zb), pt + i);
-      STC(__longlong_as_double(__double_as_longlong(in[1]) ^ zb), pd + i);
-      STC(__longlong_as_double(__double_as_longlong(in[2]) ^ zb), px + i);
-      STC(__longlong_as_double(__double_as_longlong(in[3]) ^ zb), pxp + i);
-      STC(__longlong_as_double(__double_as_longlong(in[4]) ^ zb), pz + i);
-      STC(__longlong_as_double(__double_as_longlong(in[5]) ^ zb), pzp + i);
-    } else if (MODE != MODE_STATS) {
-      STC(tau, pt + i);
-      STC(del, pd + i);
-      STC(x, px + i);
-      STC(xp, pxp + i);
-      STC(z, pz + i);
-      STC(zp, pzp + i);
+  constexpr bool MAP = MODE == MODE_TURN || MODE == MODE_TUNE;
+  constexpr int HOW = MAP && (QE || GEN || DIP) ? FAST : BOTH;
+  __shared__ MapArgs margs; // for the calls of the exact forms
+  const MapArgs A = {bk, kL, kV, kH, eps_const, phai0, rwx, rwz, P.flags, Nc, kb, rw_h, rw_v, qe, do_hist, rev};
+  if (HOW == FAST) {
+    if (tid == 0) margs = A;
+    __syncthreads();
+  }
+  // offset of item ii's slot in the tiles from the chunk's first (chunks longer
+  // than a tile cross into the next ones)
+  const auto slot_of = [&](unsigned ii) {
+    const unsigned u = o0 + ii;
+    return ((u >> TILE_SHIFT) * 6u << TILE_SHIFT) + (u & (TILE - 1));
+  };
+  // coordinates stream through once per turn: nontemporal loads and stores
+  const auto load = [&](unsigned i, double q[6]) {
+    q[0] = LDC(pt + i);
+    q[1] = LDC(pd + i);
+    q[2] = LDC(px + i);
+    q[3] = LDC(pxp + i);
+    q[4] = LDC(pz + i);
+    q[5] = LDC(pzp + i);
+  };
+  // a done macroparticle's stores (in: the loaded coordinates), moments and
+  // histogram entry
+  const auto commit = [&](unsigned i, const double q[6], const double in[6], int sl) {
+    if (MODE != MODE_STATS) {
+      // the timing pass writes a value the compiler cannot prove equal to the
+      // loaded one, so the stores (and their traffic) stay; the bits written are
+      // the bits read
+      const auto out = [&](int c) {
+        return MODE == MODE_TUNE
+                   ? __longlong_as_double(__double_as_longlong(in[c]) ^ (long long)P.zero_bits)
+                   : q[c];
+      };
+      STC(out(0), pt + i);
+      STC(out(1), pd + i);
+      STC(out(2), px + i);
+      STC(out(3), pxp + i);
+      STC(out(4), pz + i);
+      STC(out(5), pzp + i);
     }
     // ---- moments about the per-bunch shift (reassociated: no bitwise target)
-    const double v[6] = {tau, del, x, xp, z, zp};
 #pragma unroll
     for (int c = 0; c < 6; c++) {
-      const double d = v[c] - sh[c];
+      const double d = q[c] - sh[c];
       s1[c] += d;
       s2[c] = fma(d, d, s2[c]);
     }
     if (MON) {
-      am[0] += P.gamma1[0] * (tau * tau) + 2.0 * P.alpha1[0] * tau * del + P.beta1[0] * (del * del);
-      am[1] += P.gamma1[1] * (x * x) + 2.0 * P.alpha1[1] * x * xp + P.beta1[1] * (xp * xp);
-      am[2] += P.gamma1[2] * (z * z) + 2.0 * P.alpha1[2] * z * zp + P.beta1[2] * (zp * zp);
+#pragma unroll
+      for (int c = 0; c < 3; c++) {
+        const double u = q[2 * c], w = q[2 * c + 1];
+        am[c] += P.gamma1[c] * (u * u) + 2.0 * P.alpha1[c] * u * w + P.beta1[c] * (w * w);
+      }
     }
     // ---- next turn's slice histogram
     if (do_hist) {
-      const int bn = bin_fast(tau, bk);
-      const bool inr = bn >= 0 && bn < Nc;
-      if (inr) atomicAdd(&lcnt[bn], 1u);
-      else atomicAdd(&ltc[bn < 0 ? 0 : 1], 1u);
+      atomicAdd(&lcnt[sl], 1u);
       if (DIP) {
-        unsigned long long xl, xh, zl, zh;
-        if (!(fabs(x) < P.fx_lim) || !(fabs(z) < P.fx_lim)) {
-          lbad = 1;
-          xl = xh = zl = zh = 0;
-        } else {
-          fx_split(x, xl, xh);
-          fx_split(z, zl, zh);
-        }
-        if (inr) {
-          fx_atomic_add(&lsx[2 * bn], &lsx[2 * bn + 1], xl, xh);
-          fx_atomic_add(&lsz[2 * bn], &lsz[2 * bn + 1], zl, zh);
-        } else {
-          const int t = bn < 0 ? 0 : 1;
-          fx_atomic_add(&ltr[4 * t], &ltr[4 * t + 1], xl, xh);
-          fx_atomic_add(&ltr[4 * t + 2], &ltr[4 * t + 3], zl, zh);
+        const bool fit = fabs(q[2]) < P.fx_lim && fabs(q[4]) < P.fx_lim;
+        if (!fit) lbad = 1;
+        unsigned long long lx[FX_LIMBS], lz[FX_LIMBS];
+        fx_limbs(fit ? q[2] : 0.0, lx);
+        fx_limbs(fit ? q[4] : 0.0, lz);
+#pragma unroll
+        for (int k = 0; k < FX_LIMBS; k++) {
+          atomicAdd(&lsx[k * Nt + sl], lx[k]);
+          atomicAdd(&lsz[k * Nt + sl], lz[k]);
         }
       }
     }
+  };
+  // The variants that do more than stream (excitation, dipole histograms, harmonic
+  // cavity or detuning) are VALU-bound at 4 waves per SIMD and 128 registers.  They
+  // take the fast forms first, in a loop without calls: with the fallbacks inside
+  // it every value that outlives a call sat in a preserved register or on the stack
+  // and the constants were fetched again after each.  The few macroparticles that
+  // leave a fast form's range (about one in 1e8, at a slice's edge; lost ones every
+  // turn) are noted, untouched, and done with the exact forms after it.  416 x
+  // 50,021 macroparticles with excitation and dipoles: 551 -> 455 us at best, 601
+  // -> 512 a turn in a long run; 104 x 20,000 with excitation and harmonic cavity
+  // 67 -> 60.  (Two macroparticles at a time at 2 or 3 waves per SIMD: 10 % slower.)
+  // The plain variant streams at the memory's rate, and the second loop's code
+  // cost it 2-3 %, so it keeps its fallbacks in place.
+  unsigned long long redo = 0, bit = 1;
+  for (unsigned ii = tid; ii < cnt; ii += WG, bit <<= 1) {
+    const unsigned i = slot_of(ii);
+    double in[6], q[6];
+    load(i, in);
+#pragma unroll
+    for (int c = 0; c < 6; c++) q[c] = in[c];
+    int sl;
+    bool ok = true;
+    turn_particle<HOW, MAP, QE, GEN>(P, A, jloc0 + ii, q, sl, ok);
+    if (HOW != FAST || ok) commit(i, q, in, sl);
+    else redo |= bit;
+  }
+  while (HOW == FAST && redo) {
+    const unsigned ii = tid + (__ffsll((long long)redo) - 1) * WG, i = slot_of(ii);
+    double in[6], q[6];
+    load(i, in);
+#pragma unroll
+    for (int c = 0; c < 6; c++) q[c] = in[c];
+    const int sl = turn_particle_exact<MAP, QE, GEN>(&P, &margs, jloc0 + ii, q);
+    commit(i, q, in, sl);
+    redo &= redo - 1;
   }
 
   // ---- block reduction of the moment sums in a fixed order
@@ -780,22 +933,17 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
   }
   // ---- flush the block histogram with exact integer atomics
   if (do_hist) {
-    for (int i = tid; i < Nc; i += WG) {
+    for (int i = tid; i < Nt; i += WG) {
       const unsigned int n = lcnt[i];
       if (n == 0) continue;
-      const size_t gi = (size_t)b * Nc + i;
-      atomicAdd(&H.cnt[gi], n);
+      const size_t gi = i < Nc ? (size_t)b * Nc + i : 2 * (size_t)b + i - Nc;
+      atomicAdd(i < Nc ? &H.cnt[gi] : &H.tcnt[gi], n);
       if (DIP) {
-        fx_atomic_add(&H.sx[2 * gi], &H.sx[2 * gi + 1], lsx[2 * i], lsx[2 * i + 1]);
-        fx_atomic_add(&H.sz[2 * gi], &H.sz[2 * gi + 1], lsz[2 * i], lsz[2 * i + 1]);
-      }
-    }
-    if (tid < 2 && ltc[tid] > 0) {
-      const int t = tid;
-      atomicAdd(&H.tcnt[2 * b + t], ltc[t]);
-      if (DIP) {
-        fx_atomic_add(&H.tsx[4 * b + 2 * t], &H.tsx[4 * b + 2 * t + 1], ltr[4 * t], ltr[4 * t + 1]);
-        fx_atomic_add(&H.tsz[4 * b + 2 * t], &H.tsz[4 * b + 2 * t + 1], ltr[4 * t + 2], ltr[4 * t + 3]);
+        unsigned long long lo, hi, *gx = (i < Nc ? H.sx : H.tsx) + 2 * gi, *gz = (i < Nc ? H.sz : H.tsz) + 2 * gi;
+        fx_fold(lsx + i, Nt, n, lo, hi);
+        fx_atomic_add(gx, gx + 1, lo, hi);
+        fx_fold(lsz + i, Nt, n, lo, hi);
+        fx_atomic_add(gz, gz + 1, lo, hi);
       }
     }
     if (DIP && tid == 0 && lbad) H.bad[b] = 1;
@@ -1772,7 +1920,7 @@ struct mbt_ring {
   int nres;
   double *fb_hist;
   long long rw_total, st_total, fbh_total;
-  size_t lds_turn, lds_red;
+  size_t lds_turn[2], lds_red; // lds_turn: without, with dipole histograms
   int lr_lds; // k_reduce keeps the LR resonators' own wakes in LDS
   long long rev_host;
   double *pot_host;    // pinned staging of mbt_ring_potentials: 7 Nc doubles, then a TurnState
@@ -1796,9 +1944,10 @@ static int no_pending(const mbt_ring *r)
   return MBT_OK;
 }
 
-static size_t turn_lds(int Nc)
+// LDS of k_turn without / with dipole histograms, in bytes
+static size_t turn_lds(int Nc, int dip)
 {
-  return (size_t)(4 * Nc + 8) * 8 + (size_t)3 * Nc * 8 + (size_t)(Nc + 2) * 4 + 16;
+  return (size_t)(dip ? 2 * FX_LIMBS * (Nc + 2) : 0) * 8 + (size_t)3 * Nc * 8 + (size_t)(Nc + 2) * 4 + 16;
 }
 
 static void fill_params(const mbt_config *c, const int planes[3], DevParams &P)
@@ -1882,6 +2031,9 @@ static void fill_params(const mbt_config *c, const int planes[3], DevParams &P)
   P.convL = planes[0] > 0;
   P.kickV = planes[2] > 0;
   P.kickH = planes[1] > 0;
+  P.flags = (P.sf_active ? TF_SF : 0) | (P.kickL ? TF_KICK_L : 0) | (P.kickV ? TF_KICK_V : 0) |
+            (P.kickH ? TF_KICK_H : 0) | (P.track_v ? TF_TRACK_V : 0) | (P.track_h ? TF_TRACK_H : 0) |
+            (P.ideal_hc ? TF_IDEAL : 0) | (P.amp_dq ? TF_AMP : 0);
   P.fb_len = c->has_rf_feedback ? abs(c->rffb_len_average) : 1;
   P.fb_switch_off = c->has_rf_feedback && c->rffb_len_average < 0;
   P.vrf_design = c->rffb_vrf_design;
@@ -2735,10 +2887,10 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
   Ro.rfbuf = r->rfbuf;
   Ro.R = R;
   r->use_graphs = !(flags & MBT_RING_NO_GRAPHS);
-  r->lds_turn = turn_lds(Nc);
+  for (int d = 0; d < 2; d++) r->lds_turn[d] = turn_lds(Nc, d);
   r->lr_lds = nres > 0 && (size_t)9 * NcA * 8 + 64 <= 64 * 1024;
   r->lds_red = (size_t)(r->lr_lds ? 9 : 6) * NcA * 8 + 64;
-  if (r->lds_turn > 64 * 1024 || r->lds_red > 64 * 1024) {
+  if (Nc > NCELL_MAX) {
     mbt_set_error("Ncell %d too large for the LDS histogram", Nc);
     mbt_ring_destroy(r);
     return MBT_EINVAL;
@@ -2943,7 +3095,7 @@ static int launch_turn_pass(mbt_ring *r, int mode)
   }
   // the turn pass also carries the resistive-wall tiles of earlier turns' rows
   RwOld ro = {};
-  size_t lds = r->lds_turn;
+  size_t lds = r->lds_turn[mode != MODE_TURN || r->any_dip]; // the statistics passes make dipole sums
   if (mode == MODE_TURN && r->rw_split) {
     ro = {r->rw_tiles, r->rw_ntile, (r->rw_ntile + 7) / 8 * 8, r->rwhist, r->rsqrt_tt, r->Ibunch, r->nfFill,
           r->rw_part, r->G};
@@ -3466,7 +3618,7 @@ extern "C" int mbt_ring_autotune(mbt_ring *r, int *best_items, double *ms)
       float t = 0.0f;
       for (int rep = 0; rep <= AUTOTUNE_REPS; rep++) {
         if (rep == 1) CK(hipEventRecord(e0, r->stream));
-        hipLaunchKernelGGL(k, dim3(r->nwg), dim3(WG), r->lds_turn, r->stream, r->P, r->C, r->wg_first, r->wg_end,
+        hipLaunchKernelGGL(k, dim3(r->nwg), dim3(WG), r->lds_turn[r->any_dip], r->stream, r->P, r->C, r->wg_first, r->wg_end,
                            r->wg_bunch, r->bunch_ring, r->bucket, r->bunch_first, r->shift, r->sfL, r->sfV, r->sfH,
                            r->LR, r->Ibunch, r->pending, r->partial, r->Hs, r->ts, RwOld{});
         CK(hipGetLastError());
