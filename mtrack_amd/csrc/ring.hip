@@ -41,6 +41,7 @@
 #include <string.h>
 #include <math.h>
 #include "mbt_host.h"
+#include "wave_dev.h"
 
 #pragma clang fp contract(off)
 
@@ -168,14 +169,26 @@ enum {
 };
 
 struct TurnState {
-  long long rev;
-  int m;
+  long long rev; // turns done; a launch of turn `turn` of a block works on turn rev + turn
   int has_fb;
   double phai0, Vrf0;
   double phai0_prev, Vrf0_prev; // before this turn's RF-feedback solve
   double Iring, scan_val;
   long long fb_count;
 };
+
+// a mod d for a >= 0 (turn counters fit 32 bits in any run of a lifetime; a 64-bit
+// remainder is some hundred instructions)
+__device__ __forceinline__ unsigned umod(long long a, unsigned d)
+{
+  return (unsigned long long)a >> 32 ? (unsigned)((unsigned long long)a % d) : (unsigned)a % d;
+}
+
+// The resistive wall's trigger counts turns since the last scan step.
+__device__ __forceinline__ int rw_trigger(long long rev, long long NrevScan)
+{
+  return (NrevScan >> 32 ? rev % NrevScan : (long long)umod(rev, (unsigned)NrevScan)) < 50 ? 1 : 0;
+}
 
 struct LRConst {
   int ring, plane, l, fb;
@@ -532,13 +545,13 @@ struct RwOld {
 // rounding apart, and a multiply instead of a division keeps these blocks short
 // beside the map's); one plane per sweep keeps the register count low.
 __device__ void rw_old_tile(const DevParams *__restrict__ Pr, const RwOld &RO, int t, const int *bucket,
-                            const TurnState *__restrict__ tsr, double *sm)
+                            const TurnState *__restrict__ tsr, int turn, double *sm)
 {
   const int4 T = RO.tiles[t];
   const DevParams &P = Pr[T.x];
   const int tid = threadIdx.x;
   const int h = P.h, n = (P.Nmlt + 2) * h, M = (P.Nmlt + 1) * h;
-  const long long rev = tsr[T.x].rev;
+  const long long rev = tsr[T.x].rev + turn;
   const int m0 = 1 + T.w * RW_TILE_TAPS;
   const int m1 = min(m0 + RW_TILE_TAPS - 1, M);
   const int kb_lo = bucket[T.y], kb_hi = bucket[T.y + T.z - 1];
@@ -718,13 +731,13 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
                                                                 const double *sfV, const double *sfH,
                                                                 LRDev LR, const double *Ibunch,
                                                                 const double *pending, double *partial, HistPtr H,
-                                                                const TurnState *__restrict__ tsr, RwOld RO)
+                                                                const TurnState *__restrict__ tsr, int turn, RwOld RO)
 {
   extern __shared__ unsigned long long smem[];
   if (MODE == MODE_TURN && (int)blockIdx.x < RO.nlead) {
     // leading blocks: the resistive-wall taps of earlier turns' rows, dispatched
     // first so that they finish early in the pass
-    if ((int)blockIdx.x < RO.ntile) rw_old_tile(Pr, RO, blockIdx.x, bucket, tsr, (double *)smem);
+    if ((int)blockIdx.x < RO.ntile) rw_old_tile(Pr, RO, blockIdx.x, bucket, tsr, turn, (double *)smem);
     return;
   }
   const int wg = xcd_remap(blockIdx.x - RO.nlead, gridDim.x - RO.nlead);
@@ -748,7 +761,7 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
   const int kb = bucket[b];
   const long long j0 = wg_first[wg], j1 = wg_end[wg];
   const int tid = threadIdx.x;
-  const long long rev = ts->rev;
+  const long long rev = ts->rev + turn;
   const bool do_hist = Nc > 0 && MODE != MODE_FINAL;
   const bool lr = P.lrp[3] > P.lrp[0];
   const double Ikb = lr ? Ibunch[P.bucket_off + kb] : 0.0;
@@ -907,22 +920,19 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
     redo &= redo - 1;
   }
 
-  // ---- block reduction of the moment sums in a fixed order
-  double vals[NMOM];
-#pragma unroll
-  for (int c = 0; c < 6; c++) {
-    vals[c] = s1[c];
-    vals[6 + c] = s2[c];
-  }
-  vals[12] = am[0];
-  vals[13] = am[1];
-  vals[14] = am[2];
+  // ---- block reduction of the moment sums in a fixed order: eight sums per wave
+  // at a time (20 lane exchanges for all; one by one through LDS permutes they took
+  // 144, 3.4 us at the end of every work-group)
   const int lane = tid & 63, wv = tid >> 6;
-#pragma unroll
-  for (int c = 0; c < NMOM; c++) {
-    if (!MON && c >= 12) continue;
-    double sum = wave_sum(vals[c]);
-    if (lane == 0) red[wv][c] = sum;
+  {
+    const double v0[8] = {s1[0], s1[1], s1[2], s1[3], s1[4], s1[5], s2[0], s2[1]};
+    const double v1[8] = {s2[2], s2[3], s2[4], s2[5], am[0], am[1], am[2], 0.0};
+    const double t0 = wsum64x8(v0), t1 = wsum64x8(v1);
+    const int k = lane >> 3;
+    if ((lane & 7) == 0) {
+      red[wv][k] = t0;
+      if (k < NMOM - 8) red[wv][8 + k] = t1;
+    }
   }
   __syncthreads();
   if (tid < NMOM) {
@@ -991,44 +1001,123 @@ struct RedOut {
 };
 
 // sum over k = 0 .. i of src[k] g[i - k] by the Q lanes of a group (q: the lane's
-// place): terms i - q, i - q - Q, ... per lane, then a fixed tree; every lane of
-// the group returns the sum.  MIXED: the terms in compensated FP32.
-__device__ __forceinline__ double conv_at(const double *src, const double *g, int i, int q, int Q, int mixed)
+// place).  The order of the additions does not depend on Q: sixteen interleaved
+// sums of every sixteenth term from k = i down, then a fixed tree over them; a
+// lane has 16 / Q of the sums.  mixed: the terms in compensated FP32.  A whole
+// group of terms is read before the first is added.
+template <int Q> __device__ __forceinline__ double conv_at(const double *src, const double *g, int i, int q, int mixed)
 {
-  double a = 0.0;
+  constexpr int A = 16 / Q, C = A > 8 ? A : 8;
+  double a[A];
   if (mixed) {
-    F2 s = {0.0f, 0.0f};
-    for (int k = i - q; k >= 0; k -= Q) f2_add_prod(s, src[k], g[i - k]);
-    a = (double)s.hi + (double)s.lo;
+    F2 s[A];
+#pragma unroll
+    for (int t = 0; t < A; t++) s[t] = {0.0f, 0.0f};
+    for (int k0 = i - q; k0 >= 0; k0 -= A * Q) {
+#pragma unroll
+      for (int t = 0; t < A; t++)
+        if (k0 - t * Q >= 0) f2_add_prod(s[t], src[k0 - t * Q], g[i - k0 + t * Q]);
+    }
+#pragma unroll
+    for (int t = 0; t < A; t++) a[t] = (double)s[t].hi + (double)s[t].lo;
   } else {
-#pragma unroll 4
-    for (int k = i - q; k >= 0; k -= Q) a += src[k] * g[i - k];
+#pragma unroll
+    for (int t = 0; t < A; t++) a[t] = 0.0;
+    int k0 = i - q;
+    for (; k0 - (C - 1) * Q >= 0; k0 -= C * Q) {
+      double u[C], w[C];
+#pragma unroll
+      for (int t = 0; t < C; t++) {
+        u[t] = src[k0 - t * Q];
+        w[t] = g[i - k0 + t * Q];
+      }
+#pragma unroll
+      for (int t = 0; t < C; t++) a[t % A] = fma(u[t], w[t], a[t % A]);
+    }
+    if (k0 >= 0) {
+      double u[C], w[C];
+#pragma unroll
+      for (int t = 0; t < C; t++) {
+        const int k = max(k0 - t * Q, 0);
+        u[t] = src[k];
+        w[t] = g[i - k];
+      }
+#pragma unroll
+      for (int t = 0; t < C; t++) {
+        const double v = fma(u[t], w[t], a[t % A]);
+        a[t % A] = k0 - t * Q >= 0 ? v : a[t % A];
+      }
+    }
   }
-  for (int o = Q >> 1; o >= 1; o >>= 1) a += __shfl_xor(a, o, Q);
-  return a;
+  // sum r of the sixteen is lane r % Q's a[r / Q]: partners r ^ 8, r ^ 4, r ^ 2, r ^ 1
+#pragma unroll
+  for (int o = 8; o >= Q; o >>= 1)
+#pragma unroll
+    for (int t = 0; t < o / Q; t++) a[t] += a[t + o / Q];
+#pragma unroll
+  for (int o = Q > 8 ? 8 : Q >> 1; o >= 1; o >>= 1) a[0] += __shfl_xor(a[0], o, Q);
+  return a[0];
 }
 
 // phase: 0 = means only (shift <- mean), 1 = initial statistics + RW history
 // fill, 2 = turn, 3 = final statistics.
-// Bound: latency (one block per bunch, a chain of loads, sums and convolutions).
-// The convolutions take two slices i and Nc - 1 - i per group of Q lanes, so that
-// every lane has the same (Nc + 1) / Q terms and only the planes that have a wake
-// are visited: 333 bunches x 50 slices with the sums and own wakes of three
-// resonators 26.7 -> 14.7 us (one lane per slice and plane before), 416 x 100
-// without resonators 18.6 -> 17.
-__global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr, const double *__restrict__ partial,
+// Bound: latency, one block per bunch after a pass that left its inputs in other
+// XCDs' reach.  So every load that needs only the bunch is under way before the
+// first is waited for, the ring's constants are copied to LDS in one go, the
+// statistics (wave 3) run beside the histogram (waves 0 ..), and the convolutions
+// take two slices i and Nc - 1 - i per group of Q lanes, so that every lane has the
+// same (Nc + 1) / Q terms and only the planes that have a wake are visited.  One
+// bunch x 100 slices x 3 planes 16.1 -> 9.1 us, 64 x 50 slices 10.0 -> 5.9, 416 x
+// 100 18.6 -> 10.2, 333 x 50 with three LR resonators 26.7 -> 10.1 (one lane per slice
+// and plane, loads waited for one by one, the statistics and 64-bit remainders in
+// front of the rest).
+template <int NT, int Q>
+__global__ __launch_bounds__(NT) void k_reduce(const DevParams *__restrict__ Pr, const double *__restrict__ partial,
                                                const int *__restrict__ bunch_wg0, const int *__restrict__ bunch_ring,
                                                const int *__restrict__ bucket, HistPtr H, RedOut R,
                                                const TurnState *__restrict__ tsr, int phase, int dip, LRDev LR,
-                                               int lr_lds)
+                                               int lr_lds, int turn, int Nc)
 {
   extern __shared__ double sm[];
+  __shared__ DevParams P;
+  __shared__ double edge[3][2];
+  __shared__ double mom[NMOM];
+  __shared__ int icmin_s, icmax_s;
   const int b = blockIdx.x, tid = threadIdx.x;
-  const int ring = bunch_ring[b];
-  const DevParams &P = Pr[ring];
+  const int ring = bunch_ring[b], kb = bucket[b], np = R.np[b];
+  const int w0 = bunch_wg0[b], w1 = bunch_wg0[b + 1];
+  const bool hist = phase != 0 && Nc > 0;
+  // the bunch's own inputs: histogram (the first NT slices), trash, shift, current
+  unsigned int cnt0 = 0, tc[2] = {0, 0};
+  unsigned long long xl0 = 0, xh0 = 0, zl0 = 0, zh0 = 0;
+  int badf = 0, pend = 0, tot = 0;
+  double Ib = 0.0, shift = 0.0;
+  if (hist) {
+    const size_t g = (size_t)b * Nc + min(tid, Nc - 1);
+    cnt0 = H.cnt[g];
+    if (dip) {
+      xl0 = H.sx[2 * g];
+      xh0 = H.sx[2 * g + 1];
+      zl0 = H.sz[2 * g];
+      zh0 = H.sz[2 * g + 1];
+    }
+    tc[0] = H.tcnt[2 * b];
+    tc[1] = H.tcnt[2 * b + 1];
+    badf = H.bad[b];
+    Ib = R.bunch_Ib[b];
+    if (tid < 2) {
+      pend = R.trash_pend[2 * b + tid];
+      tot = R.trash_tot[2 * b + tid];
+    }
+  }
+  if (tid >= 192 && tid < 198) shift = R.shift[b * 6 + tid - 192];
+  {
+    const unsigned long long *src = (const unsigned long long *)(Pr + ring);
+    unsigned long long *dst = (unsigned long long *)&P;
+    for (int i = tid; i < (int)(sizeof(DevParams) / 8); i += NT) dst[i] = src[i];
+  }
   const TurnState *ts = tsr + ring;
-  const int kb = bucket[b];
-  const int Nc = P.Nc;
+  const long long rev = ts->rev + turn;
   double *fnp = sm;
   double *dV = fnp + Nc;
   double *dH = dV + Nc;
@@ -1036,14 +1125,6 @@ __global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr,
   // with LR resonators: their own wakes, [plane][Nc], in LDS where it holds them,
   // and the edge slices' sums without the particles beyond them
   const double *Gl = lr_lds ? Gs + 3 * Nc : LR.G + (size_t)ring * 3 * Nc;
-  __shared__ double edge[3][2];
-  __shared__ double mom[NMOM];
-  __shared__ int icmin_s, icmax_s;
-  const long long rev = ts->rev;
-  const int w0 = bunch_wg0[b], w1 = bunch_wg0[b + 1];
-  // the final statistics leave the wakes of the next turn alone
-  const bool lrp = (phase == 1 || phase == 2) && P.lrp[3] > P.lrp[0];
-  const double Np = (double)R.np[b];
   {
     // moment sums over the bunch's workgroups: 16 lanes per moment, each summing
     // every 16th workgroup in order, then a fixed butterfly over the 16 lanes
@@ -1052,35 +1133,38 @@ __global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr,
     if (q < NMOM)
 #pragma unroll 4
       for (int w = w0 + j; w < w1; w += 16) s += partial[(size_t)w * NMOM + q];
+    if (hist) {
+      const double *Gr = R.G + (size_t)ring * 3 * Nc;
+      for (int i = tid; i < 3 * Nc; i += NT) Gs[i] = Gr[i];
+      if (lr_lds) {
+        const double *Lr = LR.G + (size_t)ring * 3 * Nc;
+        for (int i = tid; i < 3 * Nc; i += NT) Gs[3 * Nc + i] = Lr[i];
+      }
+    }
     for (int o = 8; o >= 1; o >>= 1) s += __shfl_xor(s, o, 16);
     if (q < NMOM && j == 0) mom[q] = s;
-  }
-  if (phase != 0 && Nc > 0) {
-    const double *Gr = R.G + (size_t)ring * 3 * Nc;
-    for (int i = tid; i < 3 * Nc; i += WG) Gs[i] = Gr[i];
-    if (lrp && lr_lds) {
-      const double *Lr = LR.G + (size_t)ring * 3 * Nc;
-      for (int i = tid; i < 3 * Nc; i += WG) Gs[3 * Nc + i] = Lr[i];
-    }
   }
   if (tid == 0) {
     icmin_s = Nc - 1;
     icmax_s = 0;
   }
   __syncthreads();
-  const int slot = (int)(((rev % STATS_TURNS) + STATS_TURNS) % STATS_TURNS);
-  if (tid < 6) {
+  const int slot = (int)(rev & (STATS_TURNS - 1));
+  // the final statistics leave the wakes of the next turn alone
+  const bool lrp = (phase == 1 || phase == 2) && P.lrp[3] > P.lrp[0];
+  if (tid >= 192 && tid < 198) {
     // one lane per coordinate (tau, delta, x, x', z, z')
-    const int pl = tid >> 1, c = tid & 1;
+    const int k = tid - 192, pl = k >> 1, c = k & 1;
+    const double Np = (double)np;
     const bool track = pl == 0 || (pl == 1 ? P.track_h : P.track_v);
-    const double mp = mom[tid] / Np, v = mom[6 + tid] / Np - mp * mp;
-    const double mean = track ? R.shift[b * 6 + tid] + mp : 0.0;
-    R.shift[b * 6 + tid] = mean;
+    const double mp = mom[k] / Np, v = mom[6 + k] / Np - mp * mp;
+    const double mean = track ? shift + mp : 0.0;
+    R.shift[b * 6 + k] = mean;
     if (phase != 0) {
       double *o = R.stats + ((size_t)slot * R.Gtot + b) * 12 + 6 * c + pl;
       o[0] = mean;
       o[3] = track ? sqrt(v > 0.0 ? v : 0.0) : 0.0;
-      if (phase == 2 && (rev + 1) % P.monitor_every == 0) {
+      if (phase == 2 && umod(rev + 1, (unsigned)P.monitor_every) == 0) {
         const double other = __shfl_xor(mean, 1, 2), pos = c ? other : mean, slope = c ? mean : other;
         double *a = R.amp + ((size_t)slot * R.Gtot + b) * 6 + 3 * c + pl;
         *a = !track ? 0.0
@@ -1089,24 +1173,25 @@ __global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr,
                                     P.beta1[pl] * (slope * slope));
       }
       if (P.rw && phase != 3 && c == 0 && pl > 0) {
-        double *hist = R.rwhist + P.rw_off + pl - 1;
-        const long long n = (long long)(P.Nmlt + 2) * P.h;
-        const long long k = (phase == 1 ? 0 : -rev * P.h) + kb;
-        hist[2 * (((k % n) + n) % n)] = mean;
+        // the turn's row of the cyclic history (rows go backwards), at the start
+        // also the rows of the Nmlt - 1 turns before
+        double *row = R.rwhist + P.rw_off + 2 * kb + pl - 1;
+        const int rows = P.Nmlt + 2, r0 = phase == 1 ? 0 : (int)((rows - umod(rev, rows)) % rows);
+        row[2LL * r0 * P.h] = mean;
         if (phase == 1)
-          for (int jj = 1; jj < P.Nmlt; jj++) hist[2 * (((long long)jj * P.h + kb) % n)] = mean;
+          for (int jj = 1; jj < P.Nmlt; jj++) row[2LL * jj * P.h] = mean;
       }
     }
   }
-  if (phase == 2 && b == P.bunch_off && tid == 64) {
+  if (phase == 2 && b == P.bunch_off && tid == 255) {
     // nothing changes phai0 / Vrf0 between the map and this point of the turn
     R.rfbuf[((size_t)slot * R.R + ring) * 2] = ts->phai0;
     R.rfbuf[((size_t)slot * R.R + ring) * 2 + 1] = ts->Vrf0;
   }
-  if (phase == 0 || Nc <= 0) {
+  if (!hist) {
     // consume (and clear) the histogram only on the stats passes
-    if (phase == 0 && Nc > 0) {
-      for (int i = tid; i < Nc; i += WG) {
+    if (Nc > 0) {
+      for (int i = tid; i < Nc; i += NT) {
         size_t g = (size_t)b * Nc + i;
         H.cnt[g] = 0;
         H.sx[2 * g] = H.sx[2 * g + 1] = 0;
@@ -1125,36 +1210,42 @@ __global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr,
   // dip = 0: the pass before (a turn pass without dipole histograms) left the
   // dipole sums at the zeros the last clear wrote, so they are neither read
   // nor cleared here (the outputs get the same zeros)
-  const bool bad = H.bad[b] != 0;
-  for (int i = tid; i < Nc; i += WG) {
-    size_t g = (size_t)b * Nc + i;
-    unsigned int c = H.cnt[g];
-    unsigned long long xl = 0, xh = 0, zl = 0, zh = 0;
-    if (dip) {
-      xl = H.sx[2 * g];
-      xh = H.sx[2 * g + 1];
-      zl = H.sz[2 * g];
-      zh = H.sz[2 * g + 1];
+  const bool bad = badf != 0;
+  for (int i = tid; i < Nc; i += NT) {
+    const size_t g = (size_t)b * Nc + i;
+    unsigned int c = cnt0;
+    unsigned long long xl = xl0, xh = xh0, zl = zl0, zh = zh0;
+    if (i >= NT) {
+      c = H.cnt[g];
+      if (dip) {
+        xl = H.sx[2 * g];
+        xh = H.sx[2 * g + 1];
+        zl = H.sz[2 * g];
+        zh = H.sz[2 * g + 1];
+      }
     }
     if (i == 0 || i == Nc - 1) {
       // dropped: the sums of the edge slices alone; clamped: out-of-range
       // particles join them (one slice takes both edges)
+      const double n = (double)c, ex = bad ? NAN : fx_to_double(xl, xh), ez = bad ? NAN : fx_to_double(zl, zh);
       for (int e = 0; e < 2; e++) {
         if (i != (e ? Nc - 1 : 0)) continue;
-        edge[0][e] = (double)H.cnt[g];
-        edge[1][e] = bad ? NAN : fx_to_double(dip ? H.sx[2 * g] : 0, dip ? H.sx[2 * g + 1] : 0);
-        edge[2][e] = bad ? NAN : fx_to_double(dip ? H.sz[2 * g] : 0, dip ? H.sz[2 * g + 1] : 0);
-        c += H.tcnt[2 * b + e];
+        edge[0][e] = n;
+        edge[1][e] = ex;
+        edge[2][e] = ez;
+        c += tc[e];
         if (!dip) continue;
         fx_add(xl, xh, H.tsx[4 * b + 2 * e], H.tsx[4 * b + 2 * e + 1]);
         fx_add(zl, zh, H.tsz[4 * b + 2 * e], H.tsz[4 * b + 2 * e + 1]);
       }
     }
     // icellmin / icellmax of src/transform_weak.c:633-651: the first and last
-    // occupied slice (Nc - 1 and 0 when there is none)
-    if (c > 0) {
+    // occupied slice (Nc - 1 and 0 when there is none), one update per wave
+    const unsigned long long occ = __ballot(c > 0);
+    if (c > 0 && (tid & 63) == __ffsll((long long)occ) - 1) {
+      const int i0 = i - (tid & 63);
       atomicMin(&icmin_s, i);
-      atomicMax(&icmax_s, i);
+      atomicMax(&icmax_s, i0 + 63 - __clzll((long long)occ));
     }
     const double n = (double)c, sz = bad ? NAN : fx_to_double(zl, zh), sx = bad ? NAN : fx_to_double(xl, xh);
     fnp[i] = n;
@@ -1163,26 +1254,19 @@ __global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr,
     R.fnp_out[g] = n;
     R.dipV_out[g] = sz;
     R.dipH_out[g] = sx;
-  }
-  if (tid == 0) {
-    // trash counters: the previous pending binning is consumed by this turn's kick
-    if (phase == 2) {
-      R.trash_tot[2 * b] += R.trash_pend[2 * b];
-      R.trash_tot[2 * b + 1] += R.trash_pend[2 * b + 1];
-    }
-    R.trash_pend[2 * b] = (int)H.tcnt[2 * b];
-    R.trash_pend[2 * b + 1] = (int)H.tcnt[2 * b + 1];
-  }
-  __syncthreads();
-  // clear accumulators for the next pass
-  for (int i = tid; i < Nc; i += WG) {
-    size_t g = (size_t)b * Nc + i;
+    // clear the accumulators for the next pass
     H.cnt[g] = 0;
     if (dip) {
       H.sx[2 * g] = H.sx[2 * g + 1] = 0;
       H.sz[2 * g] = H.sz[2 * g + 1] = 0;
     }
   }
+  if (tid < 2) {
+    // trash counters: the previous pending binning is consumed by this turn's kick
+    if (phase == 2) R.trash_tot[2 * b + tid] = tot + pend;
+    R.trash_pend[2 * b + tid] = (int)tc[tid];
+  }
+  __syncthreads();
   if (tid < 2) {
     H.tcnt[2 * b + tid] = 0;
     if (dip) {
@@ -1193,55 +1277,47 @@ __global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr,
   if (tid == 0) H.bad[b] = 0;
   const int icmin = icmin_s, icmax = icmax_s;
   // the next turn's kick uses the current after this turn's scan step (src/tracking.c:43-59)
-  double Ib = R.bunch_Ib[b];
   if (phase == 2 && P.scan == 1 && (rev + 1) % P.NrevScan == 0) Ib += P.scan_step / (((double)P.Nb) * 1.0e3);
-  const double factG = -P.T0 * Ib / (R.np[b] * P.E0 * 1.0e9);
+  const double factG = -P.T0 * Ib / (np * P.E0 * 1.0e9);
   const double sgm = P.sigma_tau, sgm2 = sgm * sgm, dT2 = P.dT * P.dT;
   const int np2 = (Nc + 1) >> 1; // pairs of slices (i, Nc - 1 - i)
-  int Q = 16;
-  while (Q > 1 && Q * np2 > WG) Q >>= 1;
   const int q = tid & (Q - 1);
-  if (P.convL || P.kickV || P.kickH || P.sf_active)
-    for (int t = tid / Q; t < np2; t += WG / Q)
-      for (int half = 0; half < 2; half++) {
-        const int i = half ? t : Nc - 1 - t;
-        if (half && i == Nc - 1 - t) break; // the middle slice of an odd count
-        const size_t g = (size_t)b * Nc + i;
-        {
-          double val = 0.0;
-          if (P.convL && i >= icmin) {
-            // slices below icmin are empty: nothing to add from them
-            double GL1 = conv_at(fnp, Gs, i, q, Q, P.mixed);
-            // resistive and inductive smoothing, src/transform_weak.c:670-683; reads
-            // outside [0, Ncell) count as zero
+  for (int t = tid / Q; t < np2; t += NT / Q)
+    for (int half = 0; half < 2; half++) {
+      const int i = half ? t : Nc - 1 - t;
+      if (half && i == Nc - 1 - t) break; // the middle slice of an odd count
+      const size_t g = (size_t)b * Nc + i;
+      double val = 0.0;
+      if (P.convL && i >= icmin) {
+        // slices below icmin are empty: nothing to add from them
+        double GL1 = conv_at<Q>(fnp, Gs, i, q, P.mixed);
+        // resistive and inductive smoothing, src/transform_weak.c:670-683; reads
+        // outside [0, Ncell) count as zero
 #define F(k) (((k) >= 0 && (k) < Nc) ? fnp[k] : 0.0)
-            if (P.RsisL > 0 && i >= icmin + 1 && i <= icmax) {
-              double nt = (0.5 * F(i - 1) + F(i) + 0.5 * F(i + 1)) / 2.0;
-              GL1 += P.RsisL * nt / (sgm * P.dT);
-            }
-            if (P.aindL > 0 && i >= icmin + 1 && i <= icmax) {
-              double n0 = (0.25 * F(i - 3) + 0.5 * F(i - 2) + F(i - 1) + 0.5 * F(i) + 0.25 * F(i + 1)) / 2.5;
-              double n1 = (0.25 * F(i - 1) + 0.5 * F(i) + F(i + 1) + 0.5 * F(i + 2) + 0.25 * F(i + 3)) / 2.5;
-              GL1 += (n1 - n0) / (2.0 * sgm2 * dT2) * P.aindL;
-            }
+        if (P.RsisL > 0 && i >= icmin + 1 && i <= icmax) {
+          double nt = (0.5 * F(i - 1) + F(i) + 0.5 * F(i + 1)) / 2.0;
+          GL1 += P.RsisL * nt / (sgm * P.dT);
+        }
+        if (P.aindL > 0 && i >= icmin + 1 && i <= icmax) {
+          double n0 = (0.25 * F(i - 3) + 0.5 * F(i - 2) + F(i - 1) + 0.5 * F(i) + 0.25 * F(i + 1)) / 2.5;
+          double n1 = (0.25 * F(i - 1) + 0.5 * F(i) + F(i + 1) + 0.5 * F(i + 2) + 0.25 * F(i + 3)) / 2.5;
+          GL1 += (n1 - n0) / (2.0 * sgm2 * dT2) * P.aindL;
+        }
 #undef F
-            val = GL1;
-          }
-          if (q == 0) R.sfL[g] = factG * val;
-        }
-        // a plane without a kick keeps the +0.0 of its allocation (its value
-        // here, -factG * 0 with factG <= 0), so its table is not rewritten
-        if (P.kickV) {
-          const double val = conv_at(dV, Gs + Nc, i, q, Q, P.mixed);
-          if (q == 0) R.sfV[g] = -factG * val;
-        }
-        if (P.kickH) {
-          const double val = i >= 1 ? conv_at(dH, Gs + 2 * Nc, i, q, Q, P.mixed) : 0.0;
-          if (q == 0) R.sfH[g] = -factG * val;
-        }
+        val = GL1;
       }
-  else
-    for (int i = tid; i < Nc; i += WG) R.sfL[(size_t)b * Nc + i] = factG * 0.0;
+      if (q == 0) R.sfL[g] = factG * val;
+      // a plane without a kick keeps the +0.0 of its allocation (its value
+      // here, -factG * 0 with factG <= 0), so its table is not rewritten
+      if (P.kickV) {
+        const double v = conv_at<Q>(dV, Gs + Nc, i, q, P.mixed);
+        if (q == 0) R.sfV[g] = -factG * v;
+      }
+      if (P.kickH) {
+        const double v = i >= 1 ? conv_at<Q>(dH, Gs + 2 * Nc, i, q, P.mixed) : 0.0;
+        if (q == 0) R.sfH[g] = -factG * v;
+      }
+    }
   if (!lrp) return;
   // ---- LR resonators: the histograms without the particles beyond the edges
   __syncthreads();
@@ -1252,7 +1328,7 @@ __global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr,
   __syncthreads();
   // slice sums the phasor recurrence needs, one wave per resonator
   const int nr = P.lrp[3] - P.lrp[0];
-  for (int r = P.lrp[0] + (tid >> 6); r < P.lrp[3]; r += WG / 64) {
+  for (int r = P.lrp[0] + (tid >> 6); r < P.lrp[3]; r += NT / 64) {
     const double *f = r < P.lrp[1] ? fnp : (r < P.lrp[2] ? dH : dV);
     const double2 *p = LR.pw + (size_t)r * (Nc + 1);
     double sr = 0.0, si = 0.0;
@@ -1267,13 +1343,13 @@ __global__ __launch_bounds__(WG) void k_reduce(const DevParams *__restrict__ Pr,
       LR.L[P.lr_off + (long long)(P.h - 1 - kb) * nr + r - P.lrp[0]] = make_double2(sr, si);
   }
   // the bunch's own long-range wake
-  for (int t = tid / Q; t < np2; t += WG / Q)
+  for (int t = tid / Q; t < np2; t += NT / Q)
     for (int half = 0; half < 2; half++) {
       const int i = half ? t : Nc - 1 - t;
       if (half && i == Nc - 1 - t) break;
       for (int pl = 0; pl < 3; pl++) {
         if (P.lrp[pl] == P.lrp[pl + 1]) continue;
-        const double a = conv_at(pl == 0 ? fnp : (pl == 1 ? dH : dV), Gl + pl * Nc, i, q, Q, 0);
+        const double a = conv_at<Q>(pl == 0 ? fnp : (pl == 1 ? dH : dV), Gl + pl * Nc, i, q, 0);
         if (q == 0) LR.self[((size_t)pl * LR.Gtot + b) * Nc + i] = a;
       }
     }
@@ -1343,23 +1419,19 @@ __device__ void rw_taps(const DevParams &P, int kb, long long rev, const double 
     }
 }
 
-// Turn end of one ring: RW trigger counter, current scan (src/tracking.c:43-59),
-// turn counter.
-__device__ void end_turn(const DevParams &P, TurnState *ts, double *bunch_Ib, double *Ibunch, const int *nfFill)
+// n turns of one ring are done: current scan (src/tracking.c:43-59; n = 1 then)
+// and turn counter.
+__device__ void end_turns(const DevParams &P, TurnState *ts, double *bunch_Ib, double *Ibunch, const int *nfFill, int n)
 {
-  long long rev = ts->rev;
-  if (P.rw) ts->m++;
-  if ((rev + 1) % P.NrevScan == 0) {
-    if (P.scan == 1) {
-      ts->Iring += P.scan_step;
-      ts->scan_val = ts->Iring;
-      for (int k = 0; k < P.Nb; k++) bunch_Ib[P.bunch_off + k] += P.scan_step / (((double)P.Nb) * 1.0e3);
-      for (int i = 0; i < P.h; i++)
-        if (nfFill[P.bucket_off + i]) Ibunch[P.bucket_off + i] += P.scan_step / ((double)P.Nb);
-    }
-    ts->m = 0;
+  const long long rev = ts->rev;
+  if (P.scan == 1 && (rev + 1) % P.NrevScan == 0) {
+    ts->Iring += P.scan_step;
+    ts->scan_val = ts->Iring;
+    for (int k = 0; k < P.Nb; k++) bunch_Ib[P.bunch_off + k] += P.scan_step / (((double)P.Nb) * 1.0e3);
+    for (int i = 0; i < P.h; i++)
+      if (nfFill[P.bucket_off + i]) Ibunch[P.bucket_off + i] += P.scan_step / ((double)P.Nb);
   }
-  ts->rev = rev + 1;
+  ts->rev = rev + n;
 }
 
 // RF feedback of one ring: rffb_calc_mean_voltage_phase (src/feedback_rf.c:21-34)
@@ -1400,8 +1472,8 @@ static size_t rw_old_lds(int span) { return (size_t)span * (3 * 8 + 4) + RW_TILE
 __global__ __launch_bounds__(WG) void k_rw_fresh(const DevParams *__restrict__ Pr, const int *bunch_ring,
                                                  const double *rwhist, const double *sqrt_tt, const double *Ibunch,
                                                  const int *nfFill, const int *bucket,
-                                                 const TurnState *__restrict__ tsr, const double *rw_part, int G,
-                                                 double *pending)
+                                                 const TurnState *__restrict__ tsr, int turn, const double *rw_part,
+                                                 int G, double *pending)
 {
   __shared__ double red[WG / 64][2];
   const int b = blockIdx.x, tid = threadIdx.x;
@@ -1409,9 +1481,9 @@ __global__ __launch_bounds__(WG) void k_rw_fresh(const DevParams *__restrict__ P
   const DevParams &P = Pr[ring];
   if (!P.rw) return;
   const int kb = bucket[b];
-  const TurnState *ts = tsr + ring;
+  const long long rev = tsr[ring].rev + turn;
   double fx, fz;
-  rw_taps<WG, 4>(P, kb, ts->rev, rwhist, sqrt_tt, Ibunch, nfFill, 1, (long long)(P.h - kb - 1), red, fx, fz);
+  rw_taps<WG, 4>(P, kb, rev, rwhist, sqrt_tt, Ibunch, nfFill, 1, (long long)(P.h - kb - 1), red, fx, fz);
   __syncthreads();
   // earlier rows: one tile partial per lane (fixed order)
   const int ntile = ((P.Nmlt + 1) * P.h + RW_TILE_TAPS - 1) / RW_TILE_TAPS;
@@ -1433,47 +1505,67 @@ __global__ __launch_bounds__(WG) void k_rw_fresh(const DevParams *__restrict__ P
       sx += red[w][0];
       sz += red[w][1];
     }
-    const int trig = ts->m < 50 ? 1 : 0;
+    const int trig = rw_trigger(rev, P.NrevScan);
     pending[2 * b] = P.track_h ? (sx + fx) * P.rwconst[0][trig] : 0.0;
     pending[2 * b + 1] = P.track_v ? (sz + fz) * P.rwconst[1][trig] : 0.0;
   }
 }
 
-// Small rings (the map too short to hide the earlier rows' taps): every tap in one pass, and
-// the ring's last block to finish ends the turn (every block of the ring has read
-// the turn state and the bucket currents before its increment).
-__global__ __launch_bounds__(RW_WG) void k_rw(const DevParams *__restrict__ Pr, const int *bunch_ring,
-                                              const double *rwhist, const double *sqrt_tt, double *Ibunch,
-                                              const int *nfFill, const int *bucket, double *pending,
-                                              TurnState *tsr, unsigned *ring_done, double *bunch_Ib, int fb_here)
+// Small rings (the map too short to hide the earlier rows' taps): the taps of
+// every row and bunch in one pass.  Bound: latency, so only buckets that hold
+// bunches are visited -- (Nmlt + 2) Nb pairs of a row and a bunch instead of
+// (Nmlt + 1) h taps -- and each multiplies by the tabulated 1 / sqrt(t).  64
+// bunches of h = 416, 19 turns: 9.6 -> 5.1 us (256 lanes per bunch: 5.6).
+__global__ __launch_bounds__(RW_WG) void k_rw(const DevParams *__restrict__ Pr, const int *__restrict__ bunch_ring,
+                                           const double *__restrict__ rwhist, const double *__restrict__ rsqrt_tt,
+                                           const double *__restrict__ Ibunch, const int *__restrict__ nfFill,
+                                           const int *__restrict__ bucket, double *pending,
+                                           const TurnState *__restrict__ tsr, int turn)
 {
   __shared__ double red[RW_WG / 64][2];
-  __shared__ int last;
   const int b = blockIdx.x, tid = threadIdx.x;
   const int ring = bunch_ring[b];
   const DevParams &P = Pr[ring];
-  TurnState *ts = tsr + ring;
-  if (P.rw) {
-    const int kb = bucket[b];
-    double sx, sz;
-    rw_taps<RW_WG, 4>(P, kb, ts->rev, rwhist, sqrt_tt, Ibunch, nfFill, 1, (long long)(P.Nmlt + 1) * P.h, red, sx,
-                      sz);
-    if (tid == 0) {
-      const int trig = ts->m < 50 ? 1 : 0;
-      pending[2 * b] = P.track_h ? sx * P.rwconst[0][trig] : 0.0;
-      pending[2 * b + 1] = P.track_v ? sz * P.rwconst[1][trig] : 0.0;
+  if (!P.rw) return;
+  const int kb = bucket[b], h = P.h, Nb = P.Nb, R = P.Nmlt + 2, M = (P.Nmlt + 1) * h;
+  const long long rev = tsr[ring].rev + turn;
+  const int *bk = bucket + P.bunch_off, *fill = nfFill + P.bucket_off;
+  const double2 *hist = (const double2 *)(rwhist + P.rw_off);
+  const double *rs = rsqrt_tt + P.st_off, *Ib = Ibunch + P.bucket_off;
+  // row j turns ago sits j rows after the newest, cyclically
+  const int new_row = (int)((R - umod(rev, R)) % R);
+  const int dj = RW_WG / Nb, ds = RW_WG % Nb;
+  int j = tid / Nb, q = tid % Nb;
+  double ax = 0.0, az = 0.0;
+#pragma unroll 4
+  for (int e = tid; e < R * Nb; e += RW_WG) {
+    const int k = bk[q], m = j * h + k - kb;
+    const int row = new_row + j >= R ? new_row + j - R : new_row + j;
+    const double2 d = hist[row * h + k];
+    const double w = rs[min(max(m, 1), M)], I = Ib[k];
+    const bool on = m >= 1 && m <= M && fill[k];
+    const double tx = P.fNp * d.x * I * w, tz = P.fNp * d.y * I * w;
+    ax += on ? tx : 0.0;
+    az += on ? tz : 0.0;
+    j += dj;
+    q += ds;
+    if (q >= Nb) {
+      q -= Nb;
+      j++;
     }
   }
-  if (tid == 0) {
-    __threadfence();
-    last = atomicAdd(&ring_done[ring], 1u) == (unsigned)(P.Nb - 1);
+  ax = wave_sum(ax);
+  az = wave_sum(az);
+  if ((tid & 63) == 0) {
+    red[tid >> 6][0] = ax;
+    red[tid >> 6][1] = az;
   }
   __syncthreads();
-  if (last && tid == 0) {
-    __threadfence();
-    ring_done[ring] = 0;
-    end_turn(P, ts, bunch_Ib, Ibunch, nfFill);
-    if (fb_here) fb_solve(P, ts, nullptr, 0);
+  if (tid < 2) {
+    double s = 0.0;
+    for (int w = 0; w < RW_WG / 64; w++) s += red[w][tid];
+    const int trig = rw_trigger(rev, P.NrevScan);
+    pending[2 * b + tid] = (tid ? P.track_v : P.track_h) ? s * P.rwconst[tid][trig] : 0.0;
   }
 }
 
@@ -1583,7 +1675,7 @@ __device__ __forceinline__ void rwg_rows(const double *Yf, const double *cs, int
 
 template <bool F32>
 __global__ __launch_bounds__(256) void k_rwg_tile(RWGemm Gm, const DevParams *__restrict__ Pr,
-                                                const TurnState *__restrict__ tsr, const double *rwhist,
+                                                const TurnState *__restrict__ tsr, int turn, const double *rwhist,
                                                 const double *Ibunch, const int *nfFill)
 {
   extern __shared__ double sm[];
@@ -1607,7 +1699,7 @@ __global__ __launch_bounds__(256) void k_rwg_tile(RWGemm Gm, const DevParams *__
     const int ring = j < Gm.N ? Gm.col_ring[j >> 1] : -1;
     yring[tid] = ring;
     if (ring >= 0) {
-      long long k0 = (-tsr[ring].rev * h + A0) % Gm.n;
+      long long k0 = (-(tsr[ring].rev + turn) * h + A0) % Gm.n;
       ybase[tid] = k0 < 0 ? k0 + Gm.n : k0;
       yboff[tid] = Pr[ring].bucket_off;
       yroff[tid] = Pr[ring].rw_off;
@@ -1661,7 +1753,7 @@ __global__ __launch_bounds__(256) void k_rwg_tile(RWGemm Gm, const DevParams *__
 // one lane per (bucket, column): the K slices summed in a fixed order, then the
 // pending kick of the bucket's bunch (the ring's fNp and RW constant applied)
 __global__ __launch_bounds__(256) void k_rwg_sum(RWGemm Gm, const DevParams *__restrict__ Pr,
-                                               const TurnState *__restrict__ tsr, double *pending)
+                                               const TurnState *__restrict__ tsr, int turn, double *pending)
 {
   const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
   if (e >= (long long)Gm.h * Gm.N) return;
@@ -1672,7 +1764,7 @@ __global__ __launch_bounds__(256) void k_rwg_sum(RWGemm Gm, const DevParams *__r
   if (g < 0) return;
   double sum = 0.0;
   for (int ks = 0; ks < Gm.KS; ks++) sum += Gm.part[((size_t)ks * Gm.HP + kb) * Gm.N + col];
-  const int trig = tsr[ring].m < 50 ? 1 : 0;
+  const int trig = rw_trigger(tsr[ring].rev + turn, P.NrevScan);
   const bool on = pl == 0 ? P.track_h : P.track_v;
   pending[2 * g + pl] = on ? (P.fNp * sum) * P.rwconst[pl][trig] : 0.0;
 }
@@ -1767,7 +1859,7 @@ __device__ double2 lr_turn(const LRConst &L, const LRDev &R, const DevParams &P,
   return V0;
 }
 
-// One block per ring: the turn end (end), the phasors of its resonators (a wave
+// One block per ring: the end of `end` turns, the phasors of its resonators (a wave
 // each), the RF-feedback samples and the RF-feedback solve.  init:
 // wake_phasor_init (src/transform_weak.c:869-952), the same turn replayed
 // init_turns times from a zero phasor, one wave in order taking the samples.
@@ -1777,7 +1869,7 @@ __global__ __launch_bounds__(256) void k_ring_end(const DevParams *__restrict__ 
   const int ring = blockIdx.x, tid = threadIdx.x, lane = tid & 63, nw = blockDim.x >> 6;
   const DevParams &P = Pr[ring];
   TurnState *ts = tsr + ring;
-  if (end && tid == 0) end_turn(P, ts, bunch_Ib, Ibunch, nfFill);
+  if (end && tid == 0) end_turns(P, ts, bunch_Ib, Ibunch, nfFill, end);
   const int lr0 = P.lrp[0], nr = P.lrp[3] - lr0;
   if (nr == 0) {
     if (tid == 0) fb_solve(P, ts, R.fb_hist, init);
@@ -1906,7 +1998,7 @@ struct mbt_ring {
   double *rw_part;     // [tap tiles][G][2] partial sums of earlier turns' rows
   int rw_ntile;
   size_t rw_lds;
-  unsigned *ring_done; // [R] blocks of the ring done with the turn's fused RW pass
+  int end_each;        // rings whose turn end the next turn's launches read: LR resonators, current scan
   int rw_split;        // RW sum split: earlier rows' taps in k_turn's leading blocks, then k_rw_fresh
   GraphEntry graphs[NGRAPH];
   int graph_next, use_graphs;
@@ -2099,7 +2191,7 @@ extern "C" void mbt_ring_destroy(mbt_ring *r)
                   r->P, r->partial, r->shift, r->Hs.cnt, r->Hs.sx, r->Hs.sz, r->Hs.tcnt, r->Hs.tsx,
                   r->Hs.tsz, r->Hs.bad, r->sfL, r->sfV, r->sfH, r->Gf, r->pending, r->peek,
                   r->rwhist, r->sqrt_tt, r->rsqrt_tt, r->Ibunch, r->bunch_Ib, r->stats, r->amp, r->rfbuf, r->fnp_out,
-                  r->dipV_out, r->dipH_out, r->trash_tot, r->trash_pend, r->ts, r->rw_tiles, r->rw_part, r->ring_done, r->lc, r->lr_pw, r->lr_L,
+                  r->dipV_out, r->dipH_out, r->trash_tot, r->trash_pend, r->ts, r->rw_tiles, r->rw_part, r->lc, r->lr_pw, r->lr_L,
                   r->lr_V, r->lr_G, r->lr_self, r->lr_row, r->fb_hist,
                   r->rwg_col_ring, r->rwg_bucket_bunch, r->rwg_c, r->rwg_part};
   for (size_t i = 0; i < sizeof ptrs / sizeof ptrs[0]; i++)
@@ -2727,7 +2819,6 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
   DA(r->trash_tot, (size_t)G * 2);
   DA(r->trash_pend, (size_t)G * 2);
   DA(r->ts, R);
-  DA(r->ring_done, R);
   DA(r->fb_hist, fbh_total > 0 ? fbh_total : 2);
   // ---- long-range resonator constants (host libm, reference formulas)
   int nres = 0;
@@ -2887,6 +2978,9 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
   Ro.rfbuf = r->rfbuf;
   Ro.R = R;
   r->use_graphs = !(flags & MBT_RING_NO_GRAPHS);
+  r->end_each = nres > 0;
+  for (int k = 0; k < R; k++)
+    if (r->Ph[k].scan == 1) r->end_each = 1;
   for (int d = 0; d < 2; d++) r->lds_turn[d] = turn_lds(Nc, d);
   r->lr_lds = nres > 0 && (size_t)9 * NcA * 8 + 64 <= 64 * 1024;
   r->lds_red = (size_t)(r->lr_lds ? 9 : 6) * NcA * 8 + 64;
@@ -3067,7 +3161,7 @@ extern "C" int mbt_ring_get_bunch(const mbt_ring *r, int ib, double *s) { return
 typedef void (*turn_kernel_t)(const DevParams *, Coords, const long long *, const long long *, const int *,
                               const int *, const int *, const long long *, const double *, const double *,
                               const double *, const double *, LRDev, const double *, const double *, double *,
-                              HistPtr, const TurnState *, RwOld);
+                              HistPtr, const TurnState *, int, RwOld);
 
 #define TK(Q, D, G, M) k_turn<MODE_TURN, Q, D, G, M>
 static const turn_kernel_t g_turn_kernels[16] = {
@@ -3084,7 +3178,7 @@ static const turn_kernel_t g_tune_kernels[8] = {TT(false, false, false), TT(fals
                                                 TT(true, true, false),   TT(true, true, true)};
 #undef TT
 
-static int launch_turn_pass(mbt_ring *r, int mode)
+static int launch_turn_pass(mbt_ring *r, int mode, int turn)
 {
   turn_kernel_t k;
   if (mode == MODE_STATS) k = k_turn<MODE_STATS, false, true, true, false>;
@@ -3103,18 +3197,42 @@ static int launch_turn_pass(mbt_ring *r, int mode)
   }
   hipLaunchKernelGGL(k, dim3(r->nwg + ro.nlead), dim3(WG), lds, r->stream, r->P, r->C, r->wg_first, r->wg_end,
                      r->wg_bunch, r->bunch_ring, r->bucket, r->bunch_first, r->shift, r->sfL, r->sfV, r->sfH,
-                     r->LR, r->Ibunch, r->pending, r->partial, r->Hs, r->ts, ro);
+                     r->LR, r->Ibunch, r->pending, r->partial, r->Hs, r->ts, turn, ro);
   CK(hipGetLastError());
   return MBT_OK;
 }
 
-static int launch_reduce(mbt_ring *r, int phase)
+typedef void (*reduce_kernel_t)(const DevParams *, const double *, const int *, const int *, const int *, HistPtr, RedOut,
+                                const TurnState *, int, int, LRDev, int, int, int);
+
+// k_reduce for Nc slices: the most lanes per pair of slices (of sixteen) that a
+// block has.  A block of 1,024 lanes per bunch while that is no more than a block
+// per CU, else 256 (the sums are the same: conv_at).
+#define REDUCE_WIDE 1024
+#define REDUCE_WIDE_BUNCHES 256
+
+static reduce_kernel_t reduce_kernel(int Nc, bool wide)
+{
+  const int lanes = (wide ? REDUCE_WIDE : WG) / ((Nc + 1) / 2 > 0 ? (Nc + 1) / 2 : 1);
+  if (wide)
+    return lanes >= 16 ? k_reduce<REDUCE_WIDE, 16>
+                       : (lanes >= 8 ? k_reduce<REDUCE_WIDE, 8>
+                                     : (lanes >= 4 ? k_reduce<REDUCE_WIDE, 4>
+                                                   : (lanes >= 2 ? k_reduce<REDUCE_WIDE, 2> : k_reduce<REDUCE_WIDE, 1>)));
+  return lanes >= 16 ? k_reduce<WG, 16>
+                     : (lanes >= 8 ? k_reduce<WG, 8>
+                                   : (lanes >= 4 ? k_reduce<WG, 4> : (lanes >= 2 ? k_reduce<WG, 2> : k_reduce<WG, 1>)));
+}
+
+static int launch_reduce(mbt_ring *r, int phase, int turn)
 {
   // the statistics passes (phases 0, 1, 3) always make the dipole sums; a turn
   // pass only when a ring's kicks or LR resonators need them
   const int dip = phase != 2 || r->any_dip;
-  hipLaunchKernelGGL(k_reduce, dim3(r->G), dim3(WG), r->lds_red, r->stream, r->P, r->partial, r->bunch_wg0,
-                     r->bunch_ring, r->bucket, r->Hs, r->Ro, r->ts, phase, dip, r->LR, r->lr_lds);
+  const bool wide = r->G <= REDUCE_WIDE_BUNCHES;
+  hipLaunchKernelGGL(reduce_kernel(r->Nc, wide), dim3(r->G), dim3(wide ? REDUCE_WIDE : WG), r->lds_red, r->stream, r->P, r->partial, r->bunch_wg0,
+                     r->bunch_ring, r->bucket, r->Hs, r->Ro, r->ts, phase, dip, r->LR, r->lr_lds,
+                     turn, r->Nc);
   CK(hipGetLastError());
   return MBT_OK;
 }
@@ -3167,11 +3285,11 @@ extern "C" int mbt_ring_prepare(mbt_ring *r, double *init_stats)
   int rc;
   // two stats passes: means (shift 0), then moments about the means + histograms
   CK(hipMemsetAsync(r->shift, 0, (size_t)r->G * 6 * sizeof(double), r->stream));
-  if ((rc = launch_turn_pass(r, MODE_STATS))) return rc;
-  if ((rc = launch_reduce(r, 0))) return rc;
-  if ((rc = launch_turn_pass(r, MODE_STATS))) return rc;
+  if ((rc = launch_turn_pass(r, MODE_STATS, 0))) return rc;
+  if ((rc = launch_reduce(r, 0, 0))) return rc;
+  if ((rc = launch_turn_pass(r, MODE_STATS, 0))) return rc;
   // the initial statistics land in slot (rev=0) and the RW history rows 0..Nmlt-1
-  if ((rc = launch_reduce(r, 1))) return rc;
+  if ((rc = launch_reduce(r, 1, 0))) return rc;
   if (init_stats) {
     CK(hipStreamSynchronize(r->stream));
     CK(hipMemcpy(init_stats, r->stats, (size_t)r->G * 12 * sizeof(double), hipMemcpyDeviceToHost));
@@ -3198,46 +3316,51 @@ extern "C" int mbt_ring_prepare(mbt_ring *r, double *init_stats)
   return MBT_OK;
 }
 
-// One turn's launches.  The reference runs the long-range wakes and the
-// RF-feedback solve at the start of a turn; they run here at the end of the
-// previous one (nothing changes their inputs in between).  With E, events
-// E[0..4] bracket the kernel classes for per-kernel timing.
-static int enqueue_turn(mbt_ring *r, hipEvent_t *E)
+// One turn's launches, turn `turn` of a block.  The reference runs the long-range
+// wakes and the RF-feedback solve at the start of a turn; they run here at the end
+// of the previous one (nothing changes their inputs in between).  Only long-range
+// resonators and a current scan change what the next turn's launches read of the
+// turn state; without them the launches count the turns of a block themselves and
+// one turn end serves the block (end_block).  With E, events E[0..4] bracket the
+// kernel classes for per-kernel timing.
+static int enqueue_turn(mbt_ring *r, hipEvent_t *E, int turn)
 {
   int rc;
-  const int rw_split = r->rw_split;
+  if (r->end_each) turn = 0;
   if (E) CK(hipEventRecord(E[0], r->stream));
-  if ((rc = launch_turn_pass(r, MODE_TURN))) return rc;
+  if ((rc = launch_turn_pass(r, MODE_TURN, turn))) return rc;
   if (E) CK(hipEventRecord(E[1], r->stream));
-  if ((rc = launch_reduce(r, 2))) return rc;
+  if ((rc = launch_reduce(r, 2, turn))) return rc;
   if (E) CK(hipEventRecord(E[2], r->stream));
   if (r->rwg_on) {
     const dim3 tg((r->rwg.N + 15) / 16, r->rwg.KS);
     const size_t lds = rwg_lds(r->rwg.per, r->rwg.HP);
     if (r->mixed)
-      hipLaunchKernelGGL(k_rwg_tile<true>, tg, dim3(256), lds, r->stream, r->rwg, r->P, r->ts, r->rwhist, r->Ibunch,
-                         r->nfFill);
+      hipLaunchKernelGGL(k_rwg_tile<true>, tg, dim3(256), lds, r->stream, r->rwg, r->P, r->ts, turn, r->rwhist,
+                         r->Ibunch, r->nfFill);
     else
-      hipLaunchKernelGGL(k_rwg_tile<false>, tg, dim3(256), lds, r->stream, r->rwg, r->P, r->ts, r->rwhist, r->Ibunch,
-                         r->nfFill);
+      hipLaunchKernelGGL(k_rwg_tile<false>, tg, dim3(256), lds, r->stream, r->rwg, r->P, r->ts, turn, r->rwhist,
+                         r->Ibunch, r->nfFill);
     const long long tot = (long long)r->rwg.h * r->rwg.N;
     hipLaunchKernelGGL(k_rwg_sum, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, r->stream, r->rwg, r->P, r->ts,
-                       r->pending);
-  } else if (rw_split) {
+                       turn, r->pending);
+  } else if (r->rw_split) {
     hipLaunchKernelGGL(k_rw_fresh, dim3(r->G), dim3(WG), 0, r->stream, r->P, r->bunch_ring, r->rwhist, r->sqrt_tt,
-                       r->Ibunch, r->nfFill, r->bucket, r->ts, r->rw_part, r->G, r->pending);
-  } else if (r->rw_total > 0)
-    hipLaunchKernelGGL(k_rw, dim3(r->G), dim3(RW_WG), 0, r->stream, r->P, r->bunch_ring, r->rwhist, r->sqrt_tt,
-                       r->Ibunch, r->nfFill, r->bucket, r->pending, r->ts, r->ring_done, r->bunch_Ib, r->nres == 0);
+                       r->Ibunch, r->nfFill, r->bucket, r->ts, turn, r->rw_part, r->G, r->pending);
+  } else if (r->rw_total > 0) {
+    hipLaunchKernelGGL(k_rw, dim3(r->G), dim3(RW_WG), 0, r->stream, r->P, r->bunch_ring, r->rwhist, r->rsqrt_tt,
+                       r->Ibunch, r->nfFill, r->bucket, r->pending, r->ts, turn);
+  }
   CK(hipGetLastError());
   if (E) CK(hipEventRecord(E[3], r->stream));
-  // k_rw's last block ends the turn itself
-  const int end = r->rwg_on || rw_split || r->rw_total == 0;
-  if ((end || r->nres > 0) && (rc = launch_ring_end(r, end, 0))) return rc;
+  if (r->end_each && (rc = launch_ring_end(r, 1, 0))) return rc;
   if (E) CK(hipEventRecord(E[4], r->stream));
   r->rev_host++;
   return MBT_OK;
 }
+
+// After the launches of a block of n turns.
+static int end_block(mbt_ring *r, long n) { return r->end_each ? MBT_OK : launch_ring_end(r, (int)n, 0); }
 
 // n turns from the current turn as one HIP graph.  The launches of a turn
 // depend on the turn number only through the monitor-turn variant of k_turn,
@@ -3263,7 +3386,8 @@ static int turn_graph(mbt_ring *r, long n, hipGraphExec_t *out)
   const long long rev_save = r->rev_host;
   CK(hipStreamBeginCapture(r->stream, hipStreamCaptureModeThreadLocal));
   int rc = MBT_OK;
-  for (long t = 0; t < n && rc == MBT_OK; t++) rc = enqueue_turn(r, NULL);
+  for (long t = 0; t < n && rc == MBT_OK; t++) rc = enqueue_turn(r, NULL, (int)t);
+  if (rc == MBT_OK) rc = end_block(r, n);
   r->rev_host = rev_save;
   hipGraph_t graph = nullptr;
   hipError_t e = hipStreamEndCapture(r->stream, &graph);
@@ -3327,7 +3451,8 @@ static int enqueue_block(mbt_ring *r, long n)
   int rc;
   if (!r->use_graphs) {
     for (long t = 0; t < n; t++)
-      if ((rc = enqueue_turn(r, NULL))) return rc;
+      if ((rc = enqueue_turn(r, NULL, (int)t))) return rc;
+    if ((rc = end_block(r, n))) return rc;
   } else {
     hipGraphExec_t exec;
     if ((rc = turn_graph(r, n, &exec))) return rc;
@@ -3391,7 +3516,8 @@ extern "C" int mbt_ring_track(mbt_ring *r, long nturns, double *stats, double *a
     const bool timed = r->timing != 0;
     if (timed) {
       for (long t = 0; t < n; t++)
-        if ((rc = enqueue_turn(r, r->evpool + 6 * t))) return rc;
+        if ((rc = enqueue_turn(r, r->evpool + 6 * t, (int)t))) return rc;
+      if ((rc = end_block(r, n))) return rc;
     } else if ((rc = enqueue_block(r, n))) {
       return rc;
     }
@@ -3430,13 +3556,13 @@ extern "C" int mbt_ring_final_stats(mbt_ring *r, double *stats)
   (void)hipGetLastError(); // launch checks below must not report an earlier call's error
   int rc;
   // apply the pending RW kick, then two exact passes for the statistics
-  if ((rc = launch_turn_pass(r, MODE_FINAL))) return rc;
+  if ((rc = launch_turn_pass(r, MODE_FINAL, 0))) return rc;
   CK(hipMemsetAsync(r->pending, 0, (size_t)r->G * 2 * sizeof(double), r->stream));
   CK(hipMemsetAsync(r->shift, 0, (size_t)r->G * 6 * sizeof(double), r->stream));
-  if ((rc = launch_turn_pass(r, MODE_STATS))) return rc;
-  if ((rc = launch_reduce(r, 0))) return rc;
-  if ((rc = launch_turn_pass(r, MODE_STATS))) return rc;
-  if ((rc = launch_reduce(r, 3))) return rc;
+  if ((rc = launch_turn_pass(r, MODE_STATS, 0))) return rc;
+  if ((rc = launch_reduce(r, 0, 0))) return rc;
+  if ((rc = launch_turn_pass(r, MODE_STATS, 0))) return rc;
+  if ((rc = launch_reduce(r, 3, 0))) return rc;
   CK(hipStreamSynchronize(r->stream));
   TurnState ts;
   CK(hipMemcpy(&ts, r->ts, sizeof ts, hipMemcpyDeviceToHost));
@@ -3620,7 +3746,7 @@ extern "C" int mbt_ring_autotune(mbt_ring *r, int *best_items, double *ms)
         if (rep == 1) CK(hipEventRecord(e0, r->stream));
         hipLaunchKernelGGL(k, dim3(r->nwg), dim3(WG), r->lds_turn[r->any_dip], r->stream, r->P, r->C, r->wg_first, r->wg_end,
                            r->wg_bunch, r->bunch_ring, r->bucket, r->bunch_first, r->shift, r->sfL, r->sfV, r->sfH,
-                           r->LR, r->Ibunch, r->pending, r->partial, r->Hs, r->ts, RwOld{});
+                           r->LR, r->Ibunch, r->pending, r->partial, r->Hs, r->ts, 0, RwOld{});
         CK(hipGetLastError());
       }
       CK(hipEventRecord(e1, r->stream));
