@@ -154,14 +154,14 @@ struct DevParams {
   double aV, bV, gV, aH, bH, gH, dispH, disppH;
   double CVH, CVV, CHH, CHV;
   double HC_k, m_wrf, m_phi;
-  double sigma_tau, Nsigma, dT;
+  double sigma_tau, Nsigma, dT, inv_sigma, inv_dT; // and 1 / sigma_tau, 1 / dT
   double gamma1[3], alpha1[3], beta1[3];
   double fNp;
   double rwconst[2][2]; // [plane HOR/VER][trigger off/on]
   // RF feedback (src/feedback_rf.c, src/input.c:1678-1690)
   int fb_len, fb_switch_off;
   long long fbh_off;
-  double vrf_design, phi0_design;
+  double vrf_sin, vrf_cos; // design voltage times sine and cosine of the design phase
 };
 
 enum {
@@ -177,18 +177,16 @@ struct TurnState {
   long long fb_count;
 };
 
-// a mod d for a >= 0 (turn counters fit 32 bits in any run of a lifetime; a 64-bit
-// remainder is some hundred instructions)
-__device__ __forceinline__ unsigned umod(long long a, unsigned d)
+// a mod d for a >= 0, d > 0, inline for what fits 32 bits (any turn counter of a
+// lifetime; a 64-bit remainder is some two hundred instructions)
+__device__ __noinline__ unsigned long long rem64(unsigned long long a, unsigned long long d) { return a % d; }
+__device__ __forceinline__ long long umod(long long a, long long d)
 {
-  return (unsigned long long)a >> 32 ? (unsigned)((unsigned long long)a % d) : (unsigned)a % d;
+  return (a | d) >> 32 ? (long long)rem64(a, d) : (long long)((unsigned)a % (unsigned)d);
 }
 
 // The resistive wall's trigger counts turns since the last scan step.
-__device__ __forceinline__ int rw_trigger(long long rev, long long NrevScan)
-{
-  return (NrevScan >> 32 ? rev % NrevScan : (long long)umod(rev, (unsigned)NrevScan)) < 50 ? 1 : 0;
-}
+__device__ __forceinline__ int rw_trigger(long long rev, long long NrevScan) { return umod(rev, NrevScan) < 50 ? 1 : 0; }
 
 struct LRConst {
   int ring, plane, l, fb;
@@ -397,6 +395,21 @@ struct HistPtr {
   unsigned long long *tsx;  // [Nb*2*2]
   unsigned long long *tsz;  // [Nb*2*2]
   int *bad;                 // [Nb]
+};
+
+// What a work-group of the turn pass and a block of the reduction read first, one
+// load each (an index array per field makes a chain of loads of them, each a
+// microsecond after a pass over all memory).
+struct WgInfo {
+  long long j0;     // first slot
+  int cnt, b;       // macroparticles, bunch
+  int ring, kb;     // its ring and bucket
+  unsigned jloc;    // first macroparticle's place in the bunch
+  int pad;
+};
+struct BunchInfo {
+  int ring, kb, w0, w1; // ring, bucket, work-groups [w0, w1) of the turn pass
+  int np, pad[3];
 };
 
 struct Coords {
@@ -724,10 +737,8 @@ __device__ __noinline__ int turn_particle_exact(const DevParams *P, const MapArg
 
 template <int MODE, bool QE, bool DIP, bool GEN, bool MON>
 __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams *__restrict__ Pr, Coords C,
-                                                                const long long *wg_first, const long long *wg_end,
-                                                                const int *wg_bunch, const int *bunch_ring,
-                                                                const int *bucket, const long long *bunch_first,
-                                                                const double *shift, const double *sfL,
+                                                                const WgInfo *__restrict__ wgs, int nrings,
+                                                                const int *bucket, const double *shift, const double *sfL,
                                                                 const double *sfV, const double *sfH,
                                                                 LRDev LR, const double *Ibunch,
                                                                 const double *pending, double *partial, HistPtr H,
@@ -741,8 +752,8 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
     return;
   }
   const int wg = xcd_remap(blockIdx.x - RO.nlead, gridDim.x - RO.nlead);
-  const int b = wg_bunch[wg];
-  const int ring = bunch_ring[b];
+  const WgInfo I = wgs[wg];
+  const int b = I.b, kb = I.kb, ring = nrings == 1 ? 0 : I.ring;
   const DevParams &P = Pr[ring];
   const TurnState *ts = tsr + ring;
   const int Nc = P.Nc;
@@ -758,14 +769,24 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
   __shared__ double red[WG / 64][NMOM];
   __shared__ int lbad;
 
-  const int kb = bucket[b];
-  const long long j0 = wg_first[wg], j1 = wg_end[wg];
+  const long long j0 = I.j0;
   const int tid = threadIdx.x;
   const long long rev = ts->rev + turn;
   const bool do_hist = Nc > 0 && MODE != MODE_FINAL;
   const bool lr = P.lrp[3] > P.lrp[0];
   const double Ikb = lr ? Ibunch[P.bucket_off + kb] : 0.0;
 
+  // everything uniform is fetched before the barrier, beside the tables
+  double sh[6];
+#pragma unroll
+  for (int c = 0; c < 6; c++) sh[c] = shift[b * 6 + c];
+  const bool rw_h = MODE != MODE_STATS && P.rw && P.track_h;
+  const bool rw_v = MODE != MODE_STATS && P.rw && P.track_v;
+  const double rwx = rw_h ? pending[2 * b] : 0.0;
+  const double rwz = rw_v ? pending[2 * b + 1] : 0.0;
+  const double eps_const = ts->Vrf0 / P.E0k;
+  const double phai0 = ts->phai0;
+  const BinK bk = {P.sigma_tau, P.inv_sigma, P.Nsigma, P.dT, P.inv_dT};
   if (DIP)
     for (int i = tid; i < 2 * FX_LIMBS * Nt; i += WG) lsx[i] = 0;
   for (int i = tid; i < Nt; i += WG) lcnt[i] = 0;
@@ -786,16 +807,6 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
   if (tid == 0) lbad = 0;
   __syncthreads();
 
-  const BinK bk = {P.sigma_tau, 1.0 / P.sigma_tau, P.Nsigma, P.dT, 1.0 / P.dT};
-  double sh[6];
-#pragma unroll
-  for (int c = 0; c < 6; c++) sh[c] = shift[b * 6 + c];
-  const bool rw_h = MODE != MODE_STATS && P.rw && P.track_h;
-  const bool rw_v = MODE != MODE_STATS && P.rw && P.track_v;
-  const double rwx = rw_h ? pending[2 * b] : 0.0;
-  const double rwz = rw_v ? pending[2 * b + 1] : 0.0;
-  const double eps_const = ts->Vrf0 / P.E0k;
-  const double phai0 = ts->phai0;
   const bool qe = QE && P.qe;
 
   double s1[6] = {0, 0, 0, 0, 0, 0}, s2[6] = {0, 0, 0, 0, 0, 0}, am[3] = {0, 0, 0};
@@ -808,11 +819,14 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
   double *__restrict__ pxp = px + TILE;
   double *__restrict__ pz = pxp + TILE;
   double *__restrict__ pzp = pz + TILE;
-  const unsigned cnt = (unsigned)(j1 - j0), o0 = (unsigned)(j0 & (TILE - 1));
-  const unsigned jloc0 = (unsigned)(j0 - bunch_first[b]);
+  const unsigned cnt = (unsigned)I.cnt, o0 = (unsigned)(j0 & (TILE - 1)), jloc0 = I.jloc;
 
   constexpr bool MAP = MODE == MODE_TURN || MODE == MODE_TUNE;
   constexpr int HOW = MAP && (QE || GEN || DIP) ? FAST : BOTH;
+  // the call-free loop is short of scalar registers (its constants spill to vector
+  // lanes, a read back each) and has vector ones to spare
+  if (HOW == FAST && !GEN)
+    for (int c = 0; c < 6; c++) asm("" : "+v"(sh[c]));
   __shared__ MapArgs margs; // for the calls of the exact forms
   const MapArgs A = {bk, kL, kV, kH, eps_const, phai0, rwx, rwz, P.flags, Nc, kb, rw_h, rw_v, qe, do_hist, rev};
   if (HOW == FAST) {
@@ -1005,49 +1019,55 @@ struct RedOut {
 // sums of every sixteenth term from k = i down, then a fixed tree over them; a
 // lane has 16 / Q of the sums.  mixed: the terms in compensated FP32.  A whole
 // group of terms is read before the first is added.
-template <int Q> __device__ __forceinline__ double conv_at(const double *src, const double *g, int i, int q, int mixed)
+template <int Q, bool mixed> __device__ __forceinline__ double conv_at(const double *src, const double *g, int i, int q)
 {
   constexpr int A = 16 / Q, C = A > 8 ? A : 8;
   double a[A];
-  if (mixed) {
-    F2 s[A];
+  F2 s[A];
 #pragma unroll
-    for (int t = 0; t < A; t++) s[t] = {0.0f, 0.0f};
-    for (int k0 = i - q; k0 >= 0; k0 -= A * Q) {
+  for (int t = 0; t < A; t++) {
+    a[t] = 0.0;
+    s[t] = {0.0f, 0.0f};
+  }
+  int k0 = i - q;
+  for (; k0 - (C - 1) * Q >= 0; k0 -= C * Q) {
+    double u[C], w[C];
 #pragma unroll
-      for (int t = 0; t < A; t++)
-        if (k0 - t * Q >= 0) f2_add_prod(s[t], src[k0 - t * Q], g[i - k0 + t * Q]);
+    for (int t = 0; t < C; t++) {
+      u[t] = src[k0 - t * Q];
+      w[t] = g[i - k0 + t * Q];
     }
+    if (mixed) {
 #pragma unroll
-    for (int t = 0; t < A; t++) a[t] = (double)s[t].hi + (double)s[t].lo;
-  } else {
-#pragma unroll
-    for (int t = 0; t < A; t++) a[t] = 0.0;
-    int k0 = i - q;
-    for (; k0 - (C - 1) * Q >= 0; k0 -= C * Q) {
-      double u[C], w[C];
-#pragma unroll
-      for (int t = 0; t < C; t++) {
-        u[t] = src[k0 - t * Q];
-        w[t] = g[i - k0 + t * Q];
-      }
+      for (int t = 0; t < C; t++) f2_add_prod(s[t % A], u[t], w[t]);
+    } else {
 #pragma unroll
       for (int t = 0; t < C; t++) a[t % A] = fma(u[t], w[t], a[t % A]);
     }
-    if (k0 >= 0) {
-      double u[C], w[C];
+  }
+  if (k0 >= 0) {
+    double u[C], w[C];
 #pragma unroll
-      for (int t = 0; t < C; t++) {
-        const int k = max(k0 - t * Q, 0);
-        u[t] = src[k];
-        w[t] = g[i - k];
-      }
+    for (int t = 0; t < C; t++) {
+      const int k = max(k0 - t * Q, 0);
+      u[t] = src[k];
+      w[t] = g[i - k];
+    }
+    if (mixed) {
+#pragma unroll
+      for (int t = 0; t < C; t++)
+        if (k0 - t * Q >= 0) f2_add_prod(s[t % A], u[t], w[t]);
+    } else {
 #pragma unroll
       for (int t = 0; t < C; t++) {
         const double v = fma(u[t], w[t], a[t % A]);
         a[t % A] = k0 - t * Q >= 0 ? v : a[t % A];
       }
     }
+  }
+  if (mixed) {
+#pragma unroll
+    for (int t = 0; t < A; t++) a[t] = (double)s[t].hi + (double)s[t].lo;
   }
   // sum r of the sixteen is lane r % Q's a[r / Q]: partners r ^ 8, r ^ 4, r ^ 2, r ^ 1
 #pragma unroll
@@ -1067,14 +1087,13 @@ template <int Q> __device__ __forceinline__ double conv_at(const double *src, co
 // statistics (wave 3) run beside the histogram (waves 0 ..), and the convolutions
 // take two slices i and Nc - 1 - i per group of Q lanes, so that every lane has the
 // same (Nc + 1) / Q terms and only the planes that have a wake are visited.  One
-// bunch x 100 slices x 3 planes 16.1 -> 9.1 us, 64 x 50 slices 10.0 -> 5.9, 416 x
-// 100 18.6 -> 10.2, 333 x 50 with three LR resonators 26.7 -> 10.1 (one lane per slice
+// bunch x 100 slices x 3 planes 16.1 -> 7.7 us, 64 x 50 slices 10.0 -> 5.6, 416 x
+// 100 18.6 -> 10.1, 333 x 50 with three LR resonators 26.7 -> 9.8 (one lane per slice
 // and plane, loads waited for one by one, the statistics and 64-bit remainders in
 // front of the rest).
-template <int NT, int Q>
+template <int NT, int Q, bool MIXED>
 __global__ __launch_bounds__(NT) void k_reduce(const DevParams *__restrict__ Pr, const double *__restrict__ partial,
-                                               const int *__restrict__ bunch_wg0, const int *__restrict__ bunch_ring,
-                                               const int *__restrict__ bucket, HistPtr H, RedOut R,
+                                               const BunchInfo *__restrict__ bunches, int nrings, HistPtr H, RedOut R,
                                                const TurnState *__restrict__ tsr, int phase, int dip, LRDev LR,
                                                int lr_lds, int turn, int Nc)
 {
@@ -1084,8 +1103,8 @@ __global__ __launch_bounds__(NT) void k_reduce(const DevParams *__restrict__ Pr,
   __shared__ double mom[NMOM];
   __shared__ int icmin_s, icmax_s;
   const int b = blockIdx.x, tid = threadIdx.x;
-  const int ring = bunch_ring[b], kb = bucket[b], np = R.np[b];
-  const int w0 = bunch_wg0[b], w1 = bunch_wg0[b + 1];
+  const BunchInfo I = bunches[b];
+  const int ring = nrings == 1 ? 0 : I.ring, kb = I.kb, np = I.np, w0 = I.w0, w1 = I.w1;
   const bool hist = phase != 0 && Nc > 0;
   // the bunch's own inputs: histogram (the first NT slices), trash, shift, current
   unsigned int cnt0 = 0, tc[2] = {0, 0};
@@ -1110,7 +1129,7 @@ __global__ __launch_bounds__(NT) void k_reduce(const DevParams *__restrict__ Pr,
       tot = R.trash_tot[2 * b + tid];
     }
   }
-  if (tid >= 192 && tid < 198) shift = R.shift[b * 6 + tid - 192];
+  if (tid >= NT - 64 && tid < NT - 58) shift = R.shift[b * 6 + tid - (NT - 64)];
   {
     const unsigned long long *src = (const unsigned long long *)(Pr + ring);
     unsigned long long *dst = (unsigned long long *)&P;
@@ -1125,6 +1144,7 @@ __global__ __launch_bounds__(NT) void k_reduce(const DevParams *__restrict__ Pr,
   // with LR resonators: their own wakes, [plane][Nc], in LDS where it holds them,
   // and the edge slices' sums without the particles beyond them
   const double *Gl = lr_lds ? Gs + 3 * Nc : LR.G + (size_t)ring * 3 * Nc;
+  double *raw = lr_lds ? Gs + 6 * Nc : fnp; // histograms without the particles beyond the edges
   {
     // moment sums over the bunch's workgroups: 16 lanes per moment, each summing
     // every 16th workgroup in order, then a fixed butterfly over the 16 lanes
@@ -1152,43 +1172,47 @@ __global__ __launch_bounds__(NT) void k_reduce(const DevParams *__restrict__ Pr,
   const int slot = (int)(rev & (STATS_TURNS - 1));
   // the final statistics leave the wakes of the next turn alone
   const bool lrp = (phase == 1 || phase == 2) && P.lrp[3] > P.lrp[0];
-  if (tid >= 192 && tid < 198) {
-    // one lane per coordinate (tau, delta, x, x', z, z')
-    const int k = tid - 192, pl = k >> 1, c = k & 1;
-    const double Np = (double)np;
-    const bool track = pl == 0 || (pl == 1 ? P.track_h : P.track_v);
-    const double mp = mom[k] / Np, v = mom[6 + k] / Np - mp * mp;
-    const double mean = track ? shift + mp : 0.0;
-    R.shift[b * 6 + k] = mean;
-    if (phase != 0) {
-      double *o = R.stats + ((size_t)slot * R.Gtot + b) * 12 + 6 * c + pl;
-      o[0] = mean;
-      o[3] = track ? sqrt(v > 0.0 ? v : 0.0) : 0.0;
-      if (phase == 2 && umod(rev + 1, (unsigned)P.monitor_every) == 0) {
-        const double other = __shfl_xor(mean, 1, 2), pos = c ? other : mean, slope = c ? mean : other;
-        double *a = R.amp + ((size_t)slot * R.Gtot + b) * 6 + 3 * c + pl;
-        *a = !track ? 0.0
-                    : (c == 0 ? mom[12 + pl] / Np
-                              : P.gamma1[pl] * (pos * pos) + 2.0 * P.alpha1[pl] * pos * slope +
-                                    P.beta1[pl] * (slope * slope));
-      }
-      if (P.rw && phase != 3 && c == 0 && pl > 0) {
-        // the turn's row of the cyclic history (rows go backwards), at the start
-        // also the rows of the Nmlt - 1 turns before
-        double *row = R.rwhist + P.rw_off + 2 * kb + pl - 1;
-        const int rows = P.Nmlt + 2, r0 = phase == 1 ? 0 : (int)((rows - umod(rev, rows)) % rows);
-        row[2LL * r0 * P.h] = mean;
-        if (phase == 1)
-          for (int jj = 1; jj < P.Nmlt; jj++) row[2LL * jj * P.h] = mean;
+  // the statistics, by the last wave
+  const auto statistics = [&]() {
+  if (tid >= NT - 64 && tid < NT - 58) {
+      // one lane per coordinate (tau, delta, x, x', z, z')
+      const int k = tid - (NT - 64), pl = k >> 1, c = k & 1;
+      const double Np = (double)np;
+      const bool track = pl == 0 || (pl == 1 ? P.track_h : P.track_v);
+      const double mp = mom[k] / Np, v = mom[6 + k] / Np - mp * mp;
+      const double mean = track ? shift + mp : 0.0;
+      R.shift[b * 6 + k] = mean;
+      if (phase != 0) {
+        double *o = R.stats + ((size_t)slot * R.Gtot + b) * 12 + 6 * c + pl;
+        o[0] = mean;
+        o[3] = track ? sqrt(v > 0.0 ? v : 0.0) : 0.0;
+        if (phase == 2 && umod(rev + 1, P.monitor_every) == 0) {
+          const double other = __shfl_xor(mean, 1, 2), pos = c ? other : mean, slope = c ? mean : other;
+          double *a = R.amp + ((size_t)slot * R.Gtot + b) * 6 + 3 * c + pl;
+          *a = !track ? 0.0
+                      : (c == 0 ? mom[12 + pl] / Np
+                                : P.gamma1[pl] * (pos * pos) + 2.0 * P.alpha1[pl] * pos * slope +
+                                      P.beta1[pl] * (slope * slope));
+        }
+        if (P.rw && phase != 3 && c == 0 && pl > 0) {
+          // the turn's row of the cyclic history (rows go backwards), at the start
+          // also the rows of the Nmlt - 1 turns before
+          double *row = R.rwhist + P.rw_off + 2 * kb + pl - 1;
+          const int rows = P.Nmlt + 2, r0 = phase == 1 ? 0 : (int)((rows - umod(rev, rows)) % rows);
+          row[2LL * r0 * P.h] = mean;
+          if (phase == 1)
+            for (int jj = 1; jj < P.Nmlt; jj++) row[2LL * jj * P.h] = mean;
+        }
       }
     }
-  }
-  if (phase == 2 && b == P.bunch_off && tid == 255) {
-    // nothing changes phai0 / Vrf0 between the map and this point of the turn
-    R.rfbuf[((size_t)slot * R.R + ring) * 2] = ts->phai0;
-    R.rfbuf[((size_t)slot * R.R + ring) * 2 + 1] = ts->Vrf0;
-  }
+    if (phase == 2 && b == P.bunch_off && tid == NT - 1) {
+      // nothing changes phai0 / Vrf0 between the map and this point of the turn
+      R.rfbuf[((size_t)slot * R.R + ring) * 2] = ts->phai0;
+      R.rfbuf[((size_t)slot * R.R + ring) * 2 + 1] = ts->Vrf0;
+    }
+  };
   if (!hist) {
+    statistics();
     // consume (and clear) the histogram only on the stats passes
     if (Nc > 0) {
       for (int i = tid; i < Nc; i += NT) {
@@ -1215,6 +1239,7 @@ __global__ __launch_bounds__(NT) void k_reduce(const DevParams *__restrict__ Pr,
     const size_t g = (size_t)b * Nc + i;
     unsigned int c = cnt0;
     unsigned long long xl = xl0, xh = xh0, zl = zl0, zh = zh0;
+    double edge_n = 0.0, edge_x = 0.0, edge_z = 0.0;
     if (i >= NT) {
       c = H.cnt[g];
       if (dip) {
@@ -1227,12 +1252,14 @@ __global__ __launch_bounds__(NT) void k_reduce(const DevParams *__restrict__ Pr,
     if (i == 0 || i == Nc - 1) {
       // dropped: the sums of the edge slices alone; clamped: out-of-range
       // particles join them (one slice takes both edges)
-      const double n = (double)c, ex = bad ? NAN : fx_to_double(xl, xh), ez = bad ? NAN : fx_to_double(zl, zh);
+      edge_n = (double)c;
+      edge_x = bad ? NAN : fx_to_double(xl, xh);
+      edge_z = bad ? NAN : fx_to_double(zl, zh);
       for (int e = 0; e < 2; e++) {
         if (i != (e ? Nc - 1 : 0)) continue;
-        edge[0][e] = n;
-        edge[1][e] = ex;
-        edge[2][e] = ez;
+        edge[0][e] = edge_n;
+        edge[1][e] = edge_x;
+        edge[2][e] = edge_z;
         c += tc[e];
         if (!dip) continue;
         fx_add(xl, xh, H.tsx[4 * b + 2 * e], H.tsx[4 * b + 2 * e + 1]);
@@ -1251,9 +1278,20 @@ __global__ __launch_bounds__(NT) void k_reduce(const DevParams *__restrict__ Pr,
     fnp[i] = n;
     dV[i] = sz;
     dH[i] = sx;
-    R.fnp_out[g] = n;
-    R.dipV_out[g] = sz;
-    R.dipH_out[g] = sx;
+    if (raw != fnp) {
+      raw[i] = i == 0 ? edge_n : (i == Nc - 1 ? edge_n : n);
+      raw[Nc + i] = i == 0 || i == Nc - 1 ? edge_x : sx;
+      raw[2 * Nc + i] = i == 0 || i == Nc - 1 ? edge_z : sz;
+    }
+  }
+  __syncthreads();
+  // from here on only stores leave the block (a barrier would wait for them)
+  statistics();
+  for (int i = tid; i < Nc; i += NT) {
+    const size_t g = (size_t)b * Nc + i;
+    R.fnp_out[g] = fnp[i];
+    R.dipV_out[g] = dV[i];
+    R.dipH_out[g] = dH[i];
     // clear the accumulators for the next pass
     H.cnt[g] = 0;
     if (dip) {
@@ -1265,9 +1303,6 @@ __global__ __launch_bounds__(NT) void k_reduce(const DevParams *__restrict__ Pr,
     // trash counters: the previous pending binning is consumed by this turn's kick
     if (phase == 2) R.trash_tot[2 * b + tid] = tot + pend;
     R.trash_pend[2 * b + tid] = (int)tc[tid];
-  }
-  __syncthreads();
-  if (tid < 2) {
     H.tcnt[2 * b + tid] = 0;
     if (dip) {
       H.tsx[4 * b + 2 * tid] = H.tsx[4 * b + 2 * tid + 1] = 0;
@@ -1277,59 +1312,61 @@ __global__ __launch_bounds__(NT) void k_reduce(const DevParams *__restrict__ Pr,
   if (tid == 0) H.bad[b] = 0;
   const int icmin = icmin_s, icmax = icmax_s;
   // the next turn's kick uses the current after this turn's scan step (src/tracking.c:43-59)
-  if (phase == 2 && P.scan == 1 && (rev + 1) % P.NrevScan == 0) Ib += P.scan_step / (((double)P.Nb) * 1.0e3);
+  if (phase == 2 && P.scan == 1 && umod(rev + 1, P.NrevScan) == 0) Ib += P.scan_step / (((double)P.Nb) * 1.0e3);
   const double factG = -P.T0 * Ib / (np * P.E0 * 1.0e9);
   const double sgm = P.sigma_tau, sgm2 = sgm * sgm, dT2 = P.dT * P.dT;
   const int np2 = (Nc + 1) >> 1; // pairs of slices (i, Nc - 1 - i)
   const int q = tid & (Q - 1);
-  for (int t = tid / Q; t < np2; t += NT / Q)
-    for (int half = 0; half < 2; half++) {
-      const int i = half ? t : Nc - 1 - t;
-      if (half && i == Nc - 1 - t) break; // the middle slice of an odd count
-      const size_t g = (size_t)b * Nc + i;
-      double val = 0.0;
-      if (P.convL && i >= icmin) {
-        // slices below icmin are empty: nothing to add from them
-        double GL1 = conv_at<Q>(fnp, Gs, i, q, P.mixed);
-        // resistive and inductive smoothing, src/transform_weak.c:670-683; reads
-        // outside [0, Ncell) count as zero
+  const double Rsis = P.RsisL, aind = P.aindL;
+#pragma unroll 1
+  for (int pl = 0; pl < 3; pl++) {
+    // LON, VER, HOR.  A plane without a kick keeps the +0.0 of its allocation (its
+    // value here, -factG * 0 with factG <= 0), so its table is not rewritten
+    const bool on = pl == 0 ? P.convL != 0 : (pl == 1 ? P.kickV != 0 : P.kickH != 0);
+    if (!on && pl > 0) continue;
+    const double *src = sm + pl * Nc, *g = Gs + pl * Nc;
+    double *out = (pl == 0 ? R.sfL : (pl == 1 ? R.sfV : R.sfH)) + (size_t)b * Nc;
+    const double scale = pl == 0 ? factG : -factG;
+    const int ilo = pl == 0 ? icmin : (pl == 2 ? 1 : 0); // slices below icmin are empty, HOR starts at slice 1
+    for (int t = tid / Q; t < np2; t += NT / Q)
+      for (int half = 0; half < 2; half++) {
+        const int i = half ? t : Nc - 1 - t;
+        if (half && i == Nc - 1 - t) break; // the middle slice of an odd count
+        double v = on && i >= ilo ? conv_at<Q, MIXED>(src, g, i, q) : 0.0;
+        if (pl == 0 && on && i >= icmin + 1 && i <= icmax) {
+          // resistive and inductive smoothing, src/transform_weak.c:670-683; reads
+          // outside [0, Ncell) count as zero
 #define F(k) (((k) >= 0 && (k) < Nc) ? fnp[k] : 0.0)
-        if (P.RsisL > 0 && i >= icmin + 1 && i <= icmax) {
-          double nt = (0.5 * F(i - 1) + F(i) + 0.5 * F(i + 1)) / 2.0;
-          GL1 += P.RsisL * nt / (sgm * P.dT);
-        }
-        if (P.aindL > 0 && i >= icmin + 1 && i <= icmax) {
-          double n0 = (0.25 * F(i - 3) + 0.5 * F(i - 2) + F(i - 1) + 0.5 * F(i) + 0.25 * F(i + 1)) / 2.5;
-          double n1 = (0.25 * F(i - 1) + 0.5 * F(i) + F(i + 1) + 0.5 * F(i + 2) + 0.25 * F(i + 3)) / 2.5;
-          GL1 += (n1 - n0) / (2.0 * sgm2 * dT2) * P.aindL;
-        }
+          if (Rsis > 0) {
+            double nt = (0.5 * F(i - 1) + F(i) + 0.5 * F(i + 1)) / 2.0;
+            v += Rsis * nt / (sgm * P.dT);
+          }
+          if (aind > 0) {
+            double n0 = (0.25 * F(i - 3) + 0.5 * F(i - 2) + F(i - 1) + 0.5 * F(i) + 0.25 * F(i + 1)) / 2.5;
+            double n1 = (0.25 * F(i - 1) + 0.5 * F(i) + F(i + 1) + 0.5 * F(i + 2) + 0.25 * F(i + 3)) / 2.5;
+            v += (n1 - n0) / (2.0 * sgm2 * dT2) * aind;
+          }
 #undef F
-        val = GL1;
+        }
+        if (q == 0) out[i] = scale * v;
       }
-      if (q == 0) R.sfL[g] = factG * val;
-      // a plane without a kick keeps the +0.0 of its allocation (its value
-      // here, -factG * 0 with factG <= 0), so its table is not rewritten
-      if (P.kickV) {
-        const double v = conv_at<Q>(dV, Gs + Nc, i, q, P.mixed);
-        if (q == 0) R.sfV[g] = -factG * v;
-      }
-      if (P.kickH) {
-        const double v = i >= 1 ? conv_at<Q>(dH, Gs + 2 * Nc, i, q, P.mixed) : 0.0;
-        if (q == 0) R.sfH[g] = -factG * v;
-      }
-    }
-  if (!lrp) return;
-  // ---- LR resonators: the histograms without the particles beyond the edges
-  __syncthreads();
-  if (tid < 6) {
-    const int pl = tid >> 1, e = tid & 1;
-    (pl == 0 ? fnp : (pl == 1 ? dH : dV))[e ? Nc - 1 : 0] = edge[pl][e];
   }
-  __syncthreads();
+  if (!lrp) return;
+  // ---- LR resonators: the histograms without the particles beyond the edges,
+  // from their own copy (LON, HOR, VER) or, where LDS has no room for it, in place
+  if (raw == fnp) {
+    __syncthreads();
+    if (tid < 6) {
+      const int pl = tid >> 1, e = tid & 1;
+      (pl == 0 ? fnp : (pl == 1 ? dH : dV))[e ? Nc - 1 : 0] = edge[pl][e];
+    }
+    __syncthreads();
+  }
+  const double *f0 = raw, *f1 = raw == fnp ? dH : raw + Nc, *f2 = raw == fnp ? dV : raw + 2 * Nc;
   // slice sums the phasor recurrence needs, one wave per resonator
   const int nr = P.lrp[3] - P.lrp[0];
   for (int r = P.lrp[0] + (tid >> 6); r < P.lrp[3]; r += NT / 64) {
-    const double *f = r < P.lrp[1] ? fnp : (r < P.lrp[2] ? dH : dV);
+    const double *f = r < P.lrp[1] ? f0 : (r < P.lrp[2] ? f1 : f2);
     const double2 *p = LR.pw + (size_t)r * (Nc + 1);
     double sr = 0.0, si = 0.0;
     for (int j = tid & 63; j < Nc; j += 64) {
@@ -1347,9 +1384,10 @@ __global__ __launch_bounds__(NT) void k_reduce(const DevParams *__restrict__ Pr,
     for (int half = 0; half < 2; half++) {
       const int i = half ? t : Nc - 1 - t;
       if (half && i == Nc - 1 - t) break;
+#pragma unroll 1
       for (int pl = 0; pl < 3; pl++) {
         if (P.lrp[pl] == P.lrp[pl + 1]) continue;
-        const double a = conv_at<Q>(pl == 0 ? fnp : (pl == 1 ? dH : dV), Gl + pl * Nc, i, q, 0);
+        const double a = conv_at<Q, false>(pl == 0 ? f0 : (pl == 1 ? f1 : f2), Gl + pl * Nc, i, q);
         if (q == 0) LR.self[((size_t)pl * LR.Gtot + b) * Nc + i] = a;
       }
     }
@@ -1424,7 +1462,7 @@ __device__ void rw_taps(const DevParams &P, int kb, long long rev, const double 
 __device__ void end_turns(const DevParams &P, TurnState *ts, double *bunch_Ib, double *Ibunch, const int *nfFill, int n)
 {
   const long long rev = ts->rev;
-  if (P.scan == 1 && (rev + 1) % P.NrevScan == 0) {
+  if (P.scan == 1 && umod(rev + 1, P.NrevScan) == 0) {
     ts->Iring += P.scan_step;
     ts->scan_val = ts->Iring;
     for (int k = 0; k < P.Nb; k++) bunch_Ib[P.bunch_off + k] += P.scan_step / (((double)P.Nb) * 1.0e3);
@@ -1443,8 +1481,10 @@ __device__ void fb_apply(const DevParams &P, TurnState *ts, double vs, double ps
   const int fb_len = P.fb_len;
   double vmbar = vs / fb_len, phibar = ps / fb_len;
   vmbar = vmbar * P.E0 * 1.0e3;
-  double num = P.vrf_design * sin(P.phi0_design) - vmbar * sin(phibar);
-  double ph = atan2(num, P.vrf_design * cos(P.phi0_design) - vmbar * cos(phibar));
+  double sn, cs;
+  sincos(phibar, &sn, &cs);
+  double num = P.vrf_sin - vmbar * sn;
+  double ph = atan2(num, P.vrf_cos - vmbar * cs);
   ts->phai0 = ph;
   ts->Vrf0 = num / sin(ph);
   if (init && P.fb_switch_off) ts->has_fb = 0;
@@ -1554,17 +1594,14 @@ __global__ __launch_bounds__(RW_WG) void k_rw(const DevParams *__restrict__ Pr, 
       j++;
     }
   }
-  ax = wave_sum(ax);
-  az = wave_sum(az);
-  if ((tid & 63) == 0) {
-    red[tid >> 6][0] = ax;
-    red[tid >> 6][1] = az;
-  }
+  const double a = wsum64x2(ax, az);
+  if ((tid & 31) == 0) red[tid >> 6][tid >> 5 & 1] = a;
+  const int trig = rw_trigger(rev, P.NrevScan);
   __syncthreads();
   if (tid < 2) {
     double s = 0.0;
+#pragma unroll
     for (int w = 0; w < RW_WG / 64; w++) s += red[w][tid];
-    const int trig = rw_trigger(rev, P.NrevScan);
     pending[2 * b + tid] = (tid ? P.track_v : P.track_h) ? s * P.rwconst[tid][trig] : 0.0;
   }
 }
@@ -1706,21 +1743,29 @@ __global__ __launch_bounds__(256) void k_rwg_tile(RWGemm Gm, const DevParams *__
     }
   }
   __syncthreads();
-  const int q0 = A0 % h;
-  for (int e = tid; e < nA * 16; e += 256) {
-    const int t = e >> 4, jl = e & 15, ring = yring[jl];
-    const int a = A0 + t;
-    double v = 0.0;
-    if (ring >= 0 && a >= 1 && a < h + M) {
-      int q = q0 + t; // bucket a mod h (q0 < h, t < 4 per)
-      while (q >= h) q -= h;
-      if (nfFill[yboff[jl] + q]) {
-        long long idx = ybase[jl] + t;
-        if (idx >= Gm.n) idx %= Gm.n; // t < 4 per may exceed n when h is small
-        v = rwhist[yroff[jl] + 2 * idx + (jl & 1)] * Ibunch[yboff[jl] + q];
-      }
+  // (a thread keeps its column; every load is in range whatever the row, so that
+  // the four rows of an unrolled step are under way together: 16 rings, a
+  // block per CU, 37.5 -> 33.6 us)
+  {
+    const int jl = tid & 15, ring = yring[jl], q0 = A0 % h;
+    const double *hist = rwhist + (ring >= 0 ? yroff[jl] : 0) + (jl & 1);
+    const int *fill = nfFill + (ring >= 0 ? yboff[jl] : 0);
+    const double *Ib = Ibunch + (ring >= 0 ? yboff[jl] : 0);
+    const int base = ring >= 0 ? (int)ybase[jl] : 0, n = Gm.n;
+    int q = (q0 + (tid >> 4)) % h, idx = (base + (tid >> 4)) % n; // bucket and history slot of the row
+    const int dq = 16 % h, di = 16 % n;
+#pragma unroll 4
+    for (int t = tid >> 4; t < nA; t += 16) {
+      const int a = A0 + t;
+      const bool on = ring >= 0 && a >= 1 && a < h + M;
+      const double y = hist[2 * idx], I = Ib[q];
+      const int f = fill[q];
+      Yf[16 * t + jl] = on && f ? y * I : 0.0;
+      q += dq;
+      if (q >= h) q -= h;
+      idx += di;
+      if (idx >= n) idx -= n;
     }
-    Yf[e] = v;
   }
   const int mlo = A0 - HP + 1;
   for (int e = tid; e < nA + HP - 1; e += 256) {
@@ -1750,20 +1795,28 @@ __global__ __launch_bounds__(256) void k_rwg_tile(RWGemm Gm, const DevParams *__
   }
 }
 
-// one lane per (bucket, column): the K slices summed in a fixed order, then the
-// pending kick of the bucket's bunch (the ring's fNp and RW constant applied)
+// One block per (bucket, 16 columns): sixteen groups of lanes add every sixteenth K
+// slice, then the groups' sums in order, and the pending kick of the bucket's bunch
+// (the ring's fNp and RW constant applied).  One lane per bucket and column, adding
+// all slices, had too few loads in flight for few rings: 111 slices, 416 buckets, 16
+// rings 29.6 -> 5.8 us.
 __global__ __launch_bounds__(256) void k_rwg_sum(RWGemm Gm, const DevParams *__restrict__ Pr,
                                                const TurnState *__restrict__ tsr, int turn, double *pending)
 {
-  const long long e = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (long long)Gm.h * Gm.N) return;
-  const int kb = (int)(e / Gm.N), col = (int)(e % Gm.N);
+  __shared__ double red[16][17];
+  const int kb = blockIdx.y, col = blockIdx.x * 16 + (threadIdx.x & 15), part = threadIdx.x >> 4;
+  double sum = 0.0;
+  if (col < Gm.N)
+#pragma unroll 8
+    for (int ks = part; ks < Gm.KS; ks += 16) sum += Gm.part[((size_t)ks * Gm.HP + kb) * Gm.N + col];
+  red[part][threadIdx.x & 15] = sum;
+  __syncthreads();
+  if (part != 0 || col >= Gm.N) return;
   const int ring = Gm.col_ring[col >> 1], pl = col & 1;
   const DevParams &P = Pr[ring];
   const int g = Gm.bucket_bunch[P.bucket_off + kb];
   if (g < 0) return;
-  double sum = 0.0;
-  for (int ks = 0; ks < Gm.KS; ks++) sum += Gm.part[((size_t)ks * Gm.HP + kb) * Gm.N + col];
+  for (int k = 1; k < 16; k++) sum += red[k][threadIdx.x];
   const int trig = rw_trigger(tsr[ring].rev + turn, P.NrevScan);
   const bool on = pl == 0 ? P.track_h : P.track_v;
   pending[2 * g + pl] = on ? (P.fNp * sum) * P.rwconst[pl][trig] : 0.0;
@@ -1801,6 +1854,7 @@ __device__ __forceinline__ double2 shfl_up2(double2 v, int d)
 // 416 buckets x 50 slices, 3 resonators; the whole kernel now takes 12).
 // fbh: also take the feedback samples from number keep on (the first one is c0;
 // W: what the first reads).
+template <bool INIT>
 __device__ double2 lr_turn(const LRConst &L, const LRDev &R, const DevParams &P, int r, const double *Ib, const int *fill,
                            double2 V0, double2 W, double *fbh, int fb_len, long long c0, long long keep)
 {
@@ -1847,7 +1901,7 @@ __device__ double2 lr_turn(const LRConst &L, const LRDev &R, const DevParams &P,
         Vs[(m0 + k) * nr] = V;
         const double2 before = V, M = filled >> k & 1 ? mf : e;
         V = cadd(cmul(M, V), c[k]);
-        if (fbh) {
+        if (INIT && fbh) {
           const long long q = c0 + 2LL * (m0 + k);
           if (q >= keep) fb_sample(fbh, fb_len, q, m0 + k == 0 ? W : before, L.pb0, L.pb1);
           if (q + 1 >= keep) fb_sample(fbh, fb_len, q + 1, V, L.pa0, L.pa1);
@@ -1863,8 +1917,9 @@ __device__ double2 lr_turn(const LRConst &L, const LRDev &R, const DevParams &P,
 // each), the RF-feedback samples and the RF-feedback solve.  init:
 // wake_phasor_init (src/transform_weak.c:869-952), the same turn replayed
 // init_turns times from a zero phasor, one wave in order taking the samples.
+template <bool INIT>
 __global__ __launch_bounds__(256) void k_ring_end(const DevParams *__restrict__ Pr, TurnState *tsr, double *bunch_Ib,
-                                                  double *Ibunch, const int *nfFill, LRDev R, int end, int init)
+                                                  double *Ibunch, const int *nfFill, LRDev R, int end)
 {
   const int ring = blockIdx.x, tid = threadIdx.x, lane = tid & 63, nw = blockDim.x >> 6;
   const DevParams &P = Pr[ring];
@@ -1872,7 +1927,7 @@ __global__ __launch_bounds__(256) void k_ring_end(const DevParams *__restrict__ 
   if (end && tid == 0) end_turns(P, ts, bunch_Ib, Ibunch, nfFill, end);
   const int lr0 = P.lrp[0], nr = P.lrp[3] - lr0;
   if (nr == 0) {
-    if (tid == 0) fb_solve(P, ts, R.fb_hist, init);
+    if (tid == 0) fb_solve(P, ts, R.fb_hist, INIT);
     return;
   }
   __syncthreads();
@@ -1886,15 +1941,15 @@ __global__ __launch_bounds__(256) void k_ring_end(const DevParams *__restrict__ 
   for (int r = lr0 + (tid >> 6); r < lr0 + nr; r += nw) {
     const LRConst &L = R.lc[r];
     const double2 last = R.V[P.lr_off + (long long)h * nr + r - lr0];
-    if (!init) {
-      lr_turn(L, R, P, r, Ib, fill, last, last, nullptr, fb_len, 0, 0);
+    if (!INIT) {
+      lr_turn<INIT>(L, R, P, r, Ib, fill, last, last, nullptr, fb_len, 0, 0);
       continue;
     }
     double2 V = make_double2(0.0, 0.0);
     const long long all = 2LL * h * L.init_turns, keep = cnt0 + all - fb_len;
     for (int k = 0; k < L.init_turns; k++) {
       const long long c0 = cnt0 + 2LL * h * k;
-      V = lr_turn(L, R, P, r, Ib, fill, V, k == 0 ? last : V, L.fb && has && c0 + 2LL * h > keep ? fbh : nullptr,
+      V = lr_turn<INIT>(L, R, P, r, Ib, fill, V, k == 0 ? last : V, L.fb && has && c0 + 2LL * h > keep ? fbh : nullptr,
                   fb_len, c0, keep);
     }
   }
@@ -1903,8 +1958,8 @@ __global__ __launch_bounds__(256) void k_ring_end(const DevParams *__restrict__ 
     for (int r = lr0; r < lr0 + nr; r++) {
       const LRConst &L = R.lc[r];
       if (!L.fb) continue;
-      cnt1 += 2LL * h * (init ? L.init_turns : 1);
-      if (init) continue;
+      cnt1 += 2LL * h * (INIT ? L.init_turns : 1);
+      if (INIT) continue;
       // of the 2 h samples only the last fb_len survive in the sample ring, so only
       // those are written (no two lanes share a slot)
       const double2 *V = R.V + P.lr_off + r - lr0;
@@ -1931,7 +1986,7 @@ __global__ __launch_bounds__(256) void k_ring_end(const DevParams *__restrict__ 
   }
   vs = wave_sum(vs);
   ps = wave_sum(ps);
-  if (lane == 0) fb_apply(P, ts, vs, ps, init);
+  if (lane == 0) fb_apply(P, ts, vs, ps, INIT);
 }
 
 // The long-range wake of one bunch's slices (longitudinal), as the next turn adds it.
@@ -1980,8 +2035,10 @@ struct mbt_ring {
   int min_items;     // smallest chunk the buffers allow (1 for small rings, else 4)
   int any_qe, any_dip, any_gen, nrev_mon;
   Coords C;
-  long long *wg_first, *wg_end, *bunch_first;
-  int *wg_bunch, *bunch_wg0, *bucket, *bunch_ring, *bucket_ring, *np, *nfFill;
+  long long *bunch_first;
+  WgInfo *wgs;
+  BunchInfo *bunches;
+  int *bucket, *bunch_ring, *bucket_ring, *np, *nfFill;
   DevParams *P;
   double *partial, *shift;
   HistPtr Hs;
@@ -2104,6 +2161,8 @@ static void fill_params(const mbt_config *c, const int planes[3], DevParams &P)
   P.sigma_tau = c->sigma_tau;
   P.Nsigma = c->Nsigma;
   P.dT = c->dT;
+  P.inv_sigma = 1.0 / c->sigma_tau;
+  P.inv_dT = 1.0 / c->dT;
   for (int p = 0; p < 3; p++) {
     P.gamma1[p] = c->gamma1[p];
     P.alpha1[p] = c->alpha1[p];
@@ -2128,8 +2187,8 @@ static void fill_params(const mbt_config *c, const int planes[3], DevParams &P)
             (P.ideal_hc ? TF_IDEAL : 0) | (P.amp_dq ? TF_AMP : 0);
   P.fb_len = c->has_rf_feedback ? abs(c->rffb_len_average) : 1;
   P.fb_switch_off = c->has_rf_feedback && c->rffb_len_average < 0;
-  P.vrf_design = c->rffb_vrf_design;
-  P.phi0_design = c->rffb_phi0_design;
+  P.vrf_sin = c->rffb_vrf_design * sin(c->rffb_phi0_design);
+  P.vrf_cos = c->rffb_vrf_design * cos(c->rffb_phi0_design);
 }
 
 template <typename T> static int dalloc(T **p, size_t n)
@@ -2186,8 +2245,7 @@ extern "C" void mbt_ring_destroy(mbt_ring *r)
   (void)hipSetDevice(r->device);
   if (r->stream) (void)hipStreamSynchronize(r->stream); // turns of mbt_ring_track_async may still run
   if (r->pot_host) (void)hipHostFree(r->pot_host);
-  void *ptrs[] = {r->C.s, r->wg_first, r->wg_end, r->bunch_first,
-                  r->wg_bunch, r->bunch_wg0, r->bucket, r->bunch_ring, r->bucket_ring, r->np, r->nfFill,
+  void *ptrs[] = {r->C.s, r->wgs, r->bunches, r->bunch_first, r->bucket, r->bunch_ring, r->bucket_ring, r->np, r->nfFill,
                   r->P, r->partial, r->shift, r->Hs.cnt, r->Hs.sx, r->Hs.sz, r->Hs.tcnt, r->Hs.tsx,
                   r->Hs.tsz, r->Hs.bad, r->sfL, r->sfV, r->sfH, r->Gf, r->pending, r->peek,
                   r->rwhist, r->sqrt_tt, r->rsqrt_tt, r->Ibunch, r->bunch_Ib, r->stats, r->amp, r->rfbuf, r->fnp_out,
@@ -2281,36 +2339,29 @@ static int set_decomposition(mbt_ring *r, int items)
   }
   const int nwg = wg_count(r, items), G = r->G;
   const long long CH = (long long)WG * items;
-  long long *wf = (long long *)malloc(nwg * sizeof(long long)), *we = (long long *)malloc(nwg * sizeof(long long));
-  int *wb = (int *)malloc(nwg * sizeof(int)), *b0 = (int *)malloc((G + 1) * sizeof(int));
+  WgInfo *wi = (WgInfo *)calloc(nwg, sizeof(WgInfo));
+  BunchInfo *bi = (BunchInfo *)calloc(G, sizeof(BunchInfo));
   int w = 0, g = 0;
   long long pos = 0;
   for (int k = 0; k < r->R; k++) {
     const long long Np = r->rh[k].cfg.Np, per_b = (Np + CH - 1) / CH;
     for (int bb = 0; bb < r->rh[k].cfg.Nbunch; bb++, g++) {
-      b0[g] = w;
-      for (long long kk = 0; kk < per_b; kk++, w++) {
-        wf[w] = pos + kk * CH;
-        we[w] = pos + ((kk + 1) * CH < Np ? (kk + 1) * CH : Np);
-        wb[w] = g;
-      }
+      const int kb = r->rh[k].bucket[bb];
+      bi[g] = {k, kb, w, w + (int)per_b, (int)Np, {0, 0, 0}};
+      for (long long kk = 0; kk < per_b; kk++, w++)
+        wi[w] = {pos + kk * CH, (int)((kk + 1) * CH < Np ? CH : Np - kk * CH), g, k, kb, (unsigned)(kk * CH), 0};
       pos += padded_np(Np);
     }
   }
-  b0[G] = w;
   int rc = MBT_OK;
-  if (hipMemcpyAsync(r->wg_first, wf, nwg * sizeof(long long), hipMemcpyHostToDevice, r->stream) != hipSuccess ||
-      hipMemcpyAsync(r->wg_end, we, nwg * sizeof(long long), hipMemcpyHostToDevice, r->stream) != hipSuccess ||
-      hipMemcpyAsync(r->wg_bunch, wb, nwg * sizeof(int), hipMemcpyHostToDevice, r->stream) != hipSuccess ||
-      hipMemcpyAsync(r->bunch_wg0, b0, (G + 1) * sizeof(int), hipMemcpyHostToDevice, r->stream) != hipSuccess ||
+  if (hipMemcpyAsync(r->wgs, wi, nwg * sizeof(WgInfo), hipMemcpyHostToDevice, r->stream) != hipSuccess ||
+      hipMemcpyAsync(r->bunches, bi, G * sizeof(BunchInfo), hipMemcpyHostToDevice, r->stream) != hipSuccess ||
       hipStreamSynchronize(r->stream) != hipSuccess) {
     mbt_set_error("upload of the work-group decomposition failed");
     rc = MBT_EDEVICE;
   }
-  free(wf);
-  free(we);
-  free(wb);
-  free(b0);
+  free(wi);
+  free(bi);
   if (rc == MBT_OK) {
     r->nwg = nwg;
     r->chunk_items = items;
@@ -2768,10 +2819,8 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
       return rcp;
     }
   }
-  DA(r->wg_first, nwg);
-  DA(r->wg_end, nwg);
-  DA(r->wg_bunch, nwg);
-  DA(r->bunch_wg0, G + 1);
+  DA(r->wgs, nwg);
+  DA(r->bunches, G);
   DA(r->bunch_first, G);
   DA(r->bucket, G);
   DA(r->bunch_ring, G);
@@ -2982,8 +3031,8 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
   for (int k = 0; k < R; k++)
     if (r->Ph[k].scan == 1) r->end_each = 1;
   for (int d = 0; d < 2; d++) r->lds_turn[d] = turn_lds(Nc, d);
-  r->lr_lds = nres > 0 && (size_t)9 * NcA * 8 + 64 <= 64 * 1024;
-  r->lds_red = (size_t)(r->lr_lds ? 9 : 6) * NcA * 8 + 64;
+  r->lr_lds = nres > 0 && (size_t)12 * NcA * 8 + 64 <= 64 * 1024;
+  r->lds_red = (size_t)(r->lr_lds ? 12 : 6) * NcA * 8 + 64;
   if (Nc > NCELL_MAX) {
     mbt_set_error("Ncell %d too large for the LDS histogram", Nc);
     mbt_ring_destroy(r);
@@ -3158,9 +3207,8 @@ extern "C" int mbt_ensemble_get_bunch(const mbt_ring *r, int g, double *s)
 extern "C" int mbt_ring_set_bunch(mbt_ring *r, int ib, const double *s) { return mbt_ensemble_set_bunch(r, ib, s); }
 extern "C" int mbt_ring_get_bunch(const mbt_ring *r, int ib, double *s) { return mbt_ensemble_get_bunch(r, ib, s); }
 
-typedef void (*turn_kernel_t)(const DevParams *, Coords, const long long *, const long long *, const int *,
-                              const int *, const int *, const long long *, const double *, const double *,
-                              const double *, const double *, LRDev, const double *, const double *, double *,
+typedef void (*turn_kernel_t)(const DevParams *, Coords, const WgInfo *, int, const int *, const double *,
+                              const double *, const double *, const double *, LRDev, const double *, const double *, double *,
                               HistPtr, const TurnState *, int, RwOld);
 
 #define TK(Q, D, G, M) k_turn<MODE_TURN, Q, D, G, M>
@@ -3195,33 +3243,28 @@ static int launch_turn_pass(mbt_ring *r, int mode, int turn)
           r->rw_part, r->G};
     if (r->rw_lds > lds) lds = r->rw_lds;
   }
-  hipLaunchKernelGGL(k, dim3(r->nwg + ro.nlead), dim3(WG), lds, r->stream, r->P, r->C, r->wg_first, r->wg_end,
-                     r->wg_bunch, r->bunch_ring, r->bucket, r->bunch_first, r->shift, r->sfL, r->sfV, r->sfH,
+  hipLaunchKernelGGL(k, dim3(r->nwg + ro.nlead), dim3(WG), lds, r->stream, r->P, r->C, r->wgs, r->R,
+                     r->bucket, r->shift, r->sfL, r->sfV, r->sfH,
                      r->LR, r->Ibunch, r->pending, r->partial, r->Hs, r->ts, turn, ro);
   CK(hipGetLastError());
   return MBT_OK;
 }
 
-typedef void (*reduce_kernel_t)(const DevParams *, const double *, const int *, const int *, const int *, HistPtr, RedOut,
+typedef void (*reduce_kernel_t)(const DevParams *, const double *, const BunchInfo *, int, HistPtr, RedOut,
                                 const TurnState *, int, int, LRDev, int, int, int);
 
 // k_reduce for Nc slices: the most lanes per pair of slices (of sixteen) that a
-// block has.  A block of 1,024 lanes per bunch while that is no more than a block
+// block has.  A block of 512 lanes per bunch while that is no more than a block
 // per CU, else 256 (the sums are the same: conv_at).
-#define REDUCE_WIDE 1024
+#define REDUCE_WIDE 512
 #define REDUCE_WIDE_BUNCHES 256
 
-static reduce_kernel_t reduce_kernel(int Nc, bool wide)
+template <int NT, bool MIXED> static reduce_kernel_t reduce_kernel(int lanes)
 {
-  const int lanes = (wide ? REDUCE_WIDE : WG) / ((Nc + 1) / 2 > 0 ? (Nc + 1) / 2 : 1);
-  if (wide)
-    return lanes >= 16 ? k_reduce<REDUCE_WIDE, 16>
-                       : (lanes >= 8 ? k_reduce<REDUCE_WIDE, 8>
-                                     : (lanes >= 4 ? k_reduce<REDUCE_WIDE, 4>
-                                                   : (lanes >= 2 ? k_reduce<REDUCE_WIDE, 2> : k_reduce<REDUCE_WIDE, 1>)));
-  return lanes >= 16 ? k_reduce<WG, 16>
-                     : (lanes >= 8 ? k_reduce<WG, 8>
-                                   : (lanes >= 4 ? k_reduce<WG, 4> : (lanes >= 2 ? k_reduce<WG, 2> : k_reduce<WG, 1>)));
+  return lanes >= 16 ? k_reduce<NT, 16, MIXED>
+                     : (lanes >= 8 ? k_reduce<NT, 8, MIXED>
+                                   : (lanes >= 4 ? k_reduce<NT, 4, MIXED>
+                                                 : (lanes >= 2 ? k_reduce<NT, 2, MIXED> : k_reduce<NT, 1, MIXED>)));
 }
 
 static int launch_reduce(mbt_ring *r, int phase, int turn)
@@ -3230,8 +3273,10 @@ static int launch_reduce(mbt_ring *r, int phase, int turn)
   // pass only when a ring's kicks or LR resonators need them
   const int dip = phase != 2 || r->any_dip;
   const bool wide = r->G <= REDUCE_WIDE_BUNCHES;
-  hipLaunchKernelGGL(reduce_kernel(r->Nc, wide), dim3(r->G), dim3(wide ? REDUCE_WIDE : WG), r->lds_red, r->stream, r->P, r->partial, r->bunch_wg0,
-                     r->bunch_ring, r->bucket, r->Hs, r->Ro, r->ts, phase, dip, r->LR, r->lr_lds,
+  const int nt = wide ? REDUCE_WIDE : WG, pairs = (r->Nc + 1) / 2, lanes = nt / (pairs > 0 ? pairs : 1);
+  const reduce_kernel_t k = r->mixed ? (wide ? reduce_kernel<REDUCE_WIDE, true>(lanes) : reduce_kernel<WG, true>(lanes))
+                                     : (wide ? reduce_kernel<REDUCE_WIDE, false>(lanes) : reduce_kernel<WG, false>(lanes));
+  hipLaunchKernelGGL(k, dim3(r->G), dim3(nt), r->lds_red, r->stream, r->P, r->partial, r->bunches, r->R, r->Hs, r->Ro, r->ts, phase, dip, r->LR, r->lr_lds,
                      turn, r->Nc);
   CK(hipGetLastError());
   return MBT_OK;
@@ -3240,8 +3285,8 @@ static int launch_reduce(mbt_ring *r, int phase, int turn)
 // Turn end (end), long-range recurrence and RF-feedback solve of every ring.
 static int launch_ring_end(mbt_ring *r, int end, int init)
 {
-  hipLaunchKernelGGL(k_ring_end, dim3(r->R), dim3(r->nres > 0 ? 256 : 64), 0, r->stream, r->P, r->ts, r->bunch_Ib,
-                     r->Ibunch, r->nfFill, r->LR, end, init);
+  hipLaunchKernelGGL(init ? k_ring_end<true> : k_ring_end<false>, dim3(r->R), dim3(r->nres > 0 ? 256 : 64), 0, r->stream,
+                     r->P, r->ts, r->bunch_Ib, r->Ibunch, r->nfFill, r->LR, end);
   CK(hipGetLastError());
   return MBT_OK;
 }
@@ -3341,8 +3386,7 @@ static int enqueue_turn(mbt_ring *r, hipEvent_t *E, int turn)
     else
       hipLaunchKernelGGL(k_rwg_tile<false>, tg, dim3(256), lds, r->stream, r->rwg, r->P, r->ts, turn, r->rwhist,
                          r->Ibunch, r->nfFill);
-    const long long tot = (long long)r->rwg.h * r->rwg.N;
-    hipLaunchKernelGGL(k_rwg_sum, dim3((unsigned)((tot + 255) / 256)), dim3(256), 0, r->stream, r->rwg, r->P, r->ts,
+    hipLaunchKernelGGL(k_rwg_sum, dim3((r->rwg.N + 15) / 16, r->rwg.h), dim3(256), 0, r->stream, r->rwg, r->P, r->ts,
                        turn, r->pending);
   } else if (r->rw_split) {
     hipLaunchKernelGGL(k_rw_fresh, dim3(r->G), dim3(WG), 0, r->stream, r->P, r->bunch_ring, r->rwhist, r->sqrt_tt,
@@ -3744,8 +3788,8 @@ extern "C" int mbt_ring_autotune(mbt_ring *r, int *best_items, double *ms)
       float t = 0.0f;
       for (int rep = 0; rep <= AUTOTUNE_REPS; rep++) {
         if (rep == 1) CK(hipEventRecord(e0, r->stream));
-        hipLaunchKernelGGL(k, dim3(r->nwg), dim3(WG), r->lds_turn[r->any_dip], r->stream, r->P, r->C, r->wg_first, r->wg_end,
-                           r->wg_bunch, r->bunch_ring, r->bucket, r->bunch_first, r->shift, r->sfL, r->sfV, r->sfH,
+        hipLaunchKernelGGL(k, dim3(r->nwg), dim3(WG), r->lds_turn[r->any_dip], r->stream, r->P, r->C, r->wgs, r->R,
+                           r->bucket, r->shift, r->sfL, r->sfV, r->sfH,
                            r->LR, r->Ibunch, r->pending, r->partial, r->Hs, r->ts, 0, RwOld{});
         CK(hipGetLastError());
       }

@@ -82,4 +82,12 @@ __device__ __forceinline__ double wsum64x8(const double v[8])
   return y;
 }
 
+// Two sums over the 64 lanes of a wave: lanes 0-31 return the total of a, lanes
+// 32-63 that of b.
+__device__ __forceinline__ double wsum64x2(double a, double b)
+{
+  const double x = swap_sum<32>(a, b);
+  return rowsum16(swap_sum<16>(x, x));
+}
+
 #endif

@@ -1,12 +1,13 @@
 """The per-bunch reduction's convolutions and the one-pass resistive-wall sum at the
-edges of their ranges, and the turn count a block of launches keeps itself.
+edges of their ranges, the sum as a matrix product, and the turn count a block of launches keeps itself.
 
 Slice counts around the lanes a group of slices gets (16, 8, 4, 2 and 1 of a block
-of 256 or 1,024 lanes) and around the eight and sixteen terms read at a time, one
+of 256 or 512 lanes) and around the eight and sixteen terms read at a time, one
 bunch and more bunches than take the wide block; the wide and the narrow block give
 the same bits (a ring alone and in an ensemble past the line).  Resistive wall: one
 bunch, every bucket, more (row, bunch) pairs than lanes, the trigger's change at
-turn 50 inside and at the ends of calls.  Against the oracle within 1e-12, the
+turn 50 inside and at the ends of calls; as a matrix product buckets below, at and
+past its tiles of 16, few and many slices of its sum, one ring.  Against the oracle within 1e-12, the
 bound of the other parity tests: the same terms added in another order.
 """
 import numpy as np
@@ -36,8 +37,8 @@ def conf(d, name, h, bunches, np_, ncell=0, nmlt=0, **tracking):
                     d + "/")
 
 
-def check(cfg, calls):
-    orc, g = o.OracleRing(cfg, o.RNG_PHILOX), m.Ring(cfg)
+def check(cfg, calls, **options):
+    orc, g = o.OracleRing(cfg, o.RNG_PHILOX), m.Ring(cfg, **options)
     orc.prepare()
     g.prepare()
     for n in calls:
@@ -64,6 +65,13 @@ def test_convolutions(tmp_path, ncell, bunches):
 def test_wall_sum(tmp_path, h, bunches, nmlt, calls):
     print("case", h, bunches, nmlt, flush=True)
     check(conf(str(tmp_path), "wall", h, bunches, 31, nmlt=nmlt, triggerRW=1), calls)
+
+
+@pytest.mark.parametrize("h,bunches,nmlt", [(3, 3, 1), (15, 4, 2), (16, 16, 11), (17, 5, 12), (130, 13, 25),
+                                            (416, 416, 40)])
+def test_wall_product(tmp_path, h, bunches, nmlt):
+    print("case", h, bunches, nmlt, flush=True)
+    check(conf(str(tmp_path), "product", h, bunches, 31, nmlt=nmlt, triggerRW=1), [2 * nmlt, 7], force_gemm=True)
 
 
 def test_wide_and_narrow_blocks_agree(tmp_path):
