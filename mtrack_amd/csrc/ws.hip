@@ -102,6 +102,7 @@ struct WSD {
   double *dip;      // [2][WS_RING][G] wall dipoles of the bunches' centroids (HOR, VER), a row per turn
   const double *wall; // [trigger][2][Nmlt + 1][h] wake per tap and distance in buckets (entry d - 1)
   double2 *Exy;     // [G][S*25] (Ex, Ey) of every grid point
+  double2 *tab;     // [G][S][WS_QT] the ion train's tables of it
   double *li;       // [5][G][S*25] local ions: Nri x x' y y'
   double *cl;       // [5][cap] ion cloud
   long long cap;
@@ -410,12 +411,39 @@ __global__ __launch_bounds__(WS_WG) void k_ws_phase1(WSP P, WSD D, WSStep T)
   D.Exy[gq] = make_double2(Ex, Ey);
 }
 
+// The ion train's field table of a slice: the 5 x 5 grid fields with the edge rows in
+// x repeated once more, rows kx = 0 .. 5 for the cells [kx - 3, kx - 2]: WS_ROWS
+// double2 (Ex, Ey) of the row's lower point, as many of its step to the upper one,
+// E(kx + 1, z) - E(kx, z), zero past the edge.  The steps are the subtractions of
+// the bilinear formula, made once per table instead of once per ion.  Two arrays of
+// 16-byte entries rather than 32-byte pairs: the lanes of one read then spread over
+// all sixteen 16-byte bank groups of the LDS, not eight (measured: a sixth of the
+// bank-conflict cycles, SQ_LDS_BANK_CONFLICT).
+#define WS_ROWS 30
+#define WS_QT (2 * WS_ROWS) // double2 per slice
+
+// Entry k of the table of a slice with grid fields t.
+__device__ __forceinline__ void ws_table_entry(const double2 *t, int k, double2 *T)
+{
+  const int kx = k / 5, z = k - 5 * kx;
+  const double2 e1 = t[5 * (min(max(kx - 3, -2), 2) + 2) + z], e2 = t[5 * (min(max(kx - 2, -2), 2) + 2) + z];
+  T[k] = e1;
+  T[WS_ROWS + k] = make_double2(e2.x - e1.x, e2.y - e1.y);
+}
+
 // The ions every bunch creates, one per thread: one per local grid point of
 // each slice, kicked by the bunch's later slices (their field tables read from
-// the one k_ws_phase1 wrote).
+// the one k_ws_phase1 wrote); the blocks after those (ion-parallel train) write the
+// train's tables, an entry and its step per thread.
 __global__ __launch_bounds__(WS_WG) void k_ws_create(WSP P, WSD D)
 {
   const int S = P.S, npts = S * 25;
+  const int made = (int)(((long long)P.G * npts + WS_WG - 1) / WS_WG);
+  if ((int)blockIdx.x >= made) {
+    const long long k = (long long)(blockIdx.x - made) * WS_WG + threadIdx.x, sl = k / WS_ROWS;
+    if (sl < (long long)P.G * S) ws_table_entry(D.Exy + sl * 25, (int)(k - sl * WS_ROWS), D.tab + sl * WS_QT);
+    return;
+  }
   const long long gq = (long long)blockIdx.x * WS_WG + threadIdx.x;
   if (gq >= (long long)P.G * npts) return;
   const int b = (int)(gq / npts), q = (int)(gq - (long long)b * npts);
@@ -601,147 +629,184 @@ __global__ __launch_bounds__(WS_WG) void k_ws_train(WSP P, WSD D, int ib, long l
   }
 }
 
-// The ion train's field table of a slice in LDS, over the 5 x 5 grid with its
-// edge rows and columns repeated once more: entry 7 kx + kz (kx in 0 .. 5,
-// kz in 0 .. 6) of the first WS_QT double2 holds the field (Ex, Ey) at the
-// point (clamp(kx - 3), clamp(kz - 3)) of the grid, the same entry of the next
-// WS_QT its step to the next point in x, E(kx + 1, kz) - E(kx, kz) (zero past
-// the edge).  The steps are the subtractions of the bilinear formula, made once
-// per table instead of once per ion.  Two arrays of 16-byte entries rather than
-// 32-byte (field, step) pairs: the lanes of one read then spread over all
-// sixteen 16-byte bank groups of the LDS, not eight (measured: a sixth of the
-// bank-conflict cycles, SQ_LDS_BANK_CONFLICT).
-#define WS_QT 42 // entries per slice
-#define WS_CH 16 // slices per staged chunk of a bunch's tables (a multiple of 4)
+#define WS_CH 8 // slices per chunk of a bunch's tables (a multiple of 4)
+// double2 a block reads per chunk: two per lane
+#define WS_BUF (2 * WS_WG)
+static_assert(WS_CH * WS_QT <= WS_BUF, "a chunk fits its buffer");
 
-// ws_interp on a slice's table, with the cell anchored at the floor of the
-// grid quotient u: the cell [f, f + 1], f = floor(u), at weight u - f.  The
-// reference anchors at the grid point nearer zero (trunc(u)) and weighs toward
-// the next one out; for u >= 0 that is the same cell and steps, for u < 0 the
-// same bilinear interpolant taken from its other end.  The floor and the
-// weight come from t = u + 3 in one rounding (a fused multiply-add), as its
-// integer part and v_fract_f64: the weight then carries the rounding of t (at
-// most 4.4e-16 for |u| < 3) instead of that of u.  Quotients past the grid take
-// the cell [-3, -2] or [2, 3], whose outer point repeats the edge (a zero step),
-// so the field there is the edge value, as the reference's clamped partner
-// gives.  No sign tests; the four reads are fixed offsets from one address.
-__device__ __forceinline__ void ws_interp_p(const double2 *t, double iax, double iaz, double xx, double yy,
-                                            double &Ex, double &Ey)
+// An ion's cell [kx - 3, kx - 2] x [kz - 3, kz - 2] of the grid, kx, kz in 0 .. 5 the
+// floor of its grid quotient plus 3: ion_weight(x, ix, gx) is its weight in the cell
+// (the quotient's fraction), in [0, 1) as long as it stays there; e1, e3 the table's
+// entries of the cell's lower and upper row ends.  The outer cells have no step (in z
+// because both ends are the same entry), so their weight says only whether the ion is
+// still there: the quotient is scaled so that [0, 1) takes in 2^20 spacings beyond the
+// grid, as far as lost ions get, and ends 2^-30 of one outside it, clear of its rounding.
+// The reference anchors at the grid point nearer zero (trunc of the quotient) and weighs
+// toward the next one out; above zero that is the same cell and steps, below it the same
+// bilinear interpolant taken from its other end.
+struct IonCell {
+  double ix, iz, gx, gz;
+  const double2 *e1, *e3;
+};
+
+// The weights' (ix, gx) per kx, then (iz, gz) per kz, for the kernel's LDS.
+__device__ __forceinline__ double2 ion_cell_weight(const WSP &P, int i)
 {
-  // the bilinear steps as fused multiply-adds (one rounding less each)
-#pragma clang fp contract(fast)
-  const double tx = fma(xx, iax, 3.0), tz = fma(yy, iaz, 3.0);
-  const double sx = __builtin_amdgcn_fract(tx), sz = __builtin_amdgcn_fract(tz);
-  const int kx = min(max((int)tx, 0), 5), kz = min(max((int)tz, 0), 5);
-  const double2 *e = t + 7 * kx + kz;
-  const double2 e1 = e[0], e3 = e[1], d1 = e[WS_QT], d3 = e[WS_QT + 1];
-  const double y5 = e1.y + sx * d1.y;
-  const double y6 = e3.y + sx * d3.y;
-  const double x5 = e1.x + sx * d1.x;
-  const double x6 = e3.x + sx * d3.x;
-  Ey = y5 + sz * (y6 - y5);
-  Ex = x5 + sz * (x6 - x5);
+  const double far = 0x1p-20, ia = i < 6 ? P.iaAx : P.iaAz;
+  const int k = i % 6;
+  return make_double2(k == 0 || k == 5 ? ia * far : ia,
+                      k == 0 ? 2.0 - 2.0 * far - 0x1p-50 : k == 5 ? 3.0 + 2.0 * far + 0x1p-50 : (double)k);
 }
 
-// One slice c of a bunch for the lane's ion: the field at the ion, the ion's
-// kick, and the ion's share Nri E of the slice's kick.  The velocity kick
+__device__ __forceinline__ double ion_weight(double x, double ix, double gx) { return fma(x, ix, 3.0) - gx; }
+
+__device__ __forceinline__ IonCell ion_cell(const WSP &P, const double2 *qt, const double2 *wt, double x, double y)
+{
+  const int kx = min(max((int)floor(fma(x, P.iaAx, 3.0)), 0), 5);
+  const int kz = min(max((int)floor(fma(y, P.iaAz, 3.0)), 0), 5);
+  const double2 a = wt[kx], b = wt[6 + kz];
+  return {a.x, b.x, a.y, b.y, qt + 5 * kx + max(kz - 1, 0), qt + 5 * kx + min(kz, 4)};
+}
+
+// The entries the cell has in a slice's table, o entries on.
+struct IonField {
+  double2 e1, e3, d1, d3;
+};
+
+__device__ __forceinline__ IonField ion_load(const IonCell &c, int o)
+{
+  return {c.e1[o], c.e3[o], c.e1[o + WS_ROWS], c.e3[o + WS_ROWS]};
+}
+
+// High words of a weight at or above this one, unsigned: outside [0, 1), or NaN.
+#define ION_ONE 0x3ff00000u
+
+// The lane's ion.
+struct Ion {
+  double Nri, x, xd, y, yd;
+};
+
+// One slice for the lane's ion: the field at the ion, its kick, and its share Nri E of
+// the slice's kick.  f holds the entries of the ion's cell; the velocity kick
 // deltT (factF E) of the reference is taken as (deltT factF) E, one fused
 // multiply-add with the product precomputed (a rounding-level change).
-__device__ __forceinline__ void ion_slice(const WSP &P, const double2 *qt, int c, double Nri, double &x, double &xd,
-                                          double &y, double &yd, double &sx, double &sy)
+__device__ __forceinline__ void ion_kick(const WSP &P, const IonField &f, double wx, double wz, Ion &I, double &sx,
+                                         double &sy)
 {
-  // the ion's kick as fused multiply-adds
+  // the bilinear steps and the kicks as fused multiply-adds (one rounding less each)
 #pragma clang fp contract(fast)
-  double Ex, Ey;
-  ws_interp_p(qt + c * 2 * WS_QT, P.iaAx, P.iaAz, x, y, Ex, Ey);
-  xd = xd + P.dtF * Ex;
-  x = x + P.deltT * xd;
-  yd = yd + P.dtF * Ey;
-  y = y + P.deltT * yd;
-  sx = Nri * Ex;
-  sy = Nri * Ey;
+  const double y5 = f.e1.y + wx * f.d1.y;
+  const double y6 = f.e3.y + wx * f.d3.y;
+  const double x5 = f.e1.x + wx * f.d1.x;
+  const double x6 = f.e3.x + wx * f.d3.x;
+  const double Ey = y5 + wz * (y6 - y5);
+  const double Ex = x5 + wz * (x6 - x5);
+  I.xd = I.xd + P.dtF * Ex;
+  I.x = I.x + P.deltT * I.xd;
+  I.yd = I.yd + P.dtF * Ey;
+  I.y = I.y + P.deltT * I.yd;
+  sx = I.Nri * Ex;
+  sy = I.Nri * Ey;
 }
 
-// One group of four slices c0 .. c0 + 3 of a bunch for the lane's ion: the
-// kicks, then the group's eight field sums (Nri Ex, Nri Ey per slice) reduced
-// over the wave into wred.  qt holds the tables of the slices from cq on.
-// ALL: every lane's ion is in the cloud (lanes past the last ion carry Nri = 0
-// from a finite state, so they add exact zeros); FULL: all four slices exist.
-template <bool ALL, bool FULL>
-__device__ __forceinline__ void ions_group(const WSP &P, const double2 *qt, int cq, int c0, int S, bool act,
-                                           double Nri, double &x, double &xd, double &y, double &yd,
-                                           double (*wred)[WS_WG / 64], int lane, int wv)
+// The wave's sums of v into wred: the 2 N field sums of slices c0 .. in v[0 ..], into
+// rows 2 c0 .., and (CLOUD) the cloud sums Nri x, Nri y, Nri in v[4 .. 6].
+template <int N, bool CLOUD>
+__device__ __forceinline__ void ions_sum(const Ion &I, bool act, double v[8], int c0, int S,
+                                         double (*wred)[WS_WG / 64], int lane, int wv)
 {
-  double v[8];
-#pragma unroll
-  for (int k = 0; k < 4; k++) {
-    const int c = c0 + k;
-    double sx = 0.0, sy = 0.0;
-    if ((ALL || act) && (FULL || c < S)) ion_slice(P, qt, c - cq, Nri, x, xd, y, yd, sx, sy);
-    v[2 * k] = sx;
-    v[2 * k + 1] = sy;
+  if (CLOUD && act) {
+    v[4] = I.Nri * I.x;
+    v[5] = I.Nri * I.y;
+    v[6] = I.Nri;
   }
-  const double t = wsum64x8(v);
-  const int idx = lane >> 3, c = c0 + (idx >> 1);
-  if ((lane & 7) == 0 && (FULL || c < S)) wred[2 * c + (idx & 1)][wv] = t;
-}
-
-// The last r = 1 or 2 slices c0 .. c0 + r - 1 of a bunch and, after them, the
-// cloud sums Nri x, Nri y, Nri: one eight-value reduction for both.
-template <bool ALL>
-__device__ __forceinline__ void ions_tail(const WSP &P, const double2 *qt, int cq, int c0, int r, int S, bool act,
-                                          double Nri, double &x, double &xd, double &y, double &yd,
-                                          double (*wred)[WS_WG / 64], int lane, int wv)
-{
-  double v[8];
-#pragma unroll
-  for (int k = 0; k < 2; k++) {
-    double sx = 0.0, sy = 0.0;
-    if ((ALL || act) && k < r) ion_slice(P, qt, c0 + k - cq, Nri, x, xd, y, yd, sx, sy);
-    v[2 * k] = sx;
-    v[2 * k + 1] = sy;
-  }
-  v[4] = ALL || act ? Nri * x : 0.0;
-  v[5] = ALL || act ? Nri * y : 0.0;
-  v[6] = ALL || act ? Nri : 0.0;
-  v[7] = 0.0;
   const double t = wsum64x8(v);
   const int m = lane >> 3;
   if ((lane & 7) == 0) {
-    if (m < 2 * r)
+    if (m < 2 * N)
       wred[2 * c0 + m][wv] = t;
-    else if (m >= 4 && m < 7)
+    else if (CLOUD && m >= 4 && m < 7)
       wred[2 * S + m - 4][wv] = t;
   }
 }
 
-// Slices cb .. ce - 1 of a bunch for the lane's ion (qt: their tables from cb
-// on; cb a multiple of 4) and, when they end the bunch (ce = S), the cloud
-// sums Nri x, Nri y, Nri after it, over the wave into wred.
-template <bool ALL>
-__device__ __forceinline__ void ions_chunk(const WSP &P, const double2 *qt, int cb, int ce, bool act, double Nri,
-                                           double &x, double &xd, double &y, double &yd,
-                                           double (*wred)[WS_WG / 64], int lane, int wv)
+// N <= 4 slices of a bunch from entry o of the tables on: the kicks, then the 2 N field
+// sums and (CLOUD, N <= 2: the bunch's last slices) the cloud sums after them, over the
+// wave in one reduction into wred from row 2 c0 on.
+// Each slice's entries are read before the ion's place in the slice is known, from the
+// cell it had: an ion changes cells in one of five thousand slices, and the weights
+// show it (they leave [0, 1)).  Then the wave finds its cells and reads again (in one of
+// sixty slices).  One test for four slices, done again from their start where it fails,
+// with or without entries read a slice ahead, was no faster.
+template <int N, bool CLOUD>
+__device__ __forceinline__ void ions_group(const WSP &P, const double2 *qt, const double2 *wt, int o, int c0,
+                                           IonCell &cl, Ion &I, double (*wred)[WS_WG / 64], int lane, int wv)
 {
-  const int S = P.S;
+  double v[8] = {};
+#pragma unroll
+  for (int k = 0; k < N; k++) {
+    const int ok = o + k * WS_QT;
+    IonField f = ion_load(cl, ok);
+    asm volatile("" ::: "memory"); // keeps these reads here, ahead of the branch
+    double wx = ion_weight(I.x, cl.ix, cl.gx), wz = ion_weight(I.y, cl.iz, cl.gz);
+    const unsigned out = max((unsigned)__double2hiint(wx), (unsigned)__double2hiint(wz));
+    if (__builtin_expect(__any(out >= ION_ONE), 0)) {
+      cl = ion_cell(P, qt, wt, I.x, I.y);
+      f = ion_load(cl, ok);
+      wx = ion_weight(I.x, cl.ix, cl.gx);
+      wz = ion_weight(I.y, cl.iz, cl.gz);
+    }
+    ion_kick(P, f, wx, wz, I, v[2 * k], v[2 * k + 1]);
+  }
+  ions_sum<N, CLOUD>(I, true, v, c0, P.S, wred, lane, wv);
+}
+
+// The slices cb .. ce - 1 of a bunch (their tables at entry o; cb a multiple of 4) and,
+// when they end the bunch (ce = S), the cloud sums after it.
+__device__ __forceinline__ void ions_chunk(const WSP &P, const double2 *qt, const double2 *wt, int o, int cb, int ce,
+                                           IonCell &cl, Ion &I, double (*wred)[WS_WG / 64], int lane, int wv)
+{
+  if (cb == 0) cl = ion_cell(P, qt, wt, I.x, I.y);
   int c0 = cb;
-  for (; c0 + 4 <= ce; c0 += 4) ions_group<ALL, true>(P, qt, cb, c0, S, act, Nri, x, xd, y, yd, wred, lane, wv);
-  if (ce < S) return;
-  const int r = S - c0;
-  if (r == 1 || r == 2) {
-    ions_tail<ALL>(P, qt, cb, c0, r, S, act, Nri, x, xd, y, yd, wred, lane, wv);
-    return;
+  for (; c0 + 4 <= ce; c0 += 4, o += 4 * WS_QT) ions_group<4, false>(P, qt, wt, o, c0, cl, I, wred, lane, wv);
+  if (ce < P.S) return;
+  const int r = P.S - c0;
+  if (r == 1)
+    ions_group<1, true>(P, qt, wt, o, c0, cl, I, wred, lane, wv);
+  else if (r == 2)
+    ions_group<2, true>(P, qt, wt, o, c0, cl, I, wred, lane, wv);
+  else {
+    if (r) ions_group<3, false>(P, qt, wt, o, c0, cl, I, wred, lane, wv);
+    ions_group<0, true>(P, qt, wt, o, P.S, cl, I, wred, lane, wv);
   }
-  if (r) ions_group<ALL, false>(P, qt, cb, c0, S, act, Nri, x, xd, y, yd, wred, lane, wv);
-  double s0 = ALL || act ? Nri * x : 0.0, s1 = ALL || act ? Nri * y : 0.0, s2 = ALL || act ? Nri : 0.0;
-  s0 = wsum64(s0);
-  s1 = wsum64(s1);
-  s2 = wsum64(s2);
-  if (lane == 0) {
-    wred[2 * S][wv] = s0;
-    wred[2 * S + 1][wv] = s1;
-    wred[2 * S + 2][wv] = s2;
+}
+
+// The slices of a chunk in a bunch that some of the lanes' ions are not yet made in:
+// only those in the cloud (act) move and count.
+__device__ __forceinline__ void ions_chunk_some(const WSP &P, const double2 *qt, const double2 *wt, int o, int cb,
+                                                int ce, bool act, Ion &I, double (*wred)[WS_WG / 64], int lane,
+                                                int wv)
+{
+  for (int c = cb; c < ce; c++, o += WS_QT) {
+    double v[8] = {};
+    if (act) {
+      const IonCell cl = ion_cell(P, qt, wt, I.x, I.y);
+      ion_kick(P, ion_load(cl, o), ion_weight(I.x, cl.ix, cl.gx), ion_weight(I.y, cl.iz, cl.gz), I, v[0], v[1]);
+    }
+    ions_sum<1, false>(I, act, v, c, P.S, wred, lane, wv);
   }
+  if (ce < P.S) return;
+  double v[8] = {};
+  ions_sum<0, true>(I, act, v, 0, P.S, wred, lane, wv);
+}
+
+// A barrier for what the block shares in LDS alone: loads and stores of global
+// memory stay under way across it (__syncthreads waits for them).
+__device__ __forceinline__ void lds_barrier()
+{
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
 // Ion-parallel train: lane q carries ion q = j * Nions + p (ion p made by bunch
@@ -749,15 +814,25 @@ __device__ __forceinline__ void ions_chunk(const WSP &P, const double2 *qt, int 
 // each reached after its drift time.  Per bunch ib the block writes the 2 S
 // slice sums of Nri * E and the cloud sums Nri x, Nri y, Nri after the bunch,
 // each the fixed-order sum of its four waves' sums.  The bunches up to the
-// block's last creator (some lanes' ions not yet made) run with per-lane
-// predicates, the rest without.  The tables of a bunch are staged in chunks
-// of WS_CH slices (dynamic LDS: min(S, WS_CH) * 2 WS_QT double2, 21.5 KB at
-// most), so that six blocks fit a CU: 80 registers a lane allow six waves per
-// SIMD, and the 1,422 blocks of the 356-bunch train are all resident at once.
-__global__ __launch_bounds__(WS_WG) void k_ws_ions(WSP P, WSD D)
+// block's last creator (some ions not yet made) run with per-lane
+// predicates, the rest without.
+// Bound: the chain of the longest block, (G - 1) S slices one after the other, and
+// FP64 issue while all blocks are there.  So the chain has no wait for memory in it:
+// the tables of a bunch come ready-made in chunks of WS_CH slices through two buffers
+// in LDS, one barrier a chunk (for LDS alone), the next chunk's entries on their way in
+// registers while a chunk is used, and a slice's reads don't wait for its cell.  A
+// chunk is read in full: past the bunch's last slice it holds the next bunch's tables,
+// past the last bunch's the room left for it.  356 bunches x 41 slices 3.03 -> 2.82 ms,
+// 61 x 39 421 -> 350 us, results the same to the bit (tables built from the grid fields
+// by every block, waited for; the cell found in every slice).  In trials of this form
+// 16 slices a chunk were better for the short train by 8 % and worse for the long by
+// 6 %, 4 or 6 waves per SIMD worse, two ions per lane 1.2 and 1.6 times slower.
+__global__ __launch_bounds__(WS_WG, 5) void k_ws_ions(WSP P, WSD D)
 {
-  extern __shared__ double2 qt_s[];
-  __shared__ double wred[2 * WS_S + 3][WS_WG / 64];
+  constexpr int NW = WS_WG / 64;
+  __shared__ double2 qt[2 * WS_BUF];
+  __shared__ double2 wt[12];
+  __shared__ double wredb[2][2 * WS_S + 3][NW];
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, S = P.S, npts = S * 25, NQ = 2 * S + 3;
   const size_t GP = (size_t)P.G * npts;
   const long long nI = (long long)(P.G - 1) * npts;
@@ -777,50 +852,57 @@ __global__ __launch_bounds__(WS_WG) void k_ws_ions(WSP P, WSD D)
   const long long q0 = (long long)L * WS_WG, q = q0 + tid;
   const int jmin = (int)(q0 / npts);
   const int jmax = (int)(min(q0 + WS_WG - 1, nI - 1) / npts);
+  double2 g0, g1;
+  const auto fetch = [&](int ib, int cb) {
+    const double2 *t = D.tab + ((size_t)ib * S + cb) * WS_QT + tid;
+    g0 = t[0];
+    g1 = t[WS_WG];
+  };
+  const auto stage = [&](int o) {
+    qt[o + tid] = g0;
+    qt[o + WS_WG + tid] = g1;
+  };
+  fetch(jmin + 1, 0);
   const bool valid = q < nI;
   const int j = valid ? (int)(q / npts) : P.G;
-  double Nri = 0.0, x = 0.0, xd = 0.0, y = 0.0, yd = 0.0;
-  if (valid) {
-    Nri = D.li[q];
-    x = D.li[GP + q];
-    xd = D.li[2 * GP + q];
-    y = D.li[3 * GP + q];
-    yd = D.li[4 * GP + q];
-  }
-  // threads 0 .. 6 WS_QT - 1 stage entry r of the tables of slices sl0,
-  // sl0 + 6, ... of a chunk: a fixed grid point and its x neighbour per thread
-  const int sl0 = tid / WS_QT, r = tid % WS_QT, gz = min(max(r % 7 - 3, -2), 2);
-  const int src = 12 + 5 * min(max(r / 7 - 3, -2), 2) + gz, src2 = 12 + 5 * min(max(r / 7 - 2, -2), 2) + gz;
+  Ion I = {0.0, 0.0, 0.0, 0.0, 0.0};
+  if (valid) I = {D.li[q], D.li[GP + q], D.li[2 * GP + q], D.li[3 * GP + q], D.li[4 * GP + q]};
+  if (tid < 12) wt[tid] = ion_cell_weight(P, tid);
+  stage(0);
+  lds_barrier();
+  IonCell cl;
+  int o = 0;
   for (int ib = jmin + 1; ib < P.G; ib++) {
+    double(*wred)[NW] = wredb[ib & 1];
+    const double dt = D.dtime[ib];
+    const long long to = D.toff[ib];
     const bool act = ib > jmax || j < ib;
     if (act) {
-      const double dt = D.dtime[ib];
-      x = x + dt * xd;
-      y = y + dt * yd;
+      I.x = I.x + dt * I.xd;
+      I.y = I.y + dt * I.yd;
     }
-    const double2 *exy = D.Exy + (size_t)ib * npts;
     for (int cb = 0; cb < S; cb += WS_CH) {
       const int ce = min(S, cb + WS_CH);
-      __syncthreads(); // the previous chunk's tables (and bunch's sums) have been read
-      if (tid < 6 * WS_QT)
-        for (int c = cb + sl0; c < ce; c += 6) {
-          const double2 a = exy[c * 25 + src], b = exy[c * 25 + src2];
-          qt_s[(c - cb) * 2 * WS_QT + r] = a;
-          qt_s[(c - cb) * 2 * WS_QT + WS_QT + r] = make_double2(b.x - a.x, b.y - a.y);
-        }
-      __syncthreads();
-      if (ib <= jmax)
-        ions_chunk<false>(P, qt_s, cb, ce, act, Nri, x, xd, y, yd, wred, lane, wv);
+      if (ce < S)
+        fetch(ib, ce);
       else
-        ions_chunk<true>(P, qt_s, cb, ce, true, Nri, x, xd, y, yd, wred, lane, wv);
+        fetch(min(ib + 1, P.G - 1), 0);
+      if (ib <= jmax)
+        ions_chunk_some(P, qt, wt, o, cb, ce, act, I, wred, lane, wv);
+      else
+        ions_chunk(P, qt, wt, o, cb, ce, cl, I, wred, lane, wv);
+      // the other buffer's last readers are a barrier behind
+      o = WS_BUF - o;
+      stage(o);
+      lds_barrier();
     }
-    __syncthreads();
-    // quantity-major, so that k_ws_ksum reads each quantity's partials contiguously
+    // quantity-major, so that k_ws_ksum reads each quantity's partials contiguously;
+    // the bunch after next is the first to write its sums over these, a barrier on
     const long long nbi = min(((long long)ib * npts + WS_WG - 1) / WS_WG, (long long)D.nblk_ions);
     for (int i = tid; i < NQ; i += WS_WG) {
       double v = 0.0;
-      for (int w = 0; w < WS_WG / 64; w++) v += wred[i][w];
-      D.tpart[D.toff[ib] + i * nbi + L] = v;
+      for (int w = 0; w < NW; w++) v += wred[i][w];
+      D.tpart[to + i * nbi + L] = v;
     }
   }
 }
@@ -922,7 +1004,7 @@ extern "C" void mbt_ws_destroy(mbt_ws *w)
   void *p[] = {w->D.sl,  w->D.dip, w->d_wall, w->D.Exy, w->D.li,     w->D.cl,     w->D.part,    w->D.psum,
                w->D.done, w->D.cm,  w->D.mon,  w->D.ion, w->D.zcm,    w->d_bucket, w->d_npop,
                w->d_nofe, w->d_wallcur, w->d_nelec, w->d_convion, w->D.tpart, w->d_dtime, w->d_toff,
-               w->D.tot};
+               w->D.tot,  w->D.tab};
   for (size_t i = 0; i < sizeof p / sizeof p[0]; i++)
     if (p[i]) (void)hipFree(p[i]);
   if (w->ev)
@@ -1133,6 +1215,7 @@ extern "C" int mbt_ws_create(const mbt_config *c, int device, int flags, mbt_ws 
     w->serial = (flags & MBT_WS_SERIAL_TRAIN) || G < 2 || ntp * (long long)sizeof(double) > WS_TRAIN_PARTIAL_MAX;
     if (!w->serial && P.fbii) {
       WA(w->D.tpart, ntp);
+      WA(w->D.tab, (size_t)G * S * WS_QT + WS_BUF);
       WA(w->D.tot, (size_t)G * WS_TQ);
       WA(w->d_toff, G);
       WUP(w->d_toff, toff, G);
@@ -1223,13 +1306,13 @@ static int ws_enqueue(mbt_ws *w, long n)
     hipLaunchKernelGGL(k_ws_phase1, dim3(G + nbp), dim3(WS_WG), lds, w->stream, w->P, w->D, T);
     CK(hipGetLastError());
     // the ions start from the slices' positions before the betatron rotation
-    hipLaunchKernelGGL(k_ws_create, dim3(nbp), dim3(WS_WG), 0, w->stream, w->P, w->D);
+    const int nbt = relay ? 0 : (int)(((long long)G * S * WS_ROWS + WS_WG - 1) / WS_WG);
+    hipLaunchKernelGGL(k_ws_create, dim3(nbp + nbt), dim3(WS_WG), 0, w->stream, w->P, w->D);
     CK(hipGetLastError());
     const WSStep T2 = {-1, rev, (int)t, -1, 0, 0};
     if (!relay) {
       if (w->timing) CK(hipEventRecord(w->ev[2 * t], w->stream));
-      hipLaunchKernelGGL(k_ws_ions, dim3(w->D.nblk_ions), dim3(WS_WG), sizeof(double2) * 2 * WS_QT * min(w->P.S, WS_CH),
-                         w->stream, w->P, w->D);
+      hipLaunchKernelGGL(k_ws_ions, dim3(w->D.nblk_ions), dim3(WS_WG), 0, w->stream, w->P, w->D);
       CK(hipGetLastError());
       if (w->timing) CK(hipEventRecord(w->ev[2 * t + 1], w->stream));
       hipLaunchKernelGGL(k_ws_ksum, dim3(G, (2 * S + 3 + KSUM_Q - 1) / KSUM_Q + 2), dim3(64 * KSUM_Q), lds, w->stream,
