@@ -341,44 +341,6 @@ __device__ __forceinline__ void fx_atomic_add(unsigned long long *plo, unsigned 
   atomicAdd(phi, hi + carry);
 }
 
-// The block's dipole sums in LDS: x = A 2^-20 + B 2^-60 + C 2^-100 with A, B, C
-// rounded integers below 2^41 (|x| < 2^20), each added to a 64-bit accumulator of
-// its slice -- the same integer round(x 2^100) as fx_split's, cut differently, so
-// sums are as exact.  A limb is rounded by adding 1.5 2^52, whose bits then hold
-// the integer in their low half; the bits are added as they are and FX_MAGIC times
-// the particle count taken off when the block's sums are folded.  The 128-bit form
-// needed the old value of every addition for the carry, and shifts by the
-// exponent's range with a branch each: 143 instructions a macroparticle and two
-// waits for LDS, now 24 and none.
-#define FX_LIMBS 3
-#define FX_MAGIC_D 6755399441055744.0 // 1.5 2^52
-#define FX_MAGIC 0x4338000000000000ULL
-
-__device__ __forceinline__ void fx_limbs(double x, unsigned long long l[FX_LIMBS])
-{
-  const double u = 1048576.0, w = 1099511627776.0; // 2^20, 2^40
-  const double a = fma(x, u, FX_MAGIC_D);
-  double r = fma(x, u, FX_MAGIC_D - a);
-  const double b = fma(r, w, FX_MAGIC_D);
-  r = fma(r, w, FX_MAGIC_D - b);
-  const double c = fma(r, w, FX_MAGIC_D);
-  l[0] = (unsigned long long)__double_as_longlong(a);
-  l[1] = (unsigned long long)__double_as_longlong(b);
-  l[2] = (unsigned long long)__double_as_longlong(c);
-}
-
-// n particles' accumulated limbs (stride apart) as the 128-bit sum (lo, hi)
-__device__ __forceinline__ void fx_fold(const unsigned long long *l, int stride, unsigned n, unsigned long long &lo,
-                                        unsigned long long &hi)
-{
-  const long long a = (long long)(l[0] - n * FX_MAGIC), b = (long long)(l[stride] - n * FX_MAGIC),
-                  c = (long long)(l[2 * stride] - n * FX_MAGIC);
-  lo = (unsigned long long)c;
-  hi = (unsigned long long)(c >> 63);
-  fx_add(lo, hi, (unsigned long long)b << 40, (unsigned long long)(b >> 24));
-  hi += (unsigned long long)a << 16;
-}
-
 // ------------------------------------------------------------------ k_turn
 
 // MODE_TUNE: the turn's full work for timing work decompositions -- the map's
