@@ -256,9 +256,11 @@ __host__ __device__ __forceinline__ int ws_electrons_lds(int S, int G)
   return 13 * WS_PAD16(S) + 2 * WS_PAD16(G) + 8;
 }
 
-// One block's bunch b; sm: ws_electrons_lds(S, G) doubles, 16-byte aligned.
-__device__ void ws_electrons(const WSP &P, const WSD &D, int b, const WSStep &T, double *sm)
+// One block's bunch b; lds: ws_electrons_lds(S, G) doubles, as the double2 that
+// ws_add_in_order reads, so that they are aligned to it.
+__device__ void ws_electrons(const WSP &P, const WSD &D, int b, const WSStep &T, double2 *lds)
 {
+  double *sm = (double *)lds;
   const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wv = tid >> 6, S = P.S, G = P.G;
   const int kb = D.bucket[b];
   const int SP = WS_PAD16(S), GP = WS_PAD16(G);
@@ -365,7 +367,7 @@ __device__ void ws_electrons(const WSP &P, const WSD &D, int b, const WSStep &T,
 // Blocks 0 .. G-1: the electron side of a bunch each.
 __global__ __launch_bounds__(WS_STEP_WG) void k_ws_step(WSP P, WSD D, WSStep T)
 {
-  extern __shared__ double sm[];
+  extern __shared__ double2 sm[];
   ws_electrons(P, D, blockIdx.x, T, sm);
 }
 
@@ -375,7 +377,7 @@ __global__ __launch_bounds__(WS_STEP_WG) void k_ws_step(WSP P, WSD D, WSStep T)
 // transverse positions only, which kicks and phase 1 leave alone.
 __global__ __launch_bounds__(WS_WG) void k_ws_phase1(WSP P, WSD D, WSStep T)
 {
-  extern __shared__ double sm[];
+  extern __shared__ double2 sm[];
   const int tid = threadIdx.x, S = P.S;
   if ((int)blockIdx.x < P.G) {
     ws_electrons(P, D, blockIdx.x, T, sm);
@@ -918,7 +920,7 @@ __global__ __launch_bounds__(WS_WG, 5) void k_ws_ions(WSP P, WSD D)
 #define KSUM_Q 8
 __global__ __launch_bounds__(64 * KSUM_Q) void k_ws_ksum(WSP P, WSD D, WSStep T)
 {
-  extern __shared__ double sm[];
+  extern __shared__ double2 sm[];
   if (blockIdx.y == gridDim.y - 1) {
     ws_electrons(P, D, blockIdx.x, T, sm);
     return;
