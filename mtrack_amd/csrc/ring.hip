@@ -142,7 +142,7 @@ struct DevParams {
   int n_ahc;
   int monitor_every;
   int scan;
-  long long NrevScan;
+  long long NrevScan; // positive
   double scan_step;
   unsigned seed;
   int m_aHC;
@@ -2078,7 +2078,9 @@ static void fill_params(const mbt_config *c, const int planes[3], DevParams &P)
   P.n_ahc = c->n_ahc;
   P.monitor_every = (int)c->NrevMon;
   P.scan = c->scan;
-  P.NrevScan = c->NrevScan;
+  // the turn number modulo the interval is 0 on the same turns for either sign; an
+  // interval of 0 never ends
+  P.NrevScan = c->NrevScan ? llabs((long long)c->NrevScan) : LLONG_MAX;
   P.scan_step = c->scan_step;
   P.seed = (unsigned)c->iseed[0];
   for (int a = 0; a < c->n_ahc; a++) {
