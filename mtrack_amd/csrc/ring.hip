@@ -1951,13 +1951,29 @@ __global__ __launch_bounds__(256) void k_ring_end(const DevParams *__restrict__ 
   if (lane == 0) fb_apply(P, ts, vs, ps, INIT);
 }
 
-// The long-range wake of one bunch's slices (longitudinal), as the next turn adds it.
-__global__ void k_lr_row(const DevParams *__restrict__ Pr, LRDev R, const double *Ibunch, int ring, int b, int kb,
-                         double *out)
+// One bunch's tables for mbt_ring_potentials, into pinned host memory: seven rows of
+// Nc (the second the longitudinal long-range wake as the next turn adds it), then the
+// ring's turn state.  One launch and one wait, bound by them: 17 us a call (64
+// bunches, 50 slices) against 44-51 as eight small copies and 46-59 with the wake's
+// row made by a kernel beside them.
+struct PotRows {
+  const double *row[7]; // row[1] is made here
+};
+__global__ __launch_bounds__(256) void k_potentials(const DevParams *__restrict__ Pr, LRDev R, const double *Ibunch,
+                                                    const TurnState *ts, PotRows T, int ring, int b, int kb,
+                                                    double *out)
 {
   const DevParams &P = Pr[ring];
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < P.Nc) out[i] = lr_wake_at(P, R, b, kb, 0, i, Ibunch[P.bucket_off + kb]);
+  const int Nc = P.Nc;
+  for (int i = threadIdx.x; i < Nc; i += 256) {
+#pragma unroll
+    for (int k = 0; k < 7; k++)
+      out[k * Nc + i] = k == 1 ? lr_wake_at(P, R, b, kb, 0, i, Ibunch[P.bucket_off + kb]) : T.row[k][i];
+  }
+  static_assert(sizeof(TurnState) % sizeof(double) == 0, "copied as words");
+  const unsigned long long *src = (const unsigned long long *)(ts + ring);
+  unsigned long long *dst = (unsigned long long *)(out + 7 * Nc);
+  for (int i = threadIdx.x; i < (int)(sizeof(TurnState) / sizeof(double)); i += 256) dst[i] = src[i];
 }
 
 // =============================================================== host side
@@ -2027,7 +2043,7 @@ struct mbt_ring {
   LRDev LR;
   LRConst *lc;
   double2 *lr_pw, *lr_L, *lr_V;
-  double *lr_G, *lr_self, *lr_row; // lr_row: one bunch's long-range wake for mbt_ring_potentials
+  double *lr_G, *lr_self;
   int nres;
   double *fb_hist;
   long long rw_total, st_total, fbh_total;
@@ -2214,7 +2230,7 @@ extern "C" void mbt_ring_destroy(mbt_ring *r)
                   r->Hs.tsz, r->Hs.bad, r->sfL, r->sfV, r->sfH, r->Gf, r->pending, r->peek,
                   r->rwhist, r->sqrt_tt, r->rsqrt_tt, r->Ibunch, r->bunch_Ib, r->stats, r->amp, r->rfbuf, r->fnp_out,
                   r->dipV_out, r->dipH_out, r->trash_tot, r->trash_pend, r->ts, r->rw_tiles, r->rw_part, r->lc, r->lr_pw, r->lr_L,
-                  r->lr_V, r->lr_G, r->lr_self, r->lr_row, r->fb_hist,
+                  r->lr_V, r->lr_G, r->lr_self, r->fb_hist,
                   r->rwg_col_ring, r->rwg_bucket_bunch, r->rwg_c, r->rwg_part};
   for (size_t i = 0; i < sizeof ptrs / sizeof ptrs[0]; i++)
     if (ptrs[i]) (void)hipFree(ptrs[i]);
@@ -2908,7 +2924,6 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
   DA(r->lr_V, lr_total > 0 ? lr_total : 1);
   DA(r->lr_G, (size_t)R * 3 * NcA);
   DA(r->lr_self, nres > 0 ? (size_t)3 * G * NcA : 1);
-  DA(r->lr_row, NcA);
   r->LR = {r->lc, r->lr_pw, r->lr_L, r->lr_V, r->lr_G, r->lr_self, r->fb_hist, G};
   // ---- uploads
   UP(r->bunch_first, bfirst, G);
@@ -3597,17 +3612,13 @@ extern "C" int mbt_ring_potentials(const mbt_ring *r, int ib, double *out, doubl
   int ring = 0, local = ib;
   while (local >= r->rh[ring].cfg.Nbunch) local -= r->rh[ring++].cfg.Nbunch;
   const size_t Nc = r->Nc, off = (size_t)ib * Nc;
-  (void)hipGetLastError();
-  hipLaunchKernelGGL(k_lr_row, dim3((unsigned)((Nc + 255) / 256)), dim3(256), 0, r->stream, r->P, r->LR,
-                     (const double *)r->Ibunch, ring, ib, r->rh[ring].cfg.bucket[local], r->lr_row);
-  CK(hipGetLastError());
-  const double *src[7] = {r->sfL + off, r->lr_row, r->fnp_out + off, r->sfV + off, r->dipV_out + off,
-                          r->sfH + off, r->dipH_out + off};
-  // eight small copies into pinned memory, one wait
+  const PotRows T = {{r->sfL + off, NULL, r->fnp_out + off, r->sfV + off, r->dipV_out + off, r->sfH + off,
+                      r->dipH_out + off}};
   double *stage = r->pot_host;
-  for (int k = 0; k < 7; k++)
-    CK(hipMemcpyAsync(stage + k * Nc, src[k], Nc * sizeof(double), hipMemcpyDeviceToHost, r->stream));
-  CK(hipMemcpyAsync(stage + 7 * Nc, r->ts + ring, sizeof(TurnState), hipMemcpyDeviceToHost, r->stream));
+  (void)hipGetLastError();
+  hipLaunchKernelGGL(k_potentials, dim3(1), dim3(256), 0, r->stream, r->P, r->LR, (const double *)r->Ibunch, r->ts, T,
+                     ring, ib, r->rh[ring].cfg.bucket[local], stage);
+  CK(hipGetLastError());
   CK(hipStreamSynchronize(r->stream));
   memcpy(out, stage, 7 * Nc * sizeof(double));
   TurnState ts;
