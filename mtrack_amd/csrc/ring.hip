@@ -472,9 +472,14 @@ template <int HOW> __device__ __forceinline__ double sin_cw(double x, bool &ok)
 }
 
 // Slice index with reciprocal multiplies; where the truncation could depend on
-// the last bits (the approximate value is within 1e-12 of the exact one for
-// |v| < 1e6) the exact reference expression (two correctly rounded divides) takes
-// over.
+// the last bits the exact reference expression (two correctly rounded divides) takes
+// over.  The approximate value is a few units in the last place from the exact one:
+// less than the margin tested, 1e-9, for |v| < 1e6.  Beyond that a macroparticle is far
+// outside the slices (1,090 at most) and only its side counts, to which every value the
+// test lets pass belongs up to 2^31, past which the exact form's conversion gives
+// INT_MIN.  (With the line at 1e6 slices, 1 us of the production ring, macroparticles
+// lost for some thousand turns went through the exact form every turn: 104 x 50,021
+// with dipole histograms, all lost, 307 us a turn, 164 now; a tenth lost 299, 119.)
 struct BinK {
   double sgm, inv_sgm, Nsigma, dT, inv_dT;
 };
@@ -483,7 +488,7 @@ template <int HOW> __device__ __forceinline__ int bin_fast(double tau, const Bin
   if (HOW == EXACT) return bin_of(tau, k.sgm, k.Nsigma, k.dT);
   const double vf = fma(fma(-tau, k.inv_sgm, k.Nsigma), k.inv_dT, 1.0);
   const double lo = trunc(vf - 1.0e-9), hi = trunc(vf + 1.0e-9);
-  const bool in = fabs(vf) < 1.0e6 && lo == hi;
+  const bool in = fabs(vf) < 2.147483e9 && lo == hi;
   if (HOW == FAST) ok = ok && in;
   else if (!in) return bin_of(tau, k.sgm, k.Nsigma, k.dT);
   return (int)lo;
@@ -865,8 +870,8 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
   // take the fast forms first, in a loop without calls: with the fallbacks inside
   // it every value that outlives a call sat in a preserved register or on the stack
   // and the constants were fetched again after each.  The few macroparticles that
-  // leave a fast form's range (about one in 1e8, at a slice's edge; lost ones every
-  // turn) are noted, untouched, and done with the exact forms after it.  416 x
+  // leave a fast form's range (about one in 1e8, at a slice's edge; every turn those
+  // lost for so long that their RF phase is past sincos_cw's range) are noted, untouched, and done with the exact forms after it.  416 x
   // 50,021 macroparticles with excitation and dipoles: 551 -> 455 us at best, 601
   // -> 512 a turn in a long run; 104 x 20,000 with excitation and harmonic cavity
   // 67 -> 60.  (Two macroparticles at a time at 2 or 3 waves per SIMD: 10 % slower.)
