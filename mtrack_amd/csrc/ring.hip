@@ -119,7 +119,7 @@
 // ring is an ensemble of one).  Derived on the host with glibc libm from the
 // reference's formulas so that every constant equals the reference's.
 struct DevParams {
-  int ring, Nb, h, Nc, Nmlt;
+  int Nb, h, Nc, Nmlt;
   int lrp[4];       // first long-range resonator of the planes LON, HOR, VER and the end
   long long lr_off; // of the ring's [h + 1][resonators] entries in LRDev::L and V
   // bound on |x| and |z| of a particle whose dipole enters the exact fixed-point
@@ -128,7 +128,6 @@ struct DevParams {
   // beyond it marks the bunch's sums NaN
   double fx_lim;
   unsigned long long zero_bits; // always 0: the timing pass's stores xor with it
-  int mixed;                    // compensated FP32 wake convolutions (MBT_RING_MIXED)
   int bunch_off;  // first global bunch of the ring
   int bucket_off; // first global bucket of the ring
   long long rw_off, st_off; // offsets into the RW history and sqrt table
@@ -145,7 +144,6 @@ struct DevParams {
   long long NrevScan; // positive
   double scan_step;
   unsigned seed;
-  int m_aHC;
   double ahc_amp[MBT_MAX_AHC], ahc_wn[MBT_MAX_AHC], ahc_phi[MBT_MAX_AHC], ahc_nHC[MBT_MAX_AHC];
   double E0, E0k; // E0 [GeV], E0 * FKILO
   double RsisL, aindL;
@@ -189,8 +187,7 @@ __device__ __forceinline__ long long umod(long long a, long long d)
 __device__ __forceinline__ int rw_trigger(long long rev, long long NrevScan) { return umod(rev, NrevScan) < 50 ? 1 : 0; }
 
 struct LRConst {
-  int ring, plane, l, fb;
-  int h, bucket_off;
+  int fb;
   int init_turns; // wake_phasor_init replay length Nbumax / h
   double pr0, pr1;   // one bin
   double ge, gc, gs; // bucket gap
@@ -975,7 +972,6 @@ struct RedOut {
   int *trash_pend;   // [G*2]
   const double *G;   // Green functions [R][3][Nc]: Gl, Gv, Gh
   const double *bunch_Ib;
-  const int *np;
   int Gtot;
   double *rfbuf;     // [STATS_TURNS][R][2] phase and voltage the turn's map used
   int R;
@@ -1440,9 +1436,8 @@ __device__ void end_turns(const DevParams &P, TurnState *ts, double *bunch_Ib, d
 }
 
 // RF feedback of one ring: rffb_calc_mean_voltage_phase (src/feedback_rf.c:21-34)
-// and the solve of src/worker_weakweak.c:268-278; the phase and voltage before
-// the solve are kept for the potentials output.
-// The solve from the sums of the sampled voltages vs and phases ps.
+// and the solve of src/worker_weakweak.c:268-278, from the sums of the sampled
+// voltages vs and phases ps.
 __device__ void fb_apply(const DevParams &P, TurnState *ts, double vs, double ps, int init)
 {
   const int fb_len = P.fb_len;
@@ -1455,20 +1450,6 @@ __device__ void fb_apply(const DevParams &P, TurnState *ts, double vs, double ps
   ts->phai0 = ph;
   ts->Vrf0 = num / sin(ph);
   if (init && P.fb_switch_off) ts->has_fb = 0;
-}
-
-__device__ void fb_solve(const DevParams &P, TurnState *ts, const double *fb_hist, int init)
-{
-  ts->phai0_prev = ts->phai0;
-  ts->Vrf0_prev = ts->Vrf0;
-  if (!ts->has_fb) return;
-  const double *fbh = fb_hist + P.fbh_off;
-  double vs = 0, ps = 0;
-  for (int m = 0; m < P.fb_len; m++) {
-    vs += fbh[2 * m];
-    ps += fbh[2 * m + 1];
-  }
-  fb_apply(P, ts, vs, ps, init);
 }
 
 static size_t rw_old_lds(int span) { return (size_t)span * (3 * 8 + 4) + RW_TILE_TAPS * 8; }
@@ -1894,7 +1875,11 @@ __global__ __launch_bounds__(256) void k_ring_end(const DevParams *__restrict__ 
   if (end && tid == 0) end_turns(P, ts, bunch_Ib, Ibunch, nfFill, end);
   const int lr0 = P.lrp[0], nr = P.lrp[3] - lr0;
   if (nr == 0) {
-    if (tid == 0) fb_solve(P, ts, R.fb_hist, INIT);
+    // no feedback without a resonator to sample
+    if (tid == 0) {
+      ts->phai0_prev = ts->phai0;
+      ts->Vrf0_prev = ts->Vrf0;
+    }
     return;
   }
   __syncthreads();
@@ -2021,7 +2006,7 @@ struct mbt_ring {
   long long *bunch_first;
   WgInfo *wgs;
   BunchInfo *bunches;
-  int *bucket, *bunch_ring, *bucket_ring, *np, *nfFill;
+  int *bucket, *bunch_ring, *np, *nfFill;
   DevParams *P;
   double *partial, *shift;
   HistPtr Hs;
@@ -2230,7 +2215,7 @@ extern "C" void mbt_ring_destroy(mbt_ring *r)
   (void)hipSetDevice(r->device);
   if (r->stream) (void)hipStreamSynchronize(r->stream); // turns of mbt_ring_track_async may still run
   if (r->pot_host) (void)hipHostFree(r->pot_host);
-  void *ptrs[] = {r->C.s, r->wgs, r->bunches, r->bunch_first, r->bucket, r->bunch_ring, r->bucket_ring, r->np, r->nfFill,
+  void *ptrs[] = {r->C.s, r->wgs, r->bunches, r->bunch_first, r->bucket, r->bunch_ring, r->np, r->nfFill,
                   r->P, r->partial, r->shift, r->Hs.cnt, r->Hs.sx, r->Hs.sz, r->Hs.tcnt, r->Hs.tsx,
                   r->Hs.tsz, r->Hs.bad, r->sfL, r->sfV, r->sfH, r->Gf, r->pending, r->peek,
                   r->rwhist, r->sqrt_tt, r->rsqrt_tt, r->Ibunch, r->bunch_Ib, r->stats, r->amp, r->rfbuf, r->fnp_out,
@@ -2730,8 +2715,6 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
     }
     DevParams &P = r->Ph[k];
     fill_params(c, hh->planes, P);
-    P.mixed = (flags & MBT_RING_MIXED) ? 1 : 0;
-    P.ring = k;
     P.bunch_off = G;
     P.bucket_off = H;
     P.rw_off = rw_total;
@@ -2774,7 +2757,7 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
   r->nwg_cap = nwg;
   int *nph = (int *)malloc(G * sizeof(int)), *bring = (int *)malloc(G * sizeof(int)), *bk = (int *)malloc(G * sizeof(int));
   long long *bfirst = (long long *)malloc(G * sizeof(long long));
-  int *qring = (int *)malloc(H * sizeof(int)), *fill = (int *)malloc(H * sizeof(int));
+  int *fill = (int *)malloc(H * sizeof(int));
   double *Ibq = (double *)malloc(H * sizeof(double)), *bIb = (double *)malloc(G * sizeof(double));
   {
     int g = 0, q = 0;
@@ -2783,7 +2766,6 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
       const mbt_config *c = &r->rh[k].cfg;
       const long long Np = c->Np;
       for (int i = 0; i < (int)c->Nharm; i++, q++) {
-        qring[q] = k;
         fill[q] = c->nfFill[i];
         Ibq[q] = c->Ibunch[i];
       }
@@ -2809,7 +2791,6 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
   DA(r->bunch_first, G);
   DA(r->bucket, G);
   DA(r->bunch_ring, G);
-  DA(r->bucket_ring, H);
   DA(r->np, G);
   DA(r->nfFill, H);
   DA(r->P, R);
@@ -2874,11 +2855,6 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
         for (int l = 0; l < cf->n_lr[p]; l++) {
           const mbt_lr_resonator *res = &cf->lr[p][l];
           LRConst &L = lc[ir++];
-          L.ring = k;
-          L.plane = p;
-          L.l = l;
-          L.h = (int)cf->Nharm;
-          L.bucket_off = r->Ph[k].bucket_off;
           L.init_turns = (int)(cf->Nbumax / cf->h);
           double alpha = res->wr * 0.5 / res->Qfactor;
           double Amp = 2 * alpha * res->Rs * cf->T0 / cf->E0 / MBT_FGIGA;
@@ -2935,7 +2911,6 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
   UP(r->np, nph, G);
   UP(r->bunch_ring, bring, G);
   UP(r->bucket, bk, G);
-  UP(r->bucket_ring, qring, H);
   UP(r->nfFill, fill, H);
   UP(r->Ibunch, Ibq, H);
   UP(r->bunch_Ib, bIb, G);
@@ -2983,7 +2958,6 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
   free(bring);
   free(bk);
   free(bfirst);
-  free(qring);
   free(fill);
   free(Ibq);
   free(bIb);
@@ -3006,7 +2980,6 @@ static int create_rings(const mbt_config *const *cfgs, int R, int device, int fl
   Ro.trash_pend = r->trash_pend;
   Ro.G = r->Gf;
   Ro.bunch_Ib = r->bunch_Ib;
-  Ro.np = r->np;
   Ro.Gtot = G;
   Ro.rfbuf = r->rfbuf;
   Ro.R = R;

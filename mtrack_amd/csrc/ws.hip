@@ -585,7 +585,6 @@ __global__ __launch_bounds__(WS_WG) void k_ws_train(WSP P, WSD D, int ib, long l
   __syncthreads();
   if (!last) return;
   __threadfence();
-  const int kb = D.bucket[ib];
   const double nel = D.nelec[ib];
   double *xp = D.sl + (size_t)ib * 6 * S + 3 * S, *zp = xp + 2 * S;
   for (int c = tid; c < S; c += WS_WG) {
@@ -627,7 +626,6 @@ __global__ __launch_bounds__(WS_WG) void k_ws_train(WSP P, WSD D, int ib, long l
   }
   if (tid == 0) {
     *D.done = 0;
-    (void)kb;
   }
 }
 
