@@ -731,7 +731,7 @@ __device__ __forceinline__ void ions_sum(const Ion &I, bool act, double v[8], in
 }
 
 // N <= 4 slices of a bunch from entry o of the tables on: the kicks, then the 2 N field
-// sums and (CLOUD, N <= 2: the bunch's last slices) the cloud sums after them, over the
+// sums and (CLOUD, N <= 1: the bunch's last slice) the cloud sums after them, over the
 // wave in one reduction into wred from row 2 c0 on.
 // Each slice's entries are read before the ion's place in the slice is known, from the
 // cell it had: an ion changes cells in one of five thousand slices, and the weights
@@ -770,15 +770,12 @@ __device__ __forceinline__ void ions_chunk(const WSP &P, const double2 *qt, cons
   int c0 = cb;
   for (; c0 + 4 <= ce; c0 += 4, o += 4 * WS_QT) ions_group<4, false>(P, qt, wt, o, c0, cl, I, wred, lane, wv);
   if (ce < P.S) return;
-  const int r = P.S - c0;
-  if (r == 1)
-    ions_group<1, true>(P, qt, wt, o, c0, cl, I, wred, lane, wv);
-  else if (r == 2)
-    ions_group<2, true>(P, qt, wt, o, c0, cl, I, wred, lane, wv);
-  else {
-    if (r) ions_group<3, false>(P, qt, wt, o, c0, cl, I, wred, lane, wv);
+  // one slice left or three: their number is odd
+  if (P.S - c0 == 3) {
+    ions_group<3, false>(P, qt, wt, o, c0, cl, I, wred, lane, wv);
     ions_group<0, true>(P, qt, wt, o, P.S, cl, I, wred, lane, wv);
-  }
+  } else
+    ions_group<1, true>(P, qt, wt, o, c0, cl, I, wred, lane, wv);
 }
 
 // The slices of a chunk in a bunch that some of the lanes' ions are not yet made in:
