@@ -271,7 +271,9 @@ int mbt_ring_rf_state(const mbt_ring *r, int ring, double *out);
 int mbt_ring_rw_history(const mbt_ring *r, double *out);
 /* Kernel timing of the last mbt_ring_track call, milliseconds per kernel class:
  * [0] turn map pass, [1] per-bunch reduction, [2] turn end with the LR
- * recurrence and RF feedback, [3] RW sum (for small rings with the turn end). */
+ * recurrence and RF feedback, [3] RW sum.  Only rings with LR resonators or a
+ * current scan end every turn; for the others [2] holds no launch (its time is
+ * that of the events) and the one turn end of a block of turns is in no class. */
 int mbt_ring_kernel_times(const mbt_ring *r, double *ms, long *launches);
 /* Bytes of HBM the turn map pass must move per turn (algorithmic). */
 double mbt_ring_bytes_per_turn(const mbt_ring *r);

@@ -770,7 +770,7 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
   // lost for so long that their RF phase is past sincos_cw's range) are noted, untouched, and done with the exact forms after it.  416 x
   // 50,021 macroparticles with excitation and dipoles: 551 -> 455 us at best, 601
   // -> 512 a turn in a long run; 104 x 20,000 with excitation and harmonic cavity
-  // 67 -> 60.  (Two macroparticles at a time at 2 or 3 waves per SIMD: 10 % slower.)
+  // 67 -> 58.  (Two macroparticles at a time at 2 or 3 waves per SIMD: 10 % slower.)
   // The plain variant streams at the memory's rate, and the second loop's code
   // cost it 2-3 %, so it keeps its fallbacks in place.
   unsigned long long redo = 0, bit = 1;
@@ -945,14 +945,14 @@ template <int Q, bool mixed> __device__ __forceinline__ double conv_at(const dou
 // fill, 2 = turn, 3 = final statistics.
 // Bound: latency, one block per bunch after a pass that left its inputs in other
 // XCDs' reach.  So every load that needs only the bunch is under way before the
-// first is waited for, the ring's constants are copied to LDS in one go, the
-// statistics (wave 3) run beside the histogram (waves 0 ..), and the convolutions
-// take two slices i and Nc - 1 - i per group of Q lanes, so that every lane has the
-// same (Nc + 1) / Q terms and only the planes that have a wake are visited.  One
-// bunch x 100 slices x 3 planes 16.1 -> 7.7 us, 64 x 50 slices 10.0 -> 5.6, 416 x
-// 100 18.6 -> 10.1, 333 x 50 with three LR resonators 26.7 -> 9.8 (one lane per slice
-// and plane, loads waited for one by one, the statistics and 64-bit remainders in
-// front of the rest).
+// first is waited for, the ring's constants are copied to LDS in one go, all stores
+// but the long-range sums' come behind the last barrier, the statistics by the last
+// wave, and the convolutions take two slices i and Nc - 1 - i per group of Q lanes, so
+// that every lane has the same (Nc + 1) / Q terms and only the planes that have a wake
+// are visited.  One bunch x 100 slices x 3 planes 16.1 -> 7.7 us, 64 x 50 slices 10.0
+// -> 5.6, 416 x 100 18.6 -> 10.2, 333 x 50 with three LR resonators 26.7 -> 9.9 (one
+// lane per slice and plane, loads waited for one by one, the statistics and 64-bit
+// remainders in front of the rest).
 template <int NT, int Q, bool MIXED>
 __global__ __launch_bounds__(NT) void k_reduce(const DevParams *__restrict__ Pr, const double *__restrict__ partial,
                                                const BunchInfo *__restrict__ bunches, int nrings, HistPtr H, RedOut R,
@@ -1698,7 +1698,7 @@ __device__ __forceinline__ double2 shfl_up2(double2 v, int d)
 // the wave, and every lane walks its own buckets from the phasor that reaches
 // them: about 30 dependent complex products a pass of 512 buckets instead of one
 // chain over them (which took 150 us a turn with its slices, 333 bunches in
-// 416 buckets x 50 slices, 3 resonators; the whole kernel now takes 12).
+// 416 buckets x 50 slices, 3 resonators; the whole kernel now takes 10.6).
 // fbh: also take the feedback samples from number keep on (the first one is c0;
 // W: what the first reads).
 template <bool INIT>

@@ -171,7 +171,8 @@ __device__ __forceinline__ void ws_interp(const double2 *t, double aAx, double a
 // Bound: latency (sums of 41 slices and of up to h kicks kept in the
 // reference's order, one lane each).  416 bunches, 10 wall turns, per turn: 107 us
 // as three launches (one lane for all of a bunch's sums; a test of the filling, a
-// square root and two divisions per tap) -> 12.5 us as one.
+// square root and two divisions per tap) -> 13.1 us as one, kernel time; a turn takes
+// 19.5, the rest lies between the launches.
 struct WSStep {
   int kick;            // slot of the turn whose ion sums to apply, -1: none
   long long rev2;      // phase 2 of this turn, -1: none
@@ -813,9 +814,12 @@ __device__ __forceinline__ void lds_barrier()
 // each the fixed-order sum of its four waves' sums.  The bunches up to the
 // block's last creator (some ions not yet made) run with per-lane
 // predicates, the rest without.
-// Bound: the chain of the longest block, (G - 1) S slices one after the other, and
-// FP64 issue while all blocks are there.  So the chain has no wait for memory in it:
-// the tables of a bunch come ready-made in chunks of WS_CH slices through two buffers
+// Bound: vector issue for a long train, of 356 bunches 92 % of the kernel's cycles with
+// 34.7 instructions a lane, ion and slice, 61 % of them FP64; a slice's latency for a
+// short one, of 61 bunches 364 cycles per slice in the chain of the longest block's
+// (G - 1) S slices, with one wave per SIMD and vector issue 19 % of the cycles.  (The
+// long train's chain is 80 % of its time at that rate.)  So the chain has no wait for
+// memory in it: the tables of a bunch come ready-made in chunks of WS_CH slices through two buffers
 // in LDS, one barrier a chunk (for LDS alone), the next chunk's entries on their way in
 // registers while a chunk is used, and a slice's reads don't wait for its cell.  A
 // chunk is read in full: past the bunch's last slice it holds the next bunch's tables,
