@@ -945,8 +945,8 @@ template <int Q, bool mixed> __device__ __forceinline__ double conv_at(const dou
 // fill, 2 = turn, 3 = final statistics.
 // Bound: latency, one block per bunch after a pass that left its inputs in other
 // XCDs' reach.  So every load that needs only the bunch is under way before the
-// first is waited for, the ring's constants are copied to LDS in one go, all stores
-// but the long-range sums' come behind the last barrier, the statistics by the last
+// first is waited for, the ring's constants are copied to LDS in one go, the stores
+// come behind the barrier after the histogram, the statistics by the last
 // wave, and the convolutions take two slices i and Nc - 1 - i per group of Q lanes, so
 // that every lane has the same (Nc + 1) / Q terms and only the planes that have a wake
 // are visited.  One bunch x 100 slices x 3 planes 16.1 -> 7.7 us, 64 x 50 slices 10.0
