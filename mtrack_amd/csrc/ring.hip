@@ -767,10 +767,14 @@ __global__ __launch_bounds__(WG, TURN_WAVES_PER_EU) void k_turn(const DevParams 
   // it every value that outlives a call sat in a preserved register or on the stack
   // and the constants were fetched again after each.  The few macroparticles that
   // leave a fast form's range (about one in 1e8, at a slice's edge; every turn those
-  // lost for so long that their RF phase is past sincos_cw's range) are noted, untouched, and done with the exact forms after it.  416 x
-  // 50,021 macroparticles with excitation and dipoles: 551 -> 455 us at best, 601
-  // -> 512 a turn in a long run; 104 x 20,000 with excitation and harmonic cavity
-  // 67 -> 58.  (Two macroparticles at a time at 2 or 3 waves per SIMD: 10 % slower.)
+  // lost for so long that their RF phase is past sincos_cw's range) are noted,
+  // untouched, and done with the exact forms after it.  416 x 50,021 macroparticles
+  // with excitation and dipoles: 551 -> 455 us at best, 601 -> 512 a turn in a long
+  // run; 104 x 20,000 with excitation and harmonic cavity 67 -> 58.  (Two
+  // macroparticles at a time at 2 or 3 waves per SIMD: 10 % slower.  With a tenth of the
+  // macroparticles past that range the second loop doubles the pass, 155 -> 299 us for
+  // 104 x 50,021 with dipoles; taking their sine in the first loop costs every ring of
+  // these variants 2-3 %.)
   // The plain variant streams at the memory's rate, and the second loop's code
   // cost it 2-3 %, so it keeps its fallbacks in place.
   unsigned long long redo = 0, bit = 1;
@@ -2118,7 +2122,8 @@ extern "C" void mbt_ring_destroy(mbt_ring *r)
                   r->P, r->partial, r->shift, r->Hs.cnt, r->Hs.sx, r->Hs.sz, r->Hs.tcnt, r->Hs.tsx,
                   r->Hs.tsz, r->Hs.bad, r->sfL, r->sfV, r->sfH, r->Gf, r->pending, r->peek,
                   r->rwhist, r->sqrt_tt, r->rsqrt_tt, r->Ibunch, r->bunch_Ib, r->stats, r->amp, r->rfbuf, r->fnp_out,
-                  r->dipV_out, r->dipH_out, r->trash_tot, r->trash_pend, r->ts, r->rw_tiles, r->rw_part, r->lc, r->lr_pw, r->lr_L,
+                  r->dipV_out, r->dipH_out, r->trash_tot, r->trash_pend, r->ts, r->rw_tiles, r->rw_part, r->lc, r->lr_pw,
+                  r->lr_L,
                   r->lr_V, r->lr_G, r->lr_self, r->fb_hist,
                   r->rwg_col_ring, r->rwg_bucket_bunch, r->rwg_c, r->rwg_part};
   for (size_t i = 0; i < sizeof ptrs / sizeof ptrs[0]; i++)
@@ -3132,8 +3137,8 @@ static int launch_reduce(mbt_ring *r, int phase, int turn)
   const int nt = wide ? REDUCE_WIDE : WG, pairs = (r->Nc + 1) / 2, lanes = nt / (pairs > 0 ? pairs : 1);
   const reduce_kernel_t k = r->mixed ? (wide ? reduce_kernel<REDUCE_WIDE, true>(lanes) : reduce_kernel<WG, true>(lanes))
                                      : (wide ? reduce_kernel<REDUCE_WIDE, false>(lanes) : reduce_kernel<WG, false>(lanes));
-  hipLaunchKernelGGL(k, dim3(r->G), dim3(nt), r->lds_red, r->stream, r->P, r->partial, r->bunches, r->R, r->Hs, r->Ro, r->ts, phase, dip, r->LR, r->lr_lds,
-                     turn, r->Nc);
+  hipLaunchKernelGGL(k, dim3(r->G), dim3(nt), r->lds_red, r->stream, r->P, r->partial, r->bunches, r->R, r->Hs, r->Ro,
+                     r->ts, phase, dip, r->LR, r->lr_lds, turn, r->Nc);
   CK(hipGetLastError());
   return MBT_OK;
 }
