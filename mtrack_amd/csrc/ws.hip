@@ -1171,8 +1171,8 @@ extern "C" int mbt_ws_create(const mbt_config *c, int device, int flags, mbt_ws 
     WA(w->d_convion, G);
     if (P.rw) {
       // the wake W = prf / sqrt(D / c) of every distance a dipole can act over, D =
-      // d buckets (d = h: the bunch's own, one turn) and j turns
-      const size_t nw = (size_t)4 * (c->Nmlt + 1) * H;
+      // d buckets (d = h: the bunch's own, one turn) and j turns; none without a tap
+      const size_t nw = c->Nmlt < 0 ? 0 : (size_t)4 * (c->Nmlt + 1) * H;
       double *wl = (double *)malloc(sizeof(double) * nw);
       const double Dub0 = c->Lc / ((double)c->Nharm);
       for (int t = 0, i = 0; t < 2; t++)
