@@ -2164,6 +2164,10 @@ static int check_cfg(const mbt_config *c)
     mbt_set_error("NrevMon must be positive");
     return MBT_EINVAL;
   }
+  if (c->EnableRW_long && c->Nmlt < -1) {
+    mbt_set_error("Nmlt %d leaves the resistive wall no row of dipole history", c->Nmlt);
+    return MBT_EINVAL;
+  }
   int lr_tot = c->n_lr[0] + c->n_lr[1] + c->n_lr[2];
   if ((lr_tot > 0 || c->n_res > 0 || c->n_wakefile > 0) && c->Ncell <= 0) {
     mbt_set_error("wakes need Ncell > 0");
